@@ -296,6 +296,113 @@ __device__ inline int32_t wide_first_hit(const BvhView& b, f3 p, uint32_t& visit
   return r >= 0 ? r : -1;
 }
 
+// ---- the four-wide walk by quads
+// Four adjacent lanes walk one query together, lane e on entry e of every
+// record: a visit is two 16-byte loads and one box test per lane instead of
+// eight and four, and the lanes of a quad read one 128-byte line between
+// them.  What the lanes must agree on goes through quad permutes (DPP, no
+// LDS); the deferred stack is one per quad.  The visits, their order and the
+// hits are those of wide_first_hit.
+template <int CTRL>
+__device__ inline int32_t quad_perm(int32_t v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+// lane K's value in every lane of the quad
+template <int K>
+__device__ inline float quad_bcast(float v) {
+  return __int_as_float(quad_perm<K * 0x55>(__float_as_int(v)));
+}
+// the bitwise or of the quad's values, in every lane
+__device__ inline int32_t quad_or(int32_t v) {
+  v |= quad_perm<0xB1>(v);        // lanes 1 0 3 2
+  return v | quad_perm<0x4E>(v);  // lanes 2 3 0 1
+}
+
+constexpr int QSTK_QUADS = 64;   // quads of a workgroup of 256 lanes: entry k of a quad is lds[k * QSTK_QUADS]
+
+__device__ inline void qstk_put(const Spill& sp, int k, int32_t v) {
+  if (k < WSTK_LDS)
+    sp.lds[k * QSTK_QUADS] = v;
+  else
+    sp.p[(size_t)(k - WSTK_LDS) * sp.stride] = v;
+}
+__device__ inline int32_t qstk_get(const Spill& sp, int k) {
+  int32_t v = sp.lds[min(k, WSTK_LDS - 1) * QSTK_QUADS];
+  asm volatile("" : "+v"(v));
+  if (k >= WSTK_LDS) v = sp.p[(size_t)(k - WSTK_LDS) * sp.stride];
+  return v;
+}
+
+// One visit: lane e holds entry e = {a, b} of the record.  Every lane of the
+// quad returns the same (see wide_visit).
+template <bool GROUPED>
+__device__ inline int32_t quad_visit(f3 p, int e, float4 a, float4 b, const Spill& spill, int& sp, int32_t& node,
+                                     int limit) {
+  const bool in = in_box(p, a.x, a.y, a.z, a.w, b.x, b.y);
+  int32_t link = __float_as_int(b.z);
+  int32_t m = quad_or(in ? 1 << e : 0);
+  if constexpr (GROUPED) {
+    // a split record whose first candidate is in entries 0-1: entries 2-3,
+    // when both hold p, become one candidate, their parent's record
+    const int32_t split = quad_perm<0>(__float_as_int(b.w));
+    const bool fold = (split != 0) & ((m & 3) != 0) & ((m & 12) == 12);
+    link = (fold && e == 2) ? split : link;
+    m = fold ? m & 7 : m;
+  }
+  if (m == 0) {
+    if (sp == 0) return WIDE_MISS;
+    --sp;
+    node = qstk_get(spill, sp);
+    return node < 0 ? ~node : WIDE_NEXT;
+  }
+  const int f = __builtin_ctz(m);
+  const int32_t c = quad_or(e == f ? link : 0);
+  if (c < 0) return ~c;
+  const int k = __builtin_popcount(m) - 1;
+  if (sp + k > limit) {
+    trav_fault(spill, TRAV_OVERFLOW);
+    return WIDE_MISS;
+  }
+  // the later candidates, the lowest entry on top
+  if (e > f && ((m >> e) & 1)) qstk_put(spill, sp + __builtin_popcount(m >> (e + 1)), link);
+  sp += k;
+  node = c;
+  return WIDE_NEXT;
+}
+
+// Lane e's entry of the root record, loaded by the caller with its other
+// first loads.
+struct QuadRoot {
+  float4 a, b;
+};
+__device__ inline QuadRoot load_quad_root(const BvhView& b, int e) {
+  if (b.wide && b.m >= 2) return QuadRoot{b.wide[2 * e], b.wide[2 * e + 1]};
+  return QuadRoot{make_float4(0.0f, 0.0f, 0.0f, 0.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f)};
+}
+
+// The first hit of p (the same in every lane of the quad; likewise the
+// result) through the four-wide form of a body of at least two triangles.
+template <bool GROUPED>
+__device__ inline int32_t quad_first_hit(const BvhView& b, f3 p, int e, uint32_t& visits, Spill spill,
+                                         const QuadRoot& rt) {
+  int sp = 0;
+  int32_t node = 0;
+  const int limit = stack_limit(spill);
+  ++visits;
+  int32_t r = quad_visit<GROUPED>(p, e, rt.a, rt.b, spill, sp, node, limit);
+  uint32_t guard = 0;
+  for (; r == WIDE_NEXT && guard < b.m; ++guard) {
+    const float4* nd = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(b.wide) +
+                                                       (((uint32_t)node << 7) + ((uint32_t)e << 5)));
+    const float4 qa = nd[0], qb = nd[1];
+    asm volatile("" ::"v"(qb.z), "v"(qb.w));
+    ++visits;
+    r = quad_visit<GROUPED>(p, e, qa, qb, spill, sp, node, limit);
+  }
+  if (r == WIDE_NEXT) trav_fault(spill, TRAV_BOUND);
+  return r >= 0 ? r : -1;
+}
+
 // First-hit traversal (D_BVH::intersect, cudaBRT.cu:239-285): one node
 // record (64 bytes, both child boxes and links) per memory round trip.  The
 // stack never holds more entries than the node depth, and the depth of a
@@ -340,13 +447,11 @@ __device__ inline bool plane_test(const float* verts, uint4 t, f3 p, float& d, f
   return !(d > 0.0f);
 }
 
-// collision_response_projection (verlet.cu:24-50) on a position p: when the
-// first-hit leaf's plane test says inside, p += |d| n and the contact normal
-// is n, else the contact normal is 0.  Returns true when projected.
-template <bool WIDE = true>
-__device__ inline bool collide_project(const BvhView& b, f3& p, f3& n_out, int32_t& hit,
-                                       uint32_t& visits, Spill spill, const WideRoot& rt) {
-  hit = bvh_first_hit<WIDE>(b, p, visits, spill, rt);
+// collision_response_projection (verlet.cu:24-50) on a position p whose
+// first hit is leaf `hit` (-1: none): when that leaf's plane test says inside,
+// p += |d| n and the contact normal is n, else the contact normal is 0.
+// Returns true when projected.
+__device__ inline bool project_hit(const BvhView& b, int32_t hit, f3& p, f3& n_out) {
   n_out = mk(0.0f, 0.0f, 0.0f);
   if (hit < 0) return false;
   float d;
@@ -356,6 +461,23 @@ __device__ inline bool collide_project(const BvhView& b, f3& p, f3& n_out, int32
   p = p + n * dd;
   n_out = n;
   return true;
+}
+
+// The first hit of p and its projection.
+template <bool WIDE = true>
+__device__ inline bool collide_project(const BvhView& b, f3& p, f3& n_out, int32_t& hit,
+                                       uint32_t& visits, Spill spill, const WideRoot& rt) {
+  hit = bvh_first_hit<WIDE>(b, p, visits, spill, rt);
+  return project_hit(b, hit, p, n_out);
+}
+
+// The same by the four lanes of a quad (lane e; p and every result are the
+// same in all four).  The view has no body, or its four-wide form.
+__device__ inline bool collide_project_quad(const BvhView& b, f3& p, f3& n_out, int32_t& hit, uint32_t& visits,
+                                            int e, Spill spill, const QuadRoot& rt) {
+  hit = -1;
+  if (b.m) hit = b.grouped ? quad_first_hit<true>(b, p, e, visits, spill, rt) : quad_first_hit<false>(b, p, e, visits, spill, rt);
+  return project_hit(b, hit, p, n_out);
 }
 
 }  // namespace cc

@@ -17,12 +17,16 @@ __device__ inline NState ld_state(const float* __restrict__ s, uint32_t j) {
   return NState{ld3(sj), ld3(sj + 3)};
 }
 
-// One spring's term of compute_spring_force (verlet.cu:52-88) added to S:
+// One spring's term of compute_spring_force (verlet.cu:52-88), sc * dP:
 // record rr {end | type << 30, rest}, neighbour state g.  An empty slot
 // (real false) gathers the vertex itself: dP = (eps, eps, eps) > 0 and
-// sc = +0, so the products are +0 and S (never -0) is unchanged.
-__device__ inline void spring_term(f3 p, f3 vel, const NState& g, uint2 rr, bool real, const StepArgs& a,
-                                   float ks0, float ks1, float ks2, f3& S) {
+// sc = +0, so the products are +0 and a sum (never -0) is unchanged by them.
+struct SpringTerm {
+  f3 dP;
+  float sc;
+};
+__device__ inline SpringTerm spring_scale(f3 p, f3 vel, const NState& g, uint2 rr, bool real, const StepArgs& a,
+                                          float ks0, float ks1, float ks2) {
   const uint32_t t = rr.x >> 30;
   const float rest = __uint_as_float(rr.y) * a.rest_scale;
   const float ks = t == 0 ? ks0 : (t == 1 ? ks1 : ks2);
@@ -35,9 +39,33 @@ __device__ inline void spring_term(f3 p, f3 vel, const NState& g, uint2 rr, bool
   const float L = L2 * rinv;
   const float vd = fmaf(dV.z, dP.z, fmaf(dV.y, dP.y, dV.x * dP.x));
   const float sc = real ? fmaf(-ks, L - rest, a.kd * vd * rinv) * rinv : 0.0f;
-  S.x = fmaf(dP.x, sc, S.x);
-  S.y = fmaf(dP.y, sc, S.y);
-  S.z = fmaf(dP.z, sc, S.z);
+  return SpringTerm{dP, sc};
+}
+
+// The term added to S.
+__device__ inline void spring_term(f3 p, f3 vel, const NState& g, uint2 rr, bool real, const StepArgs& a,
+                                   float ks0, float ks1, float ks2, f3& S) {
+  const SpringTerm t = spring_scale(p, vel, g, rr, real, a, ks0, ks1, ks2);
+  S.x = fmaf(t.dP.x, t.sc, S.x);
+  S.y = fmaf(t.dP.y, t.sc, S.y);
+  S.z = fmaf(t.dP.z, t.sc, S.z);
+}
+
+// The Verlet update of a vertex under force F, the part of F along the
+// contact normal c removed.
+__device__ inline f3 verlet_update(f3 p, f3 q, f3 c, f3 F, const StepArgs& a) {
+  const float cf = fmaf(c.z, F.z, fmaf(c.y, F.y, c.x * F.x));
+  F = mk(fmaf(-c.x, cf, F.x), fmaf(-c.y, cf, F.y), fmaf(-c.z, cf, F.z));
+  // pos + pos - pos_old + acc*dt*dt (verlet.cu:155) evaluated as
+  // pos + ((pos - pos_old) + acc*dt^2): pos - pos_old is exact for close
+  // values, so the only rounding at |pos| is the last addition.
+  return mk(p.x + fmaf(F.x * a.inv_mass, a.dt2, p.x - q.x), p.y + fmaf(F.y * a.inv_mass, a.dt2, p.y - q.y),
+            p.z + fmaf(F.z * a.inv_mass, a.dt2, p.z - q.z));
+}
+
+__device__ inline bool same_bits(f3 a, f3 b) {
+  return __float_as_uint(a.x) == __float_as_uint(b.x) && __float_as_uint(a.y) == __float_as_uint(b.y) &&
+         __float_as_uint(a.z) == __float_as_uint(b.z);
 }
 
 // Vertex i from state `sin_` to `sout` (24 B {x_cur, x_prev} per vertex),
@@ -128,14 +156,7 @@ __device__ inline void step_vertex(uint32_t i, const float* __restrict__ sin_, f
           spring_term(p, vel, g[q], rr[q], k0 + q < r1, a, ks0, ks1, ks2, S);
       }
     }
-    F = F + S;
-    const float cf = fmaf(c.z, F.z, fmaf(c.y, F.y, c.x * F.x));
-    F = mk(fmaf(-c.x, cf, F.x), fmaf(-c.y, cf, F.y), fmaf(-c.z, cf, F.z));
-    // pos + pos - pos_old + acc*dt*dt (verlet.cu:155) evaluated as
-    // pos + ((pos - pos_old) + acc*dt^2): pos - pos_old is exact for close
-    // values, so the only rounding at |pos| is the last addition.
-    np = mk(p.x + fmaf(F.x * a.inv_mass, a.dt2, p.x - q.x), p.y + fmaf(F.y * a.inv_mass, a.dt2, p.y - q.y),
-            p.z + fmaf(F.z * a.inv_mass, a.dt2, p.z - q.z));
+    np = verlet_update(p, q, c, F + S, a);
     nq = p;
     if (DEBUG) st3(dbg_pre + 3 * (size_t)i, np);
     inside = collide_project<WIDE>(bvh, np, nc, hit, visits, spill, root);
@@ -151,9 +172,102 @@ __device__ inline void step_vertex(uint32_t i, const float* __restrict__ sin_, f
   o[3] = nq.x; o[4] = nq.y; o[5] = nq.z;
   // an update in place stores the normal only where it changed (bit for
   // bit): most vertices keep theirs (0 away from the body) from step to step
-  if (contact_out != contact_in || __float_as_uint(nc.x) != __float_as_uint(c.x) ||
-      __float_as_uint(nc.y) != __float_as_uint(c.y) || __float_as_uint(nc.z) != __float_as_uint(c.z))
-    st3(contact_out + 3 * (size_t)i, nc);
+  if (contact_out != contact_in || !same_bits(nc, c)) st3(contact_out + 3 * (size_t)i, nc);
+}
+
+// The terms of lane K's NB springs added to S in every lane of the quad, in
+// their order.
+template <int K, int NB>
+__device__ inline void quad_add(const SpringTerm (&t)[NB], f3& S) {
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const float sc = quad_bcast<K>(t[k].sc);
+    S.x = fmaf(quad_bcast<K>(t[k].dP.x), sc, S.x);
+    S.y = fmaf(quad_bcast<K>(t[k].dP.y), sc, S.y);
+    S.z = fmaf(quad_bcast<K>(t[k].dP.z), sc, S.z);
+  }
+}
+
+// step_vertex by the four lanes of a quad (lane e), the body walked by quads
+// through its four-wide form.  Lane e takes a quarter of the springs; the
+// terms are then added in row order in every lane, so the sums, and with
+// them every result, equal step_vertex's bit for bit.
+template <bool DEBUG, int EW>
+__device__ inline void step_vertex_quad(uint32_t i, int e, const float* __restrict__ sin_, float* __restrict__ sout,
+                                        const float* contact_in, float* contact_out, const uint32_t* __restrict__ row,
+                                        const uint2* __restrict__ rec, const StepArgs& a, const BvhView& bvh,
+                                        Spill spill, uint32_t& visits, float* __restrict__ dbg_pre,
+                                        int32_t* __restrict__ dbg_hit, uint8_t* __restrict__ dbg_in) {
+  constexpr bool ELL = EW > 0;
+  constexpr int NB = ELL ? EW / 4 : 3;      // springs of a lane at a time
+  uint2 er[NB];
+  if constexpr (ELL) {
+#pragma unroll
+    for (int k = 0; k < NB; ++k) er[k] = rec[(size_t)i * EW + (uint32_t)(e * NB + k)];
+  }
+  const QuadRoot root = load_quad_root(bvh, e);
+  const uint32_t r0raw = row[i], r1raw = ELL ? 0u : row[i + 1];
+  const float2* s2 = reinterpret_cast<const float2*>(sin_ + 6 * (size_t)i);
+  const float2 e0 = s2[0], e1 = s2[1], e2 = s2[2];
+  const f3 c = ld3(contact_in + 3 * (size_t)i);
+  asm volatile("" ::"v"(r0raw), "v"(r1raw), "v"(e0.x), "v"(e0.y), "v"(e1.x), "v"(e1.y), "v"(e2.x), "v"(e2.y),
+               "v"(c.x), "v"(c.y), "v"(c.z));
+  const uint32_t r0 = r0raw & ROW_MASK, r1 = r1raw & ROW_MASK;
+  const f3 p = mk(e0.x, e0.y, e1.x), q = mk(e1.y, e2.x, e2.y);
+  f3 np = p, nq = p, nc = mk(0.0f, 0.0f, 0.0f);
+  int32_t hit = -1;
+  bool inside = false;
+  if (!(r0raw & PIN_BIT)) {
+    const f3 vel = mk((p.x - q.x) * a.inv_dt, (p.y - q.y) * a.inv_dt, (p.z - q.z) * a.inv_dt);
+    const f3 F = mk(fmaf(vel.x, a.damp, a.gmx), fmaf(vel.y, a.damp, a.gmy), fmaf(vel.z, a.damp, a.gmz));
+    f3 S = mk(0.f, 0.f, 0.f);
+    const float ks0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k0)));
+    const float ks1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k1)));
+    const float ks2 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k2)));
+    uint32_t k0 = r0;
+    do {
+      if constexpr (!ELL) {
+        if (k0 >= r1) break;
+      }
+      bool real[NB];
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        if constexpr (ELL) {
+          real[k] = (er[k].x & PAD_TYPE) != PAD_TYPE;
+        } else {
+          const uint32_t at = k0 + (uint32_t)(e * NB + k);
+          real[k] = at < r1;
+          er[k] = rec[min(at, r1 - 1)];
+          if (!real[k]) er[k] = make_uint2(i, 0u);
+        }
+      }
+      NState g[NB];
+#pragma unroll
+      for (int k = 0; k < NB; ++k) g[k] = ld_state(sin_, er[k].x & END_MASK);
+      SpringTerm t[NB];
+#pragma unroll
+      for (int k = 0; k < NB; ++k) t[k] = spring_scale(p, vel, g[k], er[k], real[k], a, ks0, ks1, ks2);
+      quad_add<0>(t, S);
+      quad_add<1>(t, S);
+      quad_add<2>(t, S);
+      quad_add<3>(t, S);
+      k0 += 4 * NB;
+    } while (!ELL);
+    np = verlet_update(p, q, c, F + S, a);
+    if (DEBUG && e == 0) st3(dbg_pre + 3 * (size_t)i, np);
+    inside = collide_project_quad(bvh, np, nc, hit, visits, e, spill, root);
+    if (inside) nq = np;
+  } else if (DEBUG && e == 0) {
+    st3(dbg_pre + 3 * (size_t)i, np);
+  }
+  if (DEBUG && e == 0) {
+    dbg_hit[i] = hit;
+    dbg_in[i] = inside ? 1 : 0;
+  }
+  // lane 0 stores the position, lane 1 the one before, lane 2 the normal
+  float* o = e == 2 ? contact_out + 3 * (size_t)i : sout + 6 * (size_t)i + 3 * e;
+  const f3 v = e == 0 ? np : (e == 1 ? nq : nc);
+  if (e < 2 || (e == 2 && (contact_out != contact_in || !same_bits(nc, c)))) st3(o, v);
 }
 
 }  // namespace cc

@@ -22,6 +22,26 @@
 
 namespace cc {
 
+// Block sum of the lanes' visits and queries into the block's own counter
+// pair (no shared atomics).
+__device__ inline void count_block(uint32_t visits, bool query, unsigned long long* __restrict__ ctr) {
+  __shared__ unsigned long long wsum[2][4];
+  unsigned long long v = visits, qn = query ? 1ull : 0ull;
+  for (int off = 32; off > 0; off >>= 1) {
+    v += __shfl_down(v, off, 64);
+    qn += __shfl_down(qn, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    wsum[0][threadIdx.x >> 6] = v;
+    wsum[1][threadIdx.x >> 6] = qn;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    ctr[2 * blockIdx.x] += wsum[0][0] + wsum[0][1] + wsum[0][2] + wsum[0][3];
+    ctr[2 * blockIdx.x + 1] += wsum[1][0] + wsum[1][1] + wsum[1][2] + wsum[1][3];
+  }
+}
+
 // One thread per vertex.  Spring forces use FMA and rsqrt (positions are
 // checked against the FP64 oracle by tolerance); the collision part is exact
 // order so the contact set is bit-exact for the pre-projection positions.
@@ -47,24 +67,32 @@ __global__ __launch_bounds__(256) void k_verlet(const float* __restrict__ sin_, 
     step_vertex<DEBUG, EW, WIDE>(i, sin_, sout, contact_in, contact_out, row, rec, a, bvh,
                                  spill_of(spill, i, n, lds), visits, dbg_pre, dbg_hit, dbg_in);
   }
-  if (COUNT) {
-    // block sum into this block's own counter pair (no shared atomics)
-    __shared__ unsigned long long wsum[2][4];
-    unsigned long long v = visits, qn = active ? 1ull : 0ull;
-    for (int off = 32; off > 0; off >>= 1) {
-      v += __shfl_down(v, off, 64);
-      qn += __shfl_down(qn, off, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-      wsum[0][threadIdx.x >> 6] = v;
-      wsum[1][threadIdx.x >> 6] = qn;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      ctr[2 * blockIdx.x] += wsum[0][0] + wsum[0][1] + wsum[0][2] + wsum[0][3];
-      ctr[2 * blockIdx.x + 1] += wsum[1][0] + wsum[1][1] + wsum[1][2] + wsum[1][3];
-    }
-  }
+  if (COUNT) count_block(visits, active, ctr);
+}
+
+// The same step with four lanes per vertex (see step_vertex_quad), for cloths
+// whose waves leave most of the chip idle (by_quads): bound by the chain of
+// dependent loads of a vertex (its records, the gathers, a record per visit,
+// the hit's triangle), which a quad walks with fewer instructions and fewer
+// cache-line requests between them.  63 VGPRs (12-wide rows) against 126, so
+// eight waves per SIMD.
+template <bool DEBUG, bool COUNT, int EW>
+__global__ __launch_bounds__(256) void k_verlet_quad(const float* __restrict__ sin_, float* __restrict__ sout,
+                                                     const float* contact_in, float* contact_out,
+                                                     const uint32_t* __restrict__ row, const uint2* __restrict__ rec,
+                                                     StepArgs a, BvhView bvh, uint32_t n, int32_t* __restrict__ spill,
+                                                     float* __restrict__ dbg_pre, int32_t* __restrict__ dbg_hit,
+                                                     uint8_t* __restrict__ dbg_in,
+                                                     unsigned long long* __restrict__ ctr) {
+  __shared__ int32_t qstk[WSTK_LDS * QSTK_QUADS];
+  const uint32_t i = blockIdx.x * QSTK_QUADS + (threadIdx.x >> 2);
+  const int e = (int)(threadIdx.x & 3u);
+  uint32_t visits = 0;
+  const bool active = i < n;
+  if (active)
+    step_vertex_quad<DEBUG, EW>(i, e, sin_, sout, contact_in, contact_out, row, rec, a, bvh,
+                                spill_of(spill, i, n, qstk + (threadIdx.x >> 2)), visits, dbg_pre, dbg_hit, dbg_in);
+  if (COUNT) count_block(e == 0 ? visits : 0u, active && e == 0, ctr);
 }
 
 __global__ __launch_bounds__(256) void k_collide_points(BvhView bvh, const float* __restrict__ pts, uint32_t n,
@@ -84,10 +112,45 @@ __global__ __launch_bounds__(256) void k_collide_points(BvhView bvh, const float
   st3(out_n + 3 * (size_t)i, nc);
 }
 
+// The same query with four lanes per point.
+__global__ __launch_bounds__(256) void k_collide_quad(BvhView bvh, const float* __restrict__ pts, uint32_t n,
+                                                      int32_t* __restrict__ spill, int32_t* __restrict__ hit,
+                                                      uint8_t* __restrict__ ins, float* __restrict__ out_pos,
+                                                      float* __restrict__ out_n) {
+  const uint32_t i = blockIdx.x * QSTK_QUADS + (threadIdx.x >> 2);
+  const int e = (int)(threadIdx.x & 3u);
+  __shared__ int32_t qstk[WSTK_LDS * QSTK_QUADS];
+  if (i >= n) return;
+  f3 p = ld3(pts + 3 * (size_t)i), nc;
+  int32_t h;
+  uint32_t visits = 0;
+  const bool in = collide_project_quad(bvh, p, nc, h, visits, e, spill_of(spill, i, n, qstk + (threadIdx.x >> 2)),
+                                       load_quad_root(bvh, e));
+  if (e < 2) st3((e ? out_n : out_pos) + 3 * (size_t)i, e ? nc : p);
+  if (e == 2) hit[i] = h;
+  if (e == 3) ins[i] = in ? 1 : 0;
+}
+
+// Which walk a launch of n vertices or points takes.  Four lanes per vertex
+// shorten a vertex's chain of dependent work (a quarter of the springs, a
+// visit of two loads instead of eight) but make four times the waves, each
+// about 40% of the one-lane kernel's instructions: the better form while
+// the quads' waves all fit on the chip beside each other (four per SIMD, 16
+// quads each: 256 CUs x 4 x 4 x 16).  Measured (us per step, one lane / four
+// lanes): in contact 11.7 / 8.6 at 4,096 vertices, 17.9 / 11.2 at 16,773
+// (24-wide rows), 21.3 / 16.5 at 65,536, 25.9 / 22.4 at 131,044, 53.6 / 60.1
+// at 262,144; falling 4.8 / 3.5 at 4,096, 6.5 / 6.4 at 65,536 and 8.3 / 9.8
+// at 131,044.
+constexpr uint32_t QUAD_MAX_N = 65536;
+static bool by_quads(const BvhView& v, uint32_t n) { return n <= QUAD_MAX_N && (v.wide || v.m == 0); }
+
 void launch_collide_points(const BvhView& v, const float* pts, uint32_t n, int32_t* spill, int32_t* hit,
                            uint8_t* ins, float* out_pos, float* out_n, hipStream_t s) {
   if (n == 0) return;
-  k_collide_points<<<grid_for(n, 256), 256, 0, s>>>(v, pts, n, spill, hit, ins, out_pos, out_n);
+  if (by_quads(v, n))
+    k_collide_quad<<<grid_for(n, QSTK_QUADS), 256, 0, s>>>(v, pts, n, spill, hit, ins, out_pos, out_n);
+  else
+    k_collide_points<<<grid_for(n, 256), 256, 0, s>>>(v, pts, n, spill, hit, ins, out_pos, out_n);
   CC_LAUNCHED();
 }
 
@@ -187,7 +250,15 @@ static void launch_k_verlet(const Sim& S, unsigned g, hipStream_t s, const float
   const uint2* recs = S.ell_w ? S.ell.p : S.rec.p;
 #define CC_STEP_ARGS g, s, e0, e1, in, out, contact_in, contact_out, S.row.p, recs, a, v, S.n, S.spill.p, dbg_pre, \
                      dbg_hit, dbg_in, ctr
-  if (v.wide) {
+  if (by_quads(v, S.n)) {
+    g = grid_for(S.n, QSTK_QUADS);
+    if (S.ell_w == ELL_W)
+      launch_one(k_verlet_quad<DEBUG, COUNT, ELL_W>, CC_STEP_ARGS);
+    else if (S.ell_w == ELL_W2)
+      launch_one(k_verlet_quad<DEBUG, COUNT, ELL_W2>, CC_STEP_ARGS);
+    else
+      launch_one(k_verlet_quad<DEBUG, COUNT, 0>, CC_STEP_ARGS);
+  } else if (v.wide) {
     if (S.ell_w == ELL_W)
       launch_one(k_verlet<DEBUG, COUNT, ELL_W, true>, CC_STEP_ARGS);
     else if (S.ell_w == ELL_W2)
@@ -381,7 +452,7 @@ int cc_sim_create(const cc_cloth_desc* cloth, const cc_body_desc* bd, const cc_p
     S.state[1].zero(s);
     S.contact.alloc(3 * (size_t)S.n);
     S.contact.zero(s);
-    S.ctr.alloc(2 * (size_t)grid_for(S.n, 256));   // per-block visit / query counts
+    S.ctr.alloc(2 * (size_t)grid_for(S.n, QSTK_QUADS));   // per-block visit / query counts
     S.ctr.zero(s);
     S.flag.alloc(1);
     if (bd && bd->mode != CC_BODY_NONE) {
