@@ -55,56 +55,56 @@ __global__ __launch_bounds__(256) void k_fold_wide(const Node* __restrict__ node
   }
 }
 
-// Entry e of record o: box b6 (min xyz, max xyz), link, split word.
-__device__ inline void put_entry(float4* o, int e, const float* mn, const float* mx, int32_t link, int32_t split) {
-  o[2 * e] = make_float4(mn[0], mn[1], mn[2], mx[0]);
-  o[2 * e + 1] = make_float4(mx[1], mx[2], __int_as_float(link), __int_as_float(split));
-}
-__device__ inline void put_empty(float4* o, int e) {
-  o[2 * e] = make_float4(INFINITY, INFINITY, INFINITY, -INFINITY);
-  o[2 * e + 1] = make_float4(-INFINITY, -INFINITY, 0.0f, 0.0f);
-}
-// Entries e, e + 1: the children of internal node y in y's order of
-// consideration (a leaf child first, A before B).
-__device__ inline void put_pair(float4* o, int e, const Node& y, int32_t split) {
-  if (y.childA >= 0 && y.childB < 0) {
-    put_entry(o, e, y.b_min, y.b_max, y.childB, split);
-    put_entry(o, e + 1, y.a_min, y.a_max, y.childA, 0);
-  } else {
-    put_entry(o, e, y.a_min, y.a_max, y.childA, split);
-    put_entry(o, e + 1, y.b_min, y.b_max, y.childB, 0);
-  }
-}
-
 // The wide form of a rebuilt body, record x from internal node x: X's leaf
 // children (A before B), then the children of its internal children (A's,
-// then B's).  With both children internal, entry 0's split word is B's
-// index.  Reads nodes x, A and B (64 bytes each), writes 128 bytes.
+// then B's), each pair in its parent's order of consideration (a leaf child
+// first, A before B).  With both children internal, entry 0's split word is
+// B's index.  Four lanes per record, lane e writing entry e: bound by the 128
+// bytes written and the lines read (nodes x, A and B), which the lanes of a
+// quad share.  Three frames of 50,688 triangles: 9.9 us, against 14.8 with one
+// lane per record (eight stores 128 bytes apart).
 __global__ __launch_bounds__(256) void k_fold_grouped(PF<const Node> nodes_f, uint32_t mi, PF<float4> wide_f) {
-  const uint32_t x = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t t = blockIdx.x * 256 + threadIdx.x, x = t >> 2;
+  const int e = (int)(t & 3u);
   if (x >= mi) return;
-  const Node* __restrict__ N = pick(nodes_f);
-  float4* o = pick(wide_f) + 8 * (size_t)x;
-  const Node X = N[x];
-  const bool la = X.childA < 0, lb = X.childB < 0;
+  const float4* N = reinterpret_cast<const float4*>(pick(nodes_f));
+  const int4 lx = reinterpret_cast<const int4*>(N)[4 * (size_t)x + 3];
+  const bool la = lx.x < 0, lb = lx.y < 0;
+  // the node whose child slot the entry is, and the entry's place in its pair
+  int32_t y = (int32_t)x;
+  int at = e;
+  bool empty = false;
   if (la && lb) {
-    put_entry(o, 0, X.a_min, X.a_max, X.childA, 0);
-    put_entry(o, 1, X.b_min, X.b_max, X.childB, 0);
-    put_empty(o, 2);
-    put_empty(o, 3);
+    empty = e > 1;
   } else if (la || lb) {
-    if (la) {
-      put_entry(o, 0, X.a_min, X.a_max, X.childA, 0);
-      put_pair(o, 1, N[X.childB], 0);
+    empty = e == 3;
+    if (e > 0) {
+      y = la ? lx.y : lx.x;
+      at = e - 1;
     } else {
-      put_entry(o, 0, X.b_min, X.b_max, X.childB, 0);
-      put_pair(o, 1, N[X.childA], 0);
+      at = la ? 0 : 1;
     }
-    put_empty(o, 3);
   } else {
-    put_pair(o, 0, N[X.childA], X.childB);
-    put_pair(o, 2, N[X.childB], 0);
+    y = e < 2 ? lx.x : lx.y;
+    at = e & 1;
   }
+  const float4* ny = N + 4 * (size_t)y;
+  const float4 q0 = ny[0], q1 = ny[1], q2 = ny[2];
+  const int4 ly = reinterpret_cast<const int4*>(ny)[3];
+  // a pair whose B alone is a leaf is considered B first
+  const bool b_side = (y != (int32_t)x && ly.x >= 0 && ly.y < 0) ? at == 0 : at == 1;
+  const float inf = INFINITY;
+  float4 o0 = b_side ? make_float4(q1.z, q1.w, q2.x, q2.y) : q0;
+  float4 o1 = b_side ? make_float4(q2.z, q2.w, 0.0f, 0.0f) : make_float4(q1.x, q1.y, 0.0f, 0.0f);
+  o1.z = __int_as_float(b_side ? ly.y : ly.x);
+  if (e == 0 && !la && !lb) o1.w = __int_as_float(lx.y);
+  if (empty) {
+    o0 = make_float4(inf, inf, inf, -inf);
+    o1 = make_float4(-inf, -inf, 0.0f, 0.0f);
+  }
+  float4* o = pick(wide_f) + 2 * (size_t)t;
+  o[0] = o0;
+  o[1] = o1;
 }
 
 void Body::fold_frames(int F, const int* ks, hipStream_t s) {
@@ -115,7 +115,7 @@ void Body::fold_frames(int F, const int* ks, hipStream_t s) {
     nodes.p[f] = slot[ks[f]].nodes.p;
     wide.p[f] = slot[ks[f]].wide.p;
   }
-  k_fold_grouped<<<dim3(grid_for(m - 1, 256), (unsigned)F), 256, 0, s>>>(nodes, m - 1, wide);
+  k_fold_grouped<<<dim3(grid_for(4 * (size_t)(m - 1), 256), (unsigned)F), 256, 0, s>>>(nodes, m - 1, wide);
   CC_LAUNCHED();
 }
 
