@@ -67,7 +67,6 @@ struct BatchBodies {
   DBuf<BItem> items[2];               // [level-0 chunks * 128] unfinished nodes between levels
   DBuf<uint32_t> nitems[2];           // [level-0 chunks] their count per chunk
   DBuf<uint4> leaf_tri[2];            // [sum m]
-  DBuf<int32_t> leaf_parent[2];       // [sum m]
   DBuf<Node> nodes[2];                // [sum max(m - 1, 1)]
   DBuf<float> root[2], leaf0[2];      // [6 * nb]
   DBuf<float> motion;                 // [BB_FRAMES * nb * BB_MF]

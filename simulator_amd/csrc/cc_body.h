@@ -68,12 +68,16 @@ struct BodyDesc {
 };
 
 // A node finished by one level of the bottom-up build and handed to the
-// next (its sorted-leaf range, Karras index and box).
+// next: its sorted-leaf range, Karras index, box, the key of its first leaf
+// and the deltas of the key pairs at its two boundaries (-1 at the ends of
+// the body).
 struct alignas(16) BItem {
-  int32_t l, r, idx, pad;
+  int32_t l, r, idx, dl;
   float box[6];
-  float pad2[2];
+  uint64_t key;
+  int32_t dr, pad[3];
 };
+static_assert(sizeof(BItem) == 64, "BItem must be 64 bytes");
 
 // One workgroup of a build level: chunk q of the body's level, input slots
 // from in_base (n_in of them; leaves at level 0), output slots at out_base.
@@ -87,7 +91,7 @@ constexpr uint32_t LV_MAX_LEAVES = 1u << 21;   // leaf indices of the bottom-up 
 // The bottom-up build (bbody.hip): work tables of its levels for the given
 // bodies (level 0: chunks of 1024 leaves, level L+1: 8 chunks of level L),
 // the number of level-0 chunks of m leaves, and the launches of all levels.
-// keys / leaf_tri / boxes / leaf_parent / nodes are indexed through each
+// keys / boxes / nodes are indexed through each
 // body's t0 / n0; root and leaf0 hold 6 floats per body.
 std::vector<std::vector<LvBlock>> build_level_tables(const std::vector<BodyDesc>& h,
                                                      const std::vector<uint32_t>& bodies);
@@ -95,12 +99,10 @@ size_t level_chunks0(uint32_t m);
 // The buffers of one frame of a level build.
 struct LvFrame {
   const uint64_t* keys;
-  const uint4* leaf_tri;
   const float* boxes;
   BItem* items[2];
   uint32_t* nitems[2];
   Node* nodes;
-  int32_t* leaf_parent;
   float* root;
   float* leaf0;
 };
@@ -158,8 +160,8 @@ struct Lane {
 
 // Host copy of a built tree in the reference encoding (see cc_bvh_export):
 // sorted keys, leaf order, links, child boxes, root box.
-void export_tree_raw(uint32_t m, const uint64_t* keys_d, const uint4* leaf_tri_d, const int32_t* leaf_parent_d,
-                     const Node* nodes_d, const float* root_d, const float* leaf0_d, uint64_t* okeys,
+void export_tree_raw(uint32_t m, const uint64_t* keys_d, const uint4* leaf_tri_d, const Node* nodes_d,
+                     const float* root_d, const float* leaf0_d, uint64_t* okeys,
                      uint32_t* order, int32_t* childA, int32_t* childB, int32_t* parent_int, int32_t* parent_leaf,
                      float* box_int, float* box_leaf, float* root6, hipStream_t s);
 

@@ -68,11 +68,28 @@ __global__ __launch_bounds__(256) void k_deform(const float* __restrict__ rest, 
 // ------------------------------------------------------------ boxes + codes
 constexpr int BOX_THREADS = 256;
 
+// Component threadIdx.x (0..5) of the block's box, in its first six threads:
+// lanes reduce by shuffles, waves through red.
+template <int WAVES>
+__device__ inline float block_box(float* mn, float* mx, float (&red)[WAVES][6]) {
+  for (int off = 32; off > 0; off >>= 1)
+    for (int c = 0; c < 3; ++c) {
+      mn[c] = fminf(mn[c], __shfl_xor(mn[c], off, 64));
+      mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], off, 64));
+    }
+  if ((threadIdx.x & 63u) == 0) put6(red[threadIdx.x >> 6], mn, mx);
+  __syncthreads();
+  const uint32_t c = threadIdx.x < 6 ? threadIdx.x : 0;
+  float v = red[0][c];
+  for (int w = 1; w < WAVES; ++w) v = c < 3 ? fminf(v, red[w][c]) : fmaxf(v, red[w][c]);
+  return v;
+}
+
 // expanded box per triangle + one partial root box per block
 __global__ __launch_bounds__(BOX_THREADS) void k_prim_boxes(PF<const float> verts_f,
                                                             const uint32_t* __restrict__ tris, uint32_t m,
                                                             float depth, PF<float> boxes_f, PF<float> partial_f) {
-  __shared__ float red[6][BOX_THREADS];
+  __shared__ float red[BOX_THREADS / 64][6];
   const float* __restrict__ verts = pick(verts_f);
   float* __restrict__ boxes = pick(boxes_f);
   float* __restrict__ partial = pick(partial_f);
@@ -83,101 +100,124 @@ __global__ __launch_bounds__(BOX_THREADS) void k_prim_boxes(PF<const float> vert
     const uint32_t* t = tris + 3 * (size_t)i;
     prim_box(ld3(verts + 3 * (size_t)t[0]), ld3(verts + 3 * (size_t)t[1]), ld3(verts + 3 * (size_t)t[2]),
              depth, mn, mx);
-    float* b = boxes + 6 * (size_t)i;
-    b[0] = mn[0]; b[1] = mn[1]; b[2] = mn[2];
-    b[3] = mx[0]; b[4] = mx[1]; b[5] = mx[2];
+    put6(boxes + 6 * (size_t)i, mn, mx);
   }
-  for (int c = 0; c < 3; ++c) {
-    red[c][threadIdx.x] = mn[c];
-    red[3 + c][threadIdx.x] = mx[c];
-  }
-  __syncthreads();
-  for (int s = BOX_THREADS / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < (uint32_t)s)
-      for (int c = 0; c < 3; ++c) {
-        red[c][threadIdx.x] = fminf(red[c][threadIdx.x], red[c][threadIdx.x + s]);
-        red[3 + c][threadIdx.x] = fmaxf(red[3 + c][threadIdx.x], red[3 + c][threadIdx.x + s]);
-      }
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) partial[6 * (size_t)blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
-}
-
-// root box (sentinel U all partials, recomputed per block) then the code of
-// each box centroid (compute_morton_bbox, bvh.cu:71-79)
-__global__ __launch_bounds__(256) void k_morton(PF<const float> boxes_f, uint32_t m, PF<const float> partial_f,
-                                                uint32_t npart, PF<uint32_t> codes_f, PF<uint32_t> idx_f,
-                                                PF<float> root_f) {
-  __shared__ float red[6][256];
-  const float* __restrict__ boxes = pick(boxes_f);
-  const float* __restrict__ partial = pick(partial_f);
-  uint32_t* __restrict__ codes = pick(codes_f);
-  uint32_t* __restrict__ idx = pick(idx_f);
-  float* __restrict__ root_out = pick(root_f);
-  float mn[3], mx[3];
-  box_sentinel(mn, mx);
-  for (uint32_t q = threadIdx.x; q < npart; q += 256)
-    for (int c = 0; c < 3; ++c) {
-      mn[c] = fminf(mn[c], partial[6 * (size_t)q + c]);
-      mx[c] = fmaxf(mx[c], partial[6 * (size_t)q + 3 + c]);
-    }
-  for (int c = 0; c < 3; ++c) {
-    red[c][threadIdx.x] = mn[c];
-    red[3 + c][threadIdx.x] = mx[c];
-  }
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < (uint32_t)s)
-      for (int c = 0; c < 3; ++c) {
-        red[c][threadIdx.x] = fminf(red[c][threadIdx.x], red[c][threadIdx.x + s]);
-        red[3 + c][threadIdx.x] = fmaxf(red[3 + c][threadIdx.x], red[3 + c][threadIdx.x + s]);
-      }
-    __syncthreads();
-  }
-  const float rmin[3] = {red[0][0], red[1][0], red[2][0]};
-  const float rext[3] = {red[3][0] - red[0][0], red[4][0] - red[1][0], red[5][0] - red[2][0]};
-  if (blockIdx.x == 0 && threadIdx.x < 6) root_out[threadIdx.x] = red[threadIdx.x][0];
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= m) return;
-  const float* b = boxes + 6 * (size_t)i;
-  codes[i] = box_morton(b, b + 3, rmin, rext);
-  idx[i] = i;
+  const float v = block_box<BOX_THREADS / 64>(mn, mx, red);
+  if (threadIdx.x < 6) partial[6 * (size_t)blockIdx.x + threadIdx.x] = v;
 }
 
 // ------------------------------------------------------------ radix sort
-// Stable LSD sort of (code, index) pairs by code, 8 bits per pass.  Because
-// the indices enter in ascending order and every pass is stable, the result
-// is ordered by the full 64-bit key (code << 32 | index).
-constexpr int SORT_THREADS = 256;
-constexpr int SORT_ITEMS = 4;
-constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;
-// three passes of 10-bit digits cover the 30-bit Morton codes
+// Stable LSD sort of (code, index) pairs by code, three passes of 10-bit
+// digits (the Morton codes have 30 bits).  Because the indices enter in
+// ascending order and every pass is stable, the result is ordered by the
+// full 64-bit key (code << 32 | index).
+//
+// A pass cuts the keys into tiles of SORT_TILE, one workgroup each: the tile's
+// digit counts (by k_morton for the first pass, k_radix_hist for the others),
+// then k_radix_scatter.  A body of up to SORT_SCAN_BLOCKS tiles has no scan
+// launch between the two: the counts lie tile after tile and every scatter
+// workgroup sums the ones before it and all of them itself (at most 64 x 4
+// KB, coalesced); a larger body's counts lie digit after digit and are
+// scanned by k_radix_rowscan first, because the tiles' own sums grow with
+// the square of their number.  The chain of small launches is what a rebuild
+// of a garment-sized body costs (its lanes run beside the step, and other
+// simulators' work queues behind them).  50,688 triangles, three frames in a
+// chain: 37 us from codes to sorted leaves in six launches, against 68 us in
+// eleven (separate counts of the first pass, scans and key / leaf writing;
+// one row of 256 keys at a time between barriers).  Four rows per wave
+// instead of two: 33 us of scatters against 27.
+constexpr int SORT_THREADS = 512;
+constexpr int SORT_WAVES = SORT_THREADS / 64;
+constexpr int SORT_ROWS = 2;              // rows of 64 consecutive keys per wave
+constexpr int SORT_TILE = SORT_THREADS * SORT_ROWS;
 constexpr int RADIX_BITS = 10;
 constexpr int RADIX_DIGITS = 1 << RADIX_BITS;
 constexpr int RADIX_PASSES = 3;
-constexpr int DIGITS_PER_THREAD = RADIX_DIGITS / SORT_THREADS;
+constexpr uint32_t SORT_SCAN_BLOCKS = 64;
+// counts tile after tile are 16-bit pairs; a workgroup reads them in
+// SORT_GROUPS groups of lanes, each summing every SORT_GROUPS-th tile
+constexpr int SORT_WORDS = RADIX_DIGITS / 2;
+constexpr int SORT_GROUPS = SORT_THREADS * 4 / SORT_WORDS;
+constexpr int SORT_LOADS = SORT_SCAN_BLOCKS / SORT_GROUPS;
+static_assert(SORT_THREADS * 2 == RADIX_DIGITS, "two digits per thread");
+static_assert(SORT_LOADS * SORT_TILE < 65536, "a group's sums fit 16 bits");
 
-__global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(PF<const uint32_t> keys_f, uint32_t n, int shift,
-                                                             PF<uint32_t> hist_f, uint32_t nblk) {
-  __shared__ uint32_t h[RADIX_DIGITS];
-  const uint32_t* __restrict__ keys = pick(keys_f);
-  uint32_t* __restrict__ hist = pick(hist_f);
-  for (int q = 0; q < DIGITS_PER_THREAD; ++q) h[q * SORT_THREADS + threadIdx.x] = 0;
-  __syncthreads();
-  const uint32_t base = blockIdx.x * SORT_TILE;
-  for (int r = 0; r < SORT_ITEMS; ++r) {
-    const uint32_t e = base + r * SORT_THREADS + threadIdx.x;
-    if (e < n) atomicAdd(&h[(keys[e] >> shift) & (RADIX_DIGITS - 1)], 1u);
-  }
-  __syncthreads();
-  for (int q = 0; q < DIGITS_PER_THREAD; ++q) {
-    const uint32_t d = q * SORT_THREADS + threadIdx.x;
-    hist[(size_t)d * nblk + blockIdx.x] = h[d];
+// The workgroup's counts h to its tile's place: tile after tile (by_tile) or
+// digit after digit.
+__device__ inline void put_counts(const uint32_t* h, uint32_t* __restrict__ hist, uint32_t nblk, bool by_tile) {
+  const uint32_t t = threadIdx.x;
+  if (by_tile) {
+    hist[(size_t)blockIdx.x * SORT_WORDS + t] = h[2 * t] | (h[2 * t + 1] << 16);
+  } else {
+    hist[(size_t)(2 * t) * nblk + blockIdx.x] = h[2 * t];
+    hist[(size_t)(2 * t + 1) * nblk + blockIdx.x] = h[2 * t + 1];
   }
 }
 
-// Per digit, the exclusive prefix over blocks of the block counts (in place)
-// and the digit's total: one wave per digit, 64 blocks per round.
+// root box (sentinel U all partials, recomputed per block), then the code of
+// each box centroid (compute_morton_bbox, bvh.cu:71-79) of a sort tile and
+// the first pass's digit counts
+__global__ __launch_bounds__(SORT_THREADS) void k_morton(PF<const float> boxes_f, uint32_t m,
+                                                         PF<const float> partial_f, uint32_t npart,
+                                                         PF<uint32_t> codes_f, PF<uint32_t> hist_f, uint32_t nblk,
+                                                         bool by_tile, PF<float> root_f) {
+  __shared__ float red[SORT_WAVES][6], sroot[6];
+  __shared__ uint32_t h[RADIX_DIGITS];
+  const float* __restrict__ boxes = pick(boxes_f);
+  const float* __restrict__ partial = pick(partial_f);
+  uint32_t* __restrict__ codes = pick(codes_f);
+  float* __restrict__ root_out = pick(root_f);
+  const uint32_t tid = threadIdx.x, base = blockIdx.x * SORT_TILE;
+  float bx[SORT_ROWS][6];
+#pragma unroll
+  for (int r = 0; r < SORT_ROWS; ++r) {
+    const float* b = boxes + 6 * (size_t)min(base + r * SORT_THREADS + tid, m - 1);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) bx[r][c] = b[c];
+  }
+  float mn[3], mx[3];
+  box_sentinel(mn, mx);
+  for (uint32_t q = tid; q < npart; q += SORT_THREADS) unite(mn, mx, partial + 6 * (size_t)q);
+  h[tid] = h[tid + SORT_THREADS] = 0;
+  const float v = block_box<SORT_WAVES>(mn, mx, red);
+  if (tid < 6) {
+    sroot[tid] = v;
+    if (blockIdx.x == 0) root_out[tid] = v;
+  }
+  __syncthreads();
+  const float rmin[3] = {sroot[0], sroot[1], sroot[2]};
+  const float rext[3] = {sroot[3] - sroot[0], sroot[4] - sroot[1], sroot[5] - sroot[2]};
+#pragma unroll
+  for (int r = 0; r < SORT_ROWS; ++r) {
+    const uint32_t i = base + r * SORT_THREADS + tid;
+    if (i >= m) continue;
+    const uint32_t c = box_morton(bx[r], bx[r] + 3, rmin, rext);
+    codes[i] = c;
+    atomicAdd(&h[c & (RADIX_DIGITS - 1)], 1u);
+  }
+  __syncthreads();
+  put_counts(h, pick(hist_f), nblk, by_tile);
+}
+
+__global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(PF<const uint32_t> keys_f, uint32_t n, int shift,
+                                                             PF<uint32_t> hist_f, uint32_t nblk, bool by_tile) {
+  __shared__ uint32_t h[RADIX_DIGITS];
+  const uint32_t* __restrict__ keys = pick(keys_f);
+  const uint32_t base = blockIdx.x * SORT_TILE;
+  uint32_t k[SORT_ROWS];
+#pragma unroll
+  for (int r = 0; r < SORT_ROWS; ++r) k[r] = keys[min(base + r * SORT_THREADS + threadIdx.x, n - 1)];
+  h[threadIdx.x] = h[threadIdx.x + SORT_THREADS] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < SORT_ROWS; ++r)
+    if (base + r * SORT_THREADS + threadIdx.x < n) atomicAdd(&h[(k[r] >> shift) & (RADIX_DIGITS - 1)], 1u);
+  __syncthreads();
+  put_counts(h, pick(hist_f), nblk, by_tile);
+}
+
+// Counts digit after digit: per digit, the exclusive prefix over tiles (in
+// place) and the digit's total: one wave per digit, 64 tiles per round.
 __global__ __launch_bounds__(256) void k_radix_rowscan(PF<uint32_t> hist_f, uint32_t nblk, PF<uint32_t> total_f) {
   uint32_t* __restrict__ hist = pick(hist_f);
   uint32_t* __restrict__ total = pick(total_f);
@@ -198,96 +238,127 @@ __global__ __launch_bounds__(256) void k_radix_rowscan(PF<uint32_t> hist_f, uint
   if (lane == 0) total[d] = carry;
 }
 
-// Scatter with stable ranks: within a wave, lanes holding the same digit are
-// matched with RADIX_BITS ballots; waves are ordered through per-digit LDS
-// counts.  Thread t owns digits t, t + 256, t + 512, t + 768 in the scans.
+// Scatter with stable ranks.  Wave w owns SORT_ROWS rows of 64 consecutive
+// keys; within a row the lanes of a digit are matched with RADIX_BITS
+// ballots, and a running per-digit count of the wave's rows is kept in LDS,
+// so a tile takes three barriers.  Element order = (wave, row, lane) order.
+// FIRST: the values are the indices themselves.  LAST: the sorted keys and
+// leaf triangles are written instead of the pairs.
+template <bool FIRST, bool LAST>
 __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(PF<const uint32_t> kin_f, PF<const uint32_t> vin_f,
                                                                 uint32_t n, int shift, PF<const uint32_t> hist_f,
                                                                 PF<const uint32_t> total_f, uint32_t nblk,
-                                                                PF<uint32_t> kout_f, PF<uint32_t> vout_f) {
-  __shared__ uint32_t goff[RADIX_DIGITS];
+                                                                bool by_tile, PF<uint32_t> kout_f,
+                                                                PF<uint32_t> vout_f, const uint32_t* __restrict__ tris,
+                                                                PF<uint64_t> keys_f, PF<uint4> leaf_tri_f) {
+  __shared__ __align__(16) uint32_t wcnt[SORT_WAVES][RADIX_DIGITS];
+  __shared__ uint32_t wsum[SORT_WAVES];
   const uint32_t* __restrict__ kin = pick(kin_f);
-  const uint32_t* __restrict__ vin = pick(vin_f);
   const uint32_t* __restrict__ hist = pick(hist_f);
-  const uint32_t* __restrict__ total = pick(total_f);
-  uint32_t* __restrict__ kout = pick(kout_f);
-  uint32_t* __restrict__ vout = pick(vout_f);
-  __shared__ uint32_t run[RADIX_DIGITS];
-  __shared__ uint32_t wsum[SORT_THREADS / 64];
-  __shared__ uint32_t wcnt[SORT_THREADS / 64][RADIX_DIGITS];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-  {  // digit bases: exclusive scan of the digit totals, in rounds of 256 digits
-    uint32_t carry = 0;
-    for (int q = 0; q < DIGITS_PER_THREAD; ++q) {
-      const uint32_t d = q * SORT_THREADS + tid;
-      const uint32_t v = total[d];
-      uint32_t incl = v;
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t u = __shfl_up(incl, off, 64);
-        if (lane >= (uint32_t)off) incl += u;
-      }
-      if (lane == 63) wsum[w] = incl;
-      __syncthreads();
-      uint32_t base = carry;
-      for (uint32_t k = 0; k < w; ++k) base += wsum[k];
-      goff[d] = base + incl - v + hist[(size_t)d * nblk + blockIdx.x];
-      for (uint32_t k = 0; k < SORT_THREADS / 64; ++k) carry += wsum[k];
-      __syncthreads();
-    }
-  }
-  for (int q = 0; q < DIGITS_PER_THREAD; ++q) run[q * SORT_THREADS + tid] = 0;
   const uint32_t base = blockIdx.x * SORT_TILE;
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-  for (int r = 0; r < SORT_ITEMS; ++r) {
-    for (int q = 0; q < SORT_THREADS / 64; ++q)
-      for (int k = 0; k < DIGITS_PER_THREAD; ++k) wcnt[q][k * SORT_THREADS + tid] = 0;
-    __syncthreads();
-    const uint32_t e = base + r * SORT_THREADS + tid;
-    const bool valid = e < n;
-    const uint32_t key = valid ? kin[e] : 0u, val = valid ? vin[e] : 0u;
-    const uint32_t d = (key >> shift) & (RADIX_DIGITS - 1);
-    uint64_t msk = __ballot(valid);
-    for (int b = 0; b < RADIX_BITS; ++b) {
-      const uint32_t bit = (d >> b) & 1u;
-      const uint64_t bb = __ballot(bit);
-      msk &= bit ? bb : ~bb;
-    }
-    const uint32_t rank = __popcll(msk & lt);
-    if (valid && rank == 0) wcnt[w][d] = __popcll(msk);
-    __syncthreads();
-    for (int k = 0; k < DIGITS_PER_THREAD; ++k) {
-      const uint32_t dd = k * SORT_THREADS + tid;
-      uint32_t s = run[dd];
-      for (int q = 0; q < SORT_THREADS / 64; ++q) {
-        const uint32_t c = wcnt[q][dd];
-        wcnt[q][dd] = s;
-        s += c;
-      }
-      run[dd] = s;
-    }
-    __syncthreads();
-    if (valid) {
-      const uint32_t pos = goff[d] + wcnt[w][d] + rank;
-      kout[pos] = key;
-      vout[pos] = val;
-    }
-    __syncthreads();
+  uint32_t key[SORT_ROWS], val[SORT_ROWS], loc[SORT_ROWS];
+  bool ok[SORT_ROWS];
+#pragma unroll
+  for (int r = 0; r < SORT_ROWS; ++r) {
+    const uint32_t e = base + (w * SORT_ROWS + r) * 64 + lane;
+    ok[r] = e < n;
+    key[r] = kin[min(e, n - 1)];
+    val[r] = FIRST ? e : pick(vin_f)[min(e, n - 1)];
   }
-}
 
-__global__ __launch_bounds__(256) void k_sort_finish(PF<const uint32_t> codes_f, PF<const uint32_t> idx_f,
-                                                     const uint32_t* __restrict__ tris, uint32_t m,
-                                                     PF<uint64_t> keys_f, PF<uint4> leaf_tri_f) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= m) return;
-  const uint32_t* __restrict__ codes = pick(codes_f);
-  const uint32_t* __restrict__ idx = pick(idx_f);
-  uint64_t* __restrict__ keys = pick(keys_f);
-  uint4* __restrict__ leaf_tri = pick(leaf_tri_f);
-  const uint32_t p = idx[i];
-  keys[i] = ((uint64_t)codes[i] << 32) | p;
-  const uint32_t* t = tris + 3 * (size_t)p;
-  leaf_tri[i] = make_uint4(t[0], t[1], t[2], p);
+  // the tile's first place of each of the thread's digits 2 tid, 2 tid + 1
+  uint32_t tot[2], first[2];
+  if (by_tile) {
+    // all loads of a lane in flight at once; sums of 16-bit pairs
+    uint4* part = reinterpret_cast<uint4*>(&wcnt[0][0]);      // [2][SORT_GROUPS][SORT_WORDS] words
+    const uint32_t g = tid / (SORT_WORDS / 4), q = tid % (SORT_WORDS / 4);
+    const uint4* h4 = reinterpret_cast<const uint4*>(hist) + q;
+    uint4 c[SORT_LOADS];
+#pragma unroll
+    for (int j = 0; j < SORT_LOADS; ++j)
+      c[j] = h4[(size_t)min(g + (uint32_t)(j * SORT_GROUPS), nblk - 1) * (SORT_WORDS / 4)];
+    uint4 all = make_uint4(0, 0, 0, 0), pre = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < SORT_LOADS; ++j) {
+      const uint32_t b = g + (uint32_t)(j * SORT_GROUPS);
+      const uint32_t in = b < nblk ? ~0u : 0u, be = b < blockIdx.x ? ~0u : 0u;
+      all.x += c[j].x & in; all.y += c[j].y & in; all.z += c[j].z & in; all.w += c[j].w & in;
+      pre.x += c[j].x & be; pre.y += c[j].y & be; pre.z += c[j].z & be; pre.w += c[j].w & be;
+    }
+    part[g * (SORT_WORDS / 4) + q] = all;
+    part[(SORT_GROUPS + g) * (SORT_WORDS / 4) + q] = pre;
+    __syncthreads();
+    const uint32_t* pw = &wcnt[0][0] + tid;
+    tot[0] = tot[1] = first[0] = first[1] = 0;
+#pragma unroll
+    for (int k = 0; k < SORT_GROUPS; ++k) {
+      const uint32_t a = pw[k * SORT_WORDS], p = pw[(SORT_GROUPS + k) * SORT_WORDS];
+      tot[0] += a & 0xffffu; tot[1] += a >> 16;
+      first[0] += p & 0xffffu; first[1] += p >> 16;
+    }
+  } else {
+    const uint2 t2 = reinterpret_cast<const uint2*>(pick(total_f))[tid];
+    tot[0] = t2.x; tot[1] = t2.y;
+    for (int q = 0; q < 2; ++q) first[q] = hist[(size_t)(2 * tid + q) * nblk + blockIdx.x];
+  }
+  {
+    const uint32_t v = tot[0] + tot[1];
+    uint32_t incl = v;
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t u = __shfl_up(incl, off, 64);
+      if (lane >= (uint32_t)off) incl += u;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();                       // also: the parts have been read
+    uint32_t s = incl - v;
+    for (uint32_t q = 0; q < w; ++q) s += wsum[q];
+    first[0] += s;
+    first[1] += s + tot[0];
+  }
+  for (uint32_t d = lane; d < (uint32_t)RADIX_DIGITS / 4; d += 64)
+    reinterpret_cast<uint4*>(wcnt[w])[d] = make_uint4(0, 0, 0, 0);
+
+  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+#pragma unroll
+  for (int r = 0; r < SORT_ROWS; ++r) {
+    const uint32_t d = (key[r] >> shift) & (RADIX_DIGITS - 1);
+    uint64_t msk = __ballot(ok[r]);
+#pragma unroll
+    for (int b = 0; b < RADIX_BITS; ++b) {
+      const bool on = (d >> b) & 1u;
+      const uint64_t bb = __ballot(on);
+      msk &= on ? bb : ~bb;
+    }
+    // the wave's count of this digit in its earlier rows, then this row's
+    // lanes of the digit; the lowest such lane adds the row's count
+    const uint32_t prior = wcnt[w][d], rank = __popcll(msk & lt);
+    loc[r] = prior + rank;
+    if (ok[r] && rank == 0) wcnt[w][d] = prior + (uint32_t)__popcll(msk);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < SORT_WAVES; ++v) {   // per digit: offsets of the waves' runs
+    uint2& p = reinterpret_cast<uint2*>(wcnt[v])[tid];
+    const uint2 c = p;
+    p = make_uint2(first[0], first[1]);
+    first[0] += c.x;
+    first[1] += c.y;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < SORT_ROWS; ++r) {
+    if (!ok[r]) continue;
+    const uint32_t pos = wcnt[w][(key[r] >> shift) & (RADIX_DIGITS - 1)] + loc[r];
+    if constexpr (LAST) {
+      pick(keys_f)[pos] = ((uint64_t)key[r] << 32) | val[r];
+      const uint32_t* t = tris + 3 * (size_t)val[r];
+      pick(leaf_tri_f)[pos] = make_uint4(t[0], t[1], t[2], val[r]);
+    } else {
+      pick(kout_f)[pos] = key[r];
+      pick(vout_f)[pos] = val[r];
+    }
+  }
 }
 
 // ------------------------------------------------------------ Karras build
@@ -315,8 +386,8 @@ void Body::build_levels(int F, const int* ks, const int* ls, hipStream_t s) {
   for (int f = 0; f < F; ++f) {
     Lane& L = lane[ls[f]];
     Slot& S = slot[ks[f]];
-    fr[f] = LvFrame{L.keys.p, leaf_tri_of(ks[f]), L.boxes.p, {L.items[0].p, L.items[1].p},
-                    {L.nitems[0].p, L.nitems[1].p}, S.nodes.p, L.leaf_parent.p, S.root.p, S.leaf0_box.p};
+    fr[f] = LvFrame{L.keys.p, L.boxes.p, {L.items[0].p, L.items[1].p},
+                    {L.nitems[0].p, L.nitems[1].p}, S.nodes.p, S.root.p, S.leaf0_box.p};
   }
   launch_build_levels(bu_desc.p, tabs, bu_n, fr, F, s);
 }
@@ -493,20 +564,21 @@ void Body::build_frames(int F, const int* ks, const int* ls, hipStream_t s) {
   const uint32_t nblk_box = lane[ls[0]].nblk_box;
   k_prim_boxes<<<dim3(nblk_box, nf), BOX_THREADS, 0, s>>>(verts, tris.p, m, depth, boxes, partial);
   CC_LAUNCHED();
-  k_morton<<<dim3(grid_for(m, 256), nf), 256, 0, s>>>(boxes_c, m, partial_c, nblk_box, code[0], idx[0], root);
-  CC_LAUNCHED();
   const uint32_t nblk = grid_for(m, SORT_TILE);
-  int src = 0;
-  for (int pass = 0, shift = 0; pass < RADIX_PASSES; ++pass, shift += RADIX_BITS) {
-    k_radix_hist<<<dim3(nblk, nf), SORT_THREADS, 0, s>>>(code_c[src], m, shift, hist, nblk);
-    k_radix_rowscan<<<dim3(RADIX_DIGITS / 4, nf), 256, 0, s>>>(hist, nblk, total);
-    k_radix_scatter<<<dim3(nblk, nf), SORT_THREADS, 0, s>>>(code_c[src], idx_c[src], m, shift, hist_c, total_c,
-                                                            nblk, code[src ^ 1], idx[src ^ 1]);
-    CC_LAUNCHED();
-    src ^= 1;
-  }
-  k_sort_finish<<<dim3(grid_for(m, 256), nf), 256, 0, s>>>(code_c[src], idx_c[src], tris.p, m, keys, leaf);
+  const bool by_tile = nblk <= SORT_SCAN_BLOCKS;
+  const dim3 tiles(nblk, nf);
+  k_morton<<<tiles, SORT_THREADS, 0, s>>>(boxes_c, m, partial_c, nblk_box, code[0], hist, nblk, by_tile, root);
   CC_LAUNCHED();
+  for (int pass = 0, shift = 0; pass < RADIX_PASSES; ++pass, shift += RADIX_BITS) {
+    const int src = pass & 1, dst = src ^ 1;
+    if (pass) k_radix_hist<<<tiles, SORT_THREADS, 0, s>>>(code_c[src], m, shift, hist, nblk, by_tile);
+    if (!by_tile) k_radix_rowscan<<<dim3(RADIX_DIGITS / 4, nf), 256, 0, s>>>(hist, nblk, total);
+    auto scatter = pass == 0 ? k_radix_scatter<true, false>
+                   : pass + 1 < RADIX_PASSES ? k_radix_scatter<false, false> : k_radix_scatter<false, true>;
+    scatter<<<tiles, SORT_THREADS, 0, s>>>(code_c[src], idx_c[src], m, shift, hist_c, total_c, nblk, by_tile, code[dst],
+                                           idx[dst], tris.p, keys, leaf);
+    CC_LAUNCHED();
+  }
   if (bottom_up) {                      // tree, parent links and boxes, bottom-up
     build_levels(F, ks, ls, s);
     fold_frames(F, ks, s);
@@ -567,18 +639,17 @@ void Body::update(int k, int l, uint64_t frame, hipStream_t s) {
   }
 }
 
-void export_tree_raw(uint32_t m, const uint64_t* keys_d, const uint4* leaf_tri_d, const int32_t* leaf_parent_d,
-                     const Node* nodes_d, const float* root_d, const float* leaf0_d, uint64_t* okeys,
+// The parents follow from the child links (the bottom-up build stores none).
+void export_tree_raw(uint32_t m, const uint64_t* keys_d, const uint4* leaf_tri_d, const Node* nodes_d,
+                     const float* root_d, const float* leaf0_d, uint64_t* okeys,
                      uint32_t* order, int32_t* childA, int32_t* childB, int32_t* parent_int, int32_t* parent_leaf,
                      float* box_int, float* box_leaf, float* root6, hipStream_t s) {
   std::vector<uint64_t> kk(m);
   std::vector<uint4> lt(m);
-  std::vector<int32_t> lp(m);
   std::vector<Node> nd(m >= 2 ? m - 1 : 0);
   float r[6], l0[6];
   CC_HIP(hipMemcpyAsync(kk.data(), keys_d, m * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   CC_HIP(hipMemcpyAsync(lt.data(), leaf_tri_d, m * sizeof(uint4), hipMemcpyDeviceToHost, s));
-  CC_HIP(hipMemcpyAsync(lp.data(), leaf_parent_d, m * sizeof(int32_t), hipMemcpyDeviceToHost, s));
   if (!nd.empty())
     CC_HIP(hipMemcpyAsync(nd.data(), nodes_d, nd.size() * sizeof(Node), hipMemcpyDeviceToHost, s));
   CC_HIP(hipMemcpyAsync(r, root_d, sizeof(r), hipMemcpyDeviceToHost, s));
@@ -594,6 +665,12 @@ void export_tree_raw(uint32_t m, const uint64_t* keys_d, const uint4* leaf_tri_d
     if (parent_leaf) parent_leaf[0] = 0;
     return;
   }
+  std::vector<int32_t> lp(m, 0), np(m - 1, -1);
+  for (uint32_t x = 0; x + 1 < m; ++x)
+    for (const int32_t c : {nd[x].childA, nd[x].childB}) {
+      CC_REQUIRE(c < 0 ? (uint32_t)~c < m : (uint32_t)c < m - 1, "bvh export: child link out of range");
+      (c < 0 ? lp[~c] : np[c]) = (int32_t)x;
+    }
   auto slot_of_child = [&](int32_t par, int32_t child, float* dst) {
     const Node& p = nd[par];
     const float* src = (p.childA == child) ? p.a_min : p.b_min;
@@ -603,10 +680,10 @@ void export_tree_raw(uint32_t m, const uint64_t* keys_d, const uint4* leaf_tri_d
     const Node& n = nd[x];
     if (childA) childA[x] = n.childA >= 0 ? n.childA + 1 : n.childA;   // ~l == -(l+1)
     if (childB) childB[x] = n.childB >= 0 ? n.childB + 1 : n.childB;
-    if (parent_int) parent_int[x] = n.parent + 1;
+    if (parent_int) parent_int[x] = np[x] + 1;
     if (box_int) {
-      if (n.parent < 0) std::memcpy(box_int + 6 * (size_t)x, r, sizeof(r));
-      else slot_of_child(n.parent, (int32_t)x, box_int + 6 * (size_t)x);
+      if (np[x] < 0) std::memcpy(box_int + 6 * (size_t)x, r, sizeof(r));
+      else slot_of_child(np[x], (int32_t)x, box_int + 6 * (size_t)x);
     }
   }
   for (uint32_t l = 0; l < m; ++l) {
@@ -621,7 +698,7 @@ void Body::export_tree(int k, uint64_t* okeys, uint32_t* order, int32_t* childA,
   CC_REQUIRE(mode != CC_BODY_NONE, "bvh export: no body");
   const Lane& L = lane[0];
   const Slot& S = slot[k];
-  export_tree_raw(m, L.keys.p, leaf_tri_of(k), L.leaf_parent.p, S.nodes.p, S.root.p, S.leaf0_box.p, okeys, order,
+  export_tree_raw(m, L.keys.p, leaf_tri_of(k), S.nodes.p, S.root.p, S.leaf0_box.p, okeys, order,
                   childA, childB, parent_int, parent_leaf, box_int, box_leaf, root6, s);
 }
 
