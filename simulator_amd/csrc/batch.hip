@@ -59,16 +59,19 @@ struct Batch {
   int tile = 256, order = 0;
   DBuf<uint4> blocks;
   uint32_t nblocks = 0;
-  // moving bodies: the step runs inside the sort's launch (k_bb_sort_step)
-  // with its own tile, tuned on that launch
-  int fused_tile = 256;
-  DBuf<uint4> fblocks;
-  uint32_t nfblocks = 0;
   int cur = 0;
   hipGraphExec_t graphs[2] = {nullptr, nullptr};
+  // moving bodies: the step runs beside the body launches, on a stream of its
+  // own between two events
+  hipStream_t side = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 
   ~Batch() {
     if (stream) (void)hipStreamSynchronize(stream);   // before the buffers are freed
+    if (side) (void)hipStreamSynchronize(side);
+    if (ev_fork) (void)hipEventDestroy(ev_fork);
+    if (ev_join) (void)hipEventDestroy(ev_join);
+    if (side) (void)hipStreamDestroy(side);
     for (hipGraphExec_t& g : graphs)
       if (g) (void)hipGraphExecDestroy(g);
     if (stream) (void)hipStreamDestroy(stream);
@@ -87,7 +90,7 @@ struct Batch {
     for (uint32_t k : inst)
       for (uint32_t v = v_off[k]; v < v_off[k + 1]; v += (uint32_t)T)
         t.push_back(make_uint4(k, v, std::min<uint32_t>((uint32_t)T, v_off[k + 1] - v), 0u));
-    return t;
+    return bodies.xcd.arrange(t, [](const uint4& e) { return e.x; });
   }
 
   template <int T>
@@ -111,17 +114,8 @@ struct Batch {
       launch_t<256>(blk, nblk, s);
   }
 
-  StepLaunch fused_launch(const uint4* blk, uint32_t nblk, int T) const {
-    return StepLaunch{state[cur].p, state[cur ^ 1].p, contact.p, row.p, ell_w ? ell.p : rec.p, insts[cur].p,
-                      blk, nblk, ntotal, spill.p, (uint32_t)ell_w, (uint32_t)T};
-  }
-
-  // Time every (tile, order) candidate over a few steps from the initial
-  // state on the launch the steps will use -- the plain step kernel, or,
-  // with moving bodies, the sort's launch that carries the step -- keep the
-  // fastest, and restore the initial state.  (The sort in the timed fused
-  // launches re-sorts the set-up's boxes into the next slot, which every
-  // step rebuilds before reading.)
+  // Time every (tile, order) candidate of the step kernel over a few steps
+  // from the initial state, keep the fastest, and restore the initial state.
   void autotune() {
     const size_t n6 = 6 * (size_t)ntotal, n3 = 3 * (size_t)ntotal;
     DBuf<float> s0, c0;
@@ -131,7 +125,6 @@ struct Batch {
     CC_HIP(hipMemcpyAsync(c0.p, contact.p, n3 * sizeof(float), hipMemcpyDeviceToDevice, stream));
     const Events<2> ev;
     const hipEvent_t e0 = ev[0], e1 = ev[1];
-    const bool fused = bodies.moving && bodies.step.n_sort;
     float best = 1e30f;
     for (int T : TILES)
       for (int ord = 0; ord < 2; ++ord) {
@@ -139,10 +132,7 @@ struct Batch {
         DBuf<uint4> blk;
         blk.upload(t.data(), t.size(), stream);
         auto run = [&] {
-          if (fused)
-            bodies.sort_with_step(bodies.step, cur ^ 1, fused_launch(blk.p, (uint32_t)t.size(), T), stream);
-          else
-            launch(T, blk.p, (uint32_t)t.size(), stream);
+          launch(T, blk.p, (uint32_t)t.size(), stream);
           cur ^= 1;
         };
         for (int k = 0; k < 3; ++k) run();     // warm-up
@@ -162,34 +152,30 @@ struct Batch {
     cur = 0;
     CC_HIP(hipMemcpyAsync(state[0].p, s0.p, n6 * sizeof(float), hipMemcpyDeviceToDevice, stream));
     CC_HIP(hipMemcpyAsync(contact.p, c0.p, n3 * sizeof(float), hipMemcpyDeviceToDevice, stream));
-    // the set-up's frame-0 bodies again in both slots the timed sorts wrote
-    if (fused) {
-      bodies.launch(bodies.all, 0, 0, stream);
-      bodies.launch(bodies.all, 0, 1, stream);
-    }
     const std::vector<uint4> t = block_table(tile, order);
     blocks.upload(t.data(), t.size(), stream);
     nblocks = (uint32_t)t.size();
-    fused_tile = tile;
-    fblocks.upload(t.data(), t.size(), stream);
-    nfblocks = (uint32_t)t.size();
     CC_HIP(hipStreamSynchronize(stream));
   }
   float tuned[3][2] = {};                    // ms per step of each (tile, order) candidate
 
   // One step of frame `frame` (cur == frame % 2): the moving bodies of frame
   // + 1 are posed, sorted and built into the other slot while the cloths step
-  // against the bodies of this frame; k selects frame + 1's motion.
+  // against the bodies of this frame; k selects frame + 1's motion.  The step
+  // has a branch of its own, between two events (in a captured block a branch
+  // of the graph): the body launches leave CUs idle at their ends, and with
+  // few instances most of the time.  Measured, one stream / two: 608 / 588 us
+  // per step of 256 instances, 110 / 92 of 16, 78 / 57 of 16 with refitted
+  // bodies.
   void one_step(int k, hipStream_t s) {
     const int nxt = cur ^ 1;
     if (bodies.moving) {
-      bodies.pre(bodies.step, k, nxt, s);
-      if (bodies.step.n_sort) {
-        bodies.sort_with_step(bodies.step, nxt, fused_launch(fblocks.p, nfblocks, fused_tile), s);
-      } else {
-        launch(tile, blocks.p, nblocks, s);
-      }
-      bodies.post(bodies.step, nxt, s);
+      CC_HIP(hipEventRecord(ev_fork, s));
+      CC_HIP(hipStreamWaitEvent(side, ev_fork, 0));
+      launch(tile, blocks.p, nblocks, side);
+      CC_HIP(hipEventRecord(ev_join, side));
+      bodies.launch(bodies.step, k, nxt, s);
+      CC_HIP(hipStreamWaitEvent(s, ev_join, 0));
     } else {
       launch(tile, blocks.p, nblocks, s);
     }
@@ -326,7 +312,9 @@ int cc_batch_create(const cc_cloth_desc* cloths, const cc_body_desc* bodies, con
     }
     alloc_spill(B.spill, B.ntotal, s);
     // bodies: concatenated, frame 0 built for all of them
-    B.bodies.init(bodies, params, count, s);
+    std::vector<uint32_t> cloth_n(count);
+    for (uint32_t k = 0; k < count; ++k) cloth_n[k] = cloths[k].n;
+    B.bodies.init(bodies, params, cloth_n, count, s);
     std::vector<InstDesc> desc(count);
     for (uint32_t k = 0; k < count; ++k) {
       desc[k].a = step_args(params[k], cloths[k].ntypes);
@@ -335,6 +323,11 @@ int cc_batch_create(const cc_cloth_desc* cloths, const cc_body_desc* bodies, con
     for (int slot = 0; slot < 2; ++slot) {
       for (uint32_t j = 0; j < B.bodies.nb; ++j) desc[B.bodies.inst[j]].bvh = B.bodies.view(j, slot);
       B.insts[slot].upload(desc.data(), desc.size(), s);
+    }
+    if (B.bodies.moving) {
+      CC_HIP(hipStreamCreateWithFlags(&B.side, hipStreamNonBlocking));
+      CC_HIP(hipEventCreate(&B.ev_fork));
+      CC_HIP(hipEventCreate(&B.ev_join));
     }
     CC_HIP(hipStreamSynchronize(s));
     B.autotune();
@@ -443,7 +436,7 @@ int cc_batch_tuning(cc_batch* b, float ms[6], uint32_t* fused) {
     if (ms)
       for (int t = 0; t < 3; ++t)
         for (int o = 0; o < 2; ++o) ms[2 * t + o] = B.tuned[t][o];
-    if (fused) *fused = (B.bodies.moving && B.bodies.step.n_sort) ? 1u : 0u;
+    if (fused) *fused = 0u;   // the step has a launch of its own
   });
 }
 

@@ -3,14 +3,9 @@
 // Per frame, for all bodies at once:
 //   k_bb_deform  grid over body vertices      capsule breathing + rigid motion
 //   k_bb_boxes   grid over triangles          expanded boxes + per-block root boxes
-//   k_bb_sort    one workgroup per body       root box, Morton codes, stable
-//                                             4 x 8-bit LSD sort of (code, primitive)
+//   launch_sort  tiles of 1024 keys           root box, Morton codes, sort (sort.hip)
 //   k_bb_level   chunks of 1024 leaves, then  tree and boxes by splits, in LDS
 //                of unfinished nodes
-// The one-workgroup-per-body passes keep every cross-thread exchange inside
-// a workgroup (LDS counters, barriers): bodies are 2k-40k triangles, so one
-// workgroup per body still spreads the batch over the chip, and nothing
-// needs an agent-scope arrival protocol (on MI355X each XCD has its own L2).
 // Poses, keys, topology and boxes equal the single-body path bit for bit:
 // the arithmetic is the shared routines of cc_lbvh.h, the sort is stable
 // from ascending primitive order (so it orders the full 64-bit key), and
@@ -21,28 +16,12 @@
 
 #include "cc_bbody.h"
 #include "cc_lbvh.h"
-#include "cc_step.h"
 
 namespace cc {
 
 constexpr int BB_BLOCK = 256;       // vertices / triangles / nodes per block of the grid kernels
-constexpr int SB_THREADS = 1024;    // threads of the per-body sort
-constexpr int SB_WAVES = SB_THREADS / 64;
-constexpr int SB_ROWS = 8;          // rows of 64 elements per wave per sort tile
-constexpr int SB_TILE = SB_THREADS * SB_ROWS;
-constexpr int SB_BATCH = 4;         // elements per thread per round of the code and key loops
-constexpr int SB_BITS = 10;         // digit width: three passes cover the 30-bit Morton codes
-constexpr int SB_DIGITS = 1 << SB_BITS;
-constexpr int SB_PASSES = 3;
 constexpr uint32_t BB_MAX_M = 1u << 19;   // triangles per batched body
-
-// Barrier ordering LDS accesses only: the global stores issued before it
-// stay in flight (a full __syncthreads waits for them).
-__device__ inline void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
+static_assert(BB_BLOCK == BOX_BLOCK, "one partial root box per BOX_BLOCK triangles");
 
 // ------------------------------------------------------------ pose
 __global__ __launch_bounds__(BB_BLOCK) void k_bb_deform(const BodyDesc* __restrict__ desc,
@@ -105,208 +84,6 @@ __global__ __launch_bounds__(BB_BLOCK) void k_bb_boxes(const BodyDesc* __restric
   }
 }
 
-// ------------------------------------------------------------ sort
-// One workgroup per body.  Three passes of 10-bit digits (the Morton codes
-// have 30 bits); the digit counts of all passes come from one sweep over the
-// codes.  A pass walks tiles of SB_TILE elements; wave w owns rows
-// w*SB_ROWS .. w*SB_ROWS+7 of 64 consecutive elements, ranks each row's
-// lanes by digit with 10 ballots, and keeps a running per-digit count of its
-// rows in LDS, so a tile needs three barriers whatever its size (LDS-only
-// ones: a pass's scattered stores are waited for once, at its end).
-// Element order = (wave, row, lane) order, so the pass is stable.
-__device__ inline void bb_sort(uint32_t j, const BodyDesc* __restrict__ desc, const float* __restrict__ boxes,
-                               const float* __restrict__ partial, uint2* kv0, uint2* kv1,
-                               uint64_t* __restrict__ keys, uint4* __restrict__ leaf_tri,
-                               const uint32_t* __restrict__ tris, float* __restrict__ root) {
-  __shared__ uint32_t hist[SB_PASSES][SB_DIGITS];
-  __shared__ uint32_t wcnt[SB_WAVES][SB_DIGITS];
-  __shared__ uint32_t run[SB_DIGITS];
-  __shared__ uint32_t wtot[SB_WAVES];
-  __shared__ float red[SB_WAVES][6];
-  __shared__ float sroot[6];
-  const BodyDesc d = desc[j];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-  const uint32_t m = d.m, t0 = d.t0;
-
-  // root box: sentinel U the body's per-block boxes (k_morton's reduction)
-  float mn[3], mx[3];
-  box_sentinel(mn, mx);
-  const uint32_t np = (m + BB_BLOCK - 1) / BB_BLOCK;
-  for (uint32_t q = tid; q < np; q += SB_THREADS) unite(mn, mx, partial + 6 * (size_t)(d.p0 + q));
-  for (int off = 32; off > 0; off >>= 1)
-    for (int c = 0; c < 3; ++c) {
-      mn[c] = fminf(mn[c], __shfl_xor(mn[c], off, 64));
-      mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], off, 64));
-    }
-  if (lane == 0) put6(red[w], mn, mx);
-  for (uint32_t q = tid; q < SB_PASSES * SB_DIGITS; q += SB_THREADS) (&hist[0][0])[q] = 0;
-  __syncthreads();
-  if (tid < 6) {
-    float v = red[0][tid];
-    for (int q = 1; q < SB_WAVES; ++q) v = tid < 3 ? fminf(v, red[q][tid]) : fmaxf(v, red[q][tid]);
-    sroot[tid] = v;
-    root[6 * (size_t)j + tid] = v;
-  }
-  __syncthreads();
-  const float rmin[3] = {sroot[0], sroot[1], sroot[2]};
-  const float rext[3] = {sroot[3] - sroot[0], sroot[4] - sroot[1], sroot[5] - sroot[2]};
-
-  // codes (compute_morton_bbox, bvh.cu:71-79) and the digit counts
-  // (SB_BATCH elements per thread per round, loads issued together)
-  for (uint32_t base = 0; base < m; base += SB_BATCH * SB_THREADS) {
-    float bxs[SB_BATCH][6];
-#pragma unroll
-    for (int u = 0; u < SB_BATCH; ++u) {
-      const uint32_t t = min(base + u * SB_THREADS + tid, m - 1);
-      const float* bx = boxes + 6 * (size_t)(t0 + t);
-#pragma unroll
-      for (int c = 0; c < 6; ++c) bxs[u][c] = bx[c];
-    }
-#pragma unroll
-    for (int u = 0; u < SB_BATCH; ++u) {
-      const uint32_t t = base + u * SB_THREADS + tid;
-      if (t >= m) continue;
-      const uint32_t c = box_morton(bxs[u], bxs[u] + 3, rmin, rext);
-      kv0[t0 + t] = make_uint2(c, t);
-#pragma unroll
-      for (int p = 0; p < SB_PASSES; ++p) atomicAdd(&hist[p][(c >> (SB_BITS * p)) & (SB_DIGITS - 1)], 1u);
-    }
-  }
-  __syncthreads();
-  // exclusive scans of the counts, one pass at a time: thread = digit
-  static_assert(SB_DIGITS == SB_THREADS, "one digit per thread in the scans");
-  for (int p = 0; p < SB_PASSES; ++p) {
-    const uint32_t v = hist[p][tid];
-    uint32_t incl = v;
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t u = __shfl_up(incl, off, 64);
-      if (lane >= (uint32_t)off) incl += u;
-    }
-    if (lane == 63) wtot[w] = incl;
-    __syncthreads();
-    uint32_t base = 0;
-    for (uint32_t q = 0; q < w; ++q) base += wtot[q];
-    hist[p][tid] = base + incl - v;
-    __syncthreads();
-  }
-
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-  for (int p = 0; p < SB_PASSES; ++p) {
-    const uint2* src = ((p & 1) ? kv1 : kv0) + t0;
-    uint2* dst = ((p & 1) ? kv0 : kv1) + t0;
-    const int shift = SB_BITS * p;
-    run[tid] = hist[p][tid];
-    for (uint32_t base = 0; base < m; base += SB_TILE) {
-      for (uint32_t q = lane; q < (uint32_t)SB_DIGITS; q += 64) wcnt[w][q] = 0;
-      uint2 e[SB_ROWS];
-      uint32_t dg[SB_ROWS], loc[SB_ROWS];
-      bool ok[SB_ROWS];
-#pragma unroll
-      for (int r = 0; r < SB_ROWS; ++r) {
-        const uint32_t idx = base + (w * SB_ROWS + r) * 64 + lane;
-        ok[r] = idx < m;
-        e[r] = src[ok[r] ? idx : 0];
-      }
-#pragma unroll
-      for (int r = 0; r < SB_ROWS; ++r) {
-        dg[r] = (e[r].x >> shift) & (SB_DIGITS - 1);
-        uint64_t msk = __ballot(ok[r]);
-#pragma unroll
-        for (int bit = 0; bit < SB_BITS; ++bit) {
-          const bool on = (dg[r] >> bit) & 1u;
-          const uint64_t bb = __ballot(on);
-          msk &= on ? bb : ~bb;
-        }
-        // the wave's count of this digit in its earlier rows, then this
-        // row's lanes of the digit; the lowest such lane adds the row's
-        // count (reads of the row precede its write within the wave)
-        const uint32_t prior = wcnt[w][dg[r]];
-        const uint32_t rank = __popcll(msk & lt);
-        loc[r] = prior + rank;
-        if (ok[r] && rank == 0) wcnt[w][dg[r]] = prior + (uint32_t)__popcll(msk);
-      }
-      lds_barrier();
-      {                                // per digit: offsets of the waves' runs
-        uint32_t s = run[tid];
-        for (int q = 0; q < SB_WAVES; ++q) {
-          const uint32_t c = wcnt[q][tid];
-          wcnt[q][tid] = s;
-          s += c;
-        }
-        run[tid] = s;
-      }
-      lds_barrier();
-#pragma unroll
-      for (int r = 0; r < SB_ROWS; ++r) {
-        const uint32_t pos = wcnt[w][dg[r]] + loc[r];
-        if (ok[r] && pos < m) dst[pos] = e[r];       // pos < m always; the test keeps stores in the body
-      }
-      lds_barrier();                   // wcnt is reused; the scattered stores may still be in flight
-    }
-    __syncthreads();                   // the pass's stores are visible to the next pass's loads
-  }
-  // the passes end in kv1 (odd count) or kv0: keys (morton << 32 | primitive) and leaves
-  const uint2* sorted = ((SB_PASSES & 1) ? kv1 : kv0) + t0;
-  for (uint32_t base = 0; base < m; base += SB_BATCH * SB_THREADS) {
-    uint2 e[SB_BATCH];
-    uint32_t tv[SB_BATCH][3];
-#pragma unroll
-    for (int u = 0; u < SB_BATCH; ++u) e[u] = sorted[min(base + u * SB_THREADS + tid, m - 1)];
-#pragma unroll
-    for (int u = 0; u < SB_BATCH; ++u) {
-      const uint32_t* t = tris + 3 * ((size_t)t0 + min(e[u].y, m - 1));
-      tv[u][0] = t[0];
-      tv[u][1] = t[1];
-      tv[u][2] = t[2];
-    }
-#pragma unroll
-    for (int u = 0; u < SB_BATCH; ++u) {
-      const uint32_t i = base + u * SB_THREADS + tid;
-      if (i >= m) continue;
-      keys[t0 + i] = ((uint64_t)e[u].x << 32) | e[u].y;
-      leaf_tri[t0 + i] = make_uint4(tv[u][0], tv[u][1], tv[u][2], e[u].y);
-    }
-  }
-}
-
-__global__ __launch_bounds__(SB_THREADS) void k_bb_sort(const BodyDesc* __restrict__ desc,
-                                                        const uint32_t* __restrict__ list,
-                                                        const float* __restrict__ boxes,
-                                                        const float* __restrict__ partial, uint2* kv0, uint2* kv1,
-                                                        uint64_t* __restrict__ keys, uint4* __restrict__ leaf_tri,
-                                                        const uint32_t* __restrict__ tris,
-                                                        float* __restrict__ root) {
-  bb_sort(list[blockIdx.x], desc, boxes, partial, kv0, kv1, keys, leaf_tri, tris, root);
-}
-
-// The sort's workgroups, then one cloth step of the batch in workgroups of
-// SB_THREADS / TILE tiles of TILE vertices (the sort of frame g + 1 and the
-// step of frame g read and write disjoint buffers).
-template <int EW, int TILE>
-__global__ __launch_bounds__(SB_THREADS) void k_bb_sort_step(const BodyDesc* __restrict__ desc,
-                                                             const uint32_t* __restrict__ list, uint32_t nsort,
-                                                             const float* __restrict__ boxes,
-                                                             const float* __restrict__ partial, uint2* kv0,
-                                                             uint2* kv1, uint64_t* __restrict__ keys,
-                                                             uint4* __restrict__ leaf_tri,
-                                                             const uint32_t* __restrict__ tris,
-                                                             float* __restrict__ root, StepLaunch st) {
-  if (blockIdx.x < nsort) {
-    bb_sort(list[blockIdx.x], desc, boxes, partial, kv0, kv1, keys, leaf_tri, tris, root);
-    return;
-  }
-  const uint32_t e = (blockIdx.x - nsort) * (SB_THREADS / TILE) + threadIdx.x / TILE;
-  if (e >= st.nblocks) return;
-  const uint4 b = st.blocks[e];
-  const uint32_t lt = threadIdx.x % TILE;
-  if (lt >= b.z) return;
-  const InstDesc dd = st.insts[b.x];
-  const uint32_t i = b.y + lt;
-  uint32_t visits = 0;
-  step_vertex<false, EW, false, 6>(i, st.in, st.out, st.contact, st.contact, st.row, st.rec, dd.a, dd.bvh, spill_of(st.spill, i, st.ntotal),
-                     visits, nullptr, nullptr, nullptr);
-}
-
 // ------------------------------------------------------------ tree + boxes
 // The Karras tree (processInternalNode, cudaBRT.cu:9-161) with its boxes
 // (calculateBoudingBox, cudaBRT.cu:166-206), by splits.  Every boundary between
@@ -364,6 +141,23 @@ __device__ inline Box6 box_node(const Box6& b) {
   return r;
 }
 
+// One round of the range boxes (see k_bb_level): u holds the boxes of the runs
+// of 2^Q items, v gets those of 2^(Q+1).
+template <int Q>
+__device__ inline void level_round(const float2 (*u)[3], float2 (*v)[3], bool have, int32_t k, int32_t n, int32_t l,
+                                   int32_t r, int32_t qa, int32_t qb, bool more, Box6& run, Box6& A, Box6& B) {
+  constexpr int32_t w = 1 << Q;
+  if (qa == Q) A = box_or(lds_box(u, l), lds_box(u, k - w + 1));
+  if (qb == Q) B = box_or(lds_box(u, k + 1), lds_box(u, r - w + 1));
+  if (!more) return;
+  if (have) {
+    // (a run past the chunk's end stays as it is: nothing reads it)
+    if (k + w < n) run = box_or(run, lds_box(u, k + w));
+    lds_box_put(v, k, run);
+  }
+  __syncthreads();
+}
+
 // One level of the build: one thread per item, and per split between two
 // items.  Boxes of ranges are unions of two overlapping power-of-two runs: in
 // round q the workgroup holds the box of every run of 2^q items in LDS (each
@@ -371,18 +165,21 @@ __device__ inline Box6 box_node(const Box6& b) {
 // children's lengths lie in [2^q, 2^(q+1)) read theirs.  Ten rounds of one
 // LDS read and a barrier for 1024 items, every lane at work, where climbing
 // from the leaves node by node took up to twenty dependent steps of an LDS
-// atomic and a read with fewer lanes at each.  Three frames of 50,688
-// triangles: 16.4 us at level 0 and 10.2 at each of the two above, against
-// 22.8 and 19.0 climbing; the 4.2 M triangles of 256 bodies: 160 us at level
-// 0 against 199 (3.2 TB/s of keys, gathered boxes and nodes written).
+// atomic and a read with fewer lanes at each.  Bound by latency for one body
+// (the loads, the searches, the barriers) and by the vector instructions at
+// level 0 of a batch, hence the rounds written out and the searches on byte
+// offsets.  Three frames of 50,688 triangles: 16.4 us at level 0 and
+// 9.6 at each of the two above, against 22.8 and 19.0 climbing; the 4.2 M
+// triangles of 256 bodies: 159 us at level 0 against 199 (3.3 TB/s of keys,
+// gathered boxes and triangles, leaves and nodes written).
 template <bool LEAVES>
-__global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ desc, const LvBlock* __restrict__ blk,
-                                                   PF<const uint64_t> keys_f, PF<const float> boxes_f,
-                                                   PF<const BItem> items_in_f,
+__global__ __launch_bounds__(LV_C) void k_bb_level(const LvBlock* __restrict__ blk, PF<const uint64_t> keys_f,
+                                                   const uint32_t* __restrict__ tris, PF<const float> boxes_f,
+                                                   PF<uint4> leaf_f, PF<const BItem> items_in_f,
                                                    PF<const uint32_t> cnt_in_f, PF<BItem> items_out_f,
                                                    PF<uint32_t> cnt_out_f, PF<Node> nodes_f, PF<float> root_f,
                                                    PF<float> leaf0_f) {
-  __shared__ uint64_t sK[LV_C];          // a key of item k
+  __shared__ uint64_t sK[LV_C + 2];      // [1 + k] a key of item k; no key on either side
   __shared__ float2 U[2][LV_C][3];       // boxes of the runs of 2^q items from item k
   __shared__ int32_t sD[LV_C];           // delta at the boundary right of item k
   __shared__ int32_t sR[LV_C];           // last leaf of item k
@@ -392,8 +189,7 @@ __global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ 
   __shared__ int32_t qmax, sfirst, sdl;  // rounds needed; first leaf, and the delta left of it
   const LvBlock b = blk[blockIdx.x];
   const uint32_t tid = threadIdx.x;
-  const BodyDesc d = desc[b.body];
-  Node* N = pick(nodes_f) + d.n0;
+  Node* N = pick(nodes_f) + b.n0;
   float* R = pick(root_f) + 6 * (size_t)b.body;
   const float* box_src = nullptr;        // this thread's item's box
   int32_t n, k, gl = 0, gr = 0, dl = -1, dr = -1;
@@ -401,16 +197,21 @@ __global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ 
   Box6 run{};
   bool have;
   if constexpr (LEAVES) {
-    const int32_t m = (int32_t)d.m, c0 = (int32_t)b.q * LV_C;
+    const int32_t m = (int32_t)b.n_in, c0 = (int32_t)b.q * LV_C;
     n = min(LV_C, m - c0);
     k = (int32_t)tid;
     have = k < n;
     gl = gr = min(c0 + k, m - 1);
-    const uint64_t* K = pick(keys_f) + d.t0;
+    const uint64_t* K = pick(keys_f) + b.t0;
     const uint64_t ka = K[max(gl - 1, 0)], kc = K[min(gl + 1, m - 1)];
     key = K[gl];
-    box_src = pick(boxes_f) + 6 * ((size_t)d.t0 + (uint32_t)key);   // the key's low half is its primitive
+    const size_t prim = (size_t)b.t0 + (uint32_t)key;   // the key's low half is its primitive
+    box_src = pick(boxes_f) + 6 * prim;
     for (int c = 0; c < 6; ++c) run.v[c] = box_src[c];
+    if (b.write_leaves) {
+      const uint32_t* t = tris + 3 * prim;
+      if (have) pick(leaf_f)[(size_t)b.t0 + gl] = make_uint4(t[0], t[1], t[2], (uint32_t)key);
+    }
     dl = gl > 0 ? __clzll(ka ^ key) : -1;
     dr = gl + 1 < m ? __clzll(key ^ kc) : -1;
     if (m == 1) {                          // a single leaf: no internal node
@@ -453,9 +254,10 @@ __global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ 
   if (tid == 0) {
     npend = 0;
     qmax = -1;
+    sK[0] = sK[n + 1] = ~0ull;             // differs from every key (30-bit codes) in the top bit
   }
   if (have) {
-    sK[k] = key;
+    sK[1 + k] = key;
     sD[k] = dr;
     if (!LEAVES) sR[k] = gr;
     lds_box_put(U[0], k, run);
@@ -466,22 +268,25 @@ __global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ 
   }
   __syncthreads();
 
-  // the range [l, r] of the split right of this item
+  // the range [l, r] of the split right of this item: the keys that differ
+  // from this one in the bits of `rest` only
   int32_t l = k, r = k, ndl = 0, ndr = 0;
   bool node = false;
   if (have && k < n - 1) {
-    const uint64_t rest = ~0ull >> dr;     // keys of the range differ from this one in these bits only
-    int32_t lo = 0, hi = n - 1;            // l in [lo, k], r in [k + 1, hi]
-    r = k + 1;
-    for (int step = 0; step < LV_LOG; ++step) {
-      const int32_t ml = (lo + l) >> 1, mr = (r + hi + 1) >> 1;
-      const uint64_t xl = sK[ml] ^ key, xr = sK[mr] ^ key;
-      const bool il = xl <= rest, ir = xr <= rest;
-      l = il ? ml : l;
-      lo = il ? lo : ml + 1;
-      r = ir ? mr : r;
-      hi = ir ? hi : mr - 1;
+    const uint64_t rest = ~0ull >> dr;
+    const char* K8 = reinterpret_cast<const char*>(sK);
+    int32_t a = 8 * (1 + k), z = a + 8;    // byte offsets of l's and r's keys
+    const int32_t last = 8 * (n + 1);
+#pragma unroll
+    for (int32_t step = 4 * LV_C; step >= 8; step >>= 1) {
+      const int32_t na = max(a - step, 0), nz = min(z + step, last);
+      const uint64_t xa = *reinterpret_cast<const uint64_t*>(K8 + na) ^ key;
+      const uint64_t xz = *reinterpret_cast<const uint64_t*>(K8 + nz) ^ key;
+      a = xa <= rest ? na : a;
+      z = xz <= rest ? nz : z;
     }
+    l = a / 8 - 1;
+    r = z / 8 - 1;
     ndl = l > 0 ? sD[l - 1] : sdl;
     ndr = sD[r];
     node = ndl < dr && ndr < dr;
@@ -496,19 +301,11 @@ __global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ 
   __syncthreads();
   Box6 A{}, B{};
   const int32_t rounds = qmax;
-  for (int32_t q = 0; q <= rounds; ++q) {
-    const float2(*u)[3] = U[q & 1];
-    const int32_t w = 1 << q;
-    if (qa == q) A = box_or(lds_box(u, l), lds_box(u, k - w + 1));
-    if (qb == q) B = box_or(lds_box(u, k + 1), lds_box(u, r - w + 1));
-    if (q < rounds) {
-      if (have) {
-        if (k + w < n) run = box_or(run, lds_box(u, k + w));
-        lds_box_put(U[(q & 1) ^ 1], k, run);
-      }
-      __syncthreads();
-    }
-  }
+#define CC_ROUND(Q) \
+  if (rounds >= Q) level_round<Q>(U[Q & 1], U[(Q & 1) ^ 1], have, k, n, l, r, qa, qb, rounds > Q, run, A, B)
+  CC_ROUND(0); CC_ROUND(1); CC_ROUND(2); CC_ROUND(3); CC_ROUND(4);
+  CC_ROUND(5); CC_ROUND(6); CC_ROUND(7); CC_ROUND(8); CC_ROUND(9);
+#undef CC_ROUND
   // the node's links and boxes
   auto pend_put = [&](int32_t pl, int32_t pr, int32_t idx, int32_t pdl, int32_t pdr, uint64_t pkey, const float* bx) {
     BItem& o = pend[min(atomicAdd(&npend, 1u), (uint32_t)LV_CAP - 1)];
@@ -535,12 +332,13 @@ __global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ 
     // is not its index
     reinterpret_cast<int4*>(o)[3] = make_int4(first < s ? s : ~s, s + 1 < last ? s + 1 : ~(s + 1), -1,
                                               root || !left ? last : first);
-    const Box6 box = box_node(box_or(A, B));
-    if (root) {
-      put6(R, box.v, box.v + 3);
-    } else {
-      const int32_t p = left ? r : l - 1;    // the parent's split
-      if (p < 0 || p >= n - 1 || !built[p]) pend_put(first, last, me, ndl, ndr, sK[l], box.v);
+    const int32_t p = left ? r : l - 1;    // the parent's split
+    if (root || p < 0 || p >= n - 1 || !built[p]) {
+      const Box6 box = box_node(box_or(A, B));
+      if (root)
+        put6(R, box.v, box.v + 3);
+      else
+        pend_put(first, last, me, ndl, ndr, sK[1 + l], box.v);
     }
   }
   // the item itself, when its parent is not built here
@@ -566,7 +364,8 @@ __global__ __launch_bounds__(LV_C) void k_bb_level(const BodyDesc* __restrict__ 
 size_t level_chunks0(uint32_t m) { return (m + LV_C - 1) / LV_C; }
 
 std::vector<std::vector<LvBlock>> build_level_tables(const std::vector<BodyDesc>& h,
-                                                     const std::vector<uint32_t>& bodies) {
+                                                     const std::vector<uint32_t>& bodies,
+                                                     const std::function<bool(uint32_t)>& write_leaves) {
   // level 0 over the leaves, level L+1 over LV_G chunks of level L, until a
   // body's level has a single chunk; slot bases are per level, in list order
   std::vector<std::vector<LvBlock>> out;
@@ -586,6 +385,9 @@ std::vector<std::vector<LvBlock>> build_level_tables(const std::vector<BodyDesc>
         e.in_base = prev_base[j];
         e.out_base = base;
         e.n_in = L == 0 ? h[j].m : prev_n[j];
+        e.t0 = h[j].t0;
+        e.n0 = h[j].n0;
+        e.write_leaves = write_leaves(j) ? 1 : 0;
         t.push_back(e);
       }
       base += chunks[j];
@@ -601,11 +403,12 @@ std::vector<std::vector<LvBlock>> build_level_tables(const std::vector<BodyDesc>
   return out;
 }
 
-void launch_build_levels(const BodyDesc* desc, const LvBlock* const* level, const uint32_t* n_level,
+void launch_build_levels(const LvBlock* const* level, const uint32_t* n_level,
                          const LvFrame* frames, int nframes, hipStream_t s) {
   CC_REQUIRE(nframes >= 1 && nframes <= MAX_FRAMES, "level build: frame count");
   PF<const uint64_t> keys{};
   PF<const float> boxes{};
+  PF<uint4> leaf{};
   PF<BItem> items[2] = {};
   PF<const BItem> items_c[2] = {};
   PF<uint32_t> nitems[2] = {};
@@ -616,6 +419,7 @@ void launch_build_levels(const BodyDesc* desc, const LvBlock* const* level, cons
     const LvFrame& F = frames[f];
     keys.p[f] = F.keys;
     boxes.p[f] = F.boxes;
+    leaf.p[f] = F.leaf_tri;
     for (int q = 0; q < 2; ++q) {
       items[q].p[f] = F.items[q];
       items_c[q].p[f] = F.items[q];
@@ -631,10 +435,10 @@ void launch_build_levels(const BodyDesc* desc, const LvBlock* const* level, cons
     const int in = (L + 1) & 1, out = L == 0 ? 0 : (L & 1);
     const dim3 grid(n_level[L], (unsigned)nframes);
     if (L == 0)
-      k_bb_level<true><<<grid, LV_C, 0, s>>>(desc, level[L], keys, boxes, items_c[in], nitems_c[in],
+      k_bb_level<true><<<grid, LV_C, 0, s>>>(level[L], keys, frames[0].tris, boxes, leaf, items_c[in], nitems_c[in],
                                               items[out], nitems[out], nodes, root, leaf0);
     else
-      k_bb_level<false><<<grid, LV_C, 0, s>>>(desc, level[L], keys, boxes, items_c[in], nitems_c[in],
+      k_bb_level<false><<<grid, LV_C, 0, s>>>(level[L], keys, frames[0].tris, boxes, leaf, items_c[in], nitems_c[in],
                                                items[out], nitems[out], nodes, root, leaf0);
     CC_LAUNCHED();
   }
@@ -663,15 +467,38 @@ void upload_list(DBuf<uint4>& d, uint32_t& n, const std::vector<uint4>& h, hipSt
   if (h.empty()) d.zero(s);
 }
 
-void upload_list(DBuf<uint32_t>& d, uint32_t& n, const std::vector<uint32_t>& h, hipStream_t s) {
-  n = (uint32_t)h.size();
-  d.upload(h.data(), std::max<size_t>(h.size(), 1), s);
-  if (h.empty()) d.zero(s);
-}
-
 }  // namespace
 
-void BatchBodies::init(const cc_body_desc* bodies, const cc_params* params, uint32_t count, hipStream_t s) {
+void XcdMap::init(const std::vector<double>& a, const std::vector<double>& b) {
+  double sa = 0.0, sb = 0.0;
+  for (double v : a) sa += v;
+  for (double v : b) sb += v;
+  auto part = [&](size_t k) { return (sa > 0 ? a[k] / sa : 0.0) + (sb > 0 ? b[k] / sb : 0.0); };
+  std::vector<uint32_t> order(a.size());
+  std::iota(order.begin(), order.end(), 0u);
+  std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return part(x) > part(y); });
+  double la[XCDS] = {}, lb[XCDS] = {};
+  of.assign(a.size(), 0);
+  for (uint32_t k : order) {
+    size_t best = 0;
+    double least = 1e300;
+    for (size_t x = 0; x < XCDS; ++x) {
+      const double w = std::max(sa > 0 ? (la[x] + a[k]) / sa : 0.0, sb > 0 ? (lb[x] + b[k]) / sb : 0.0);
+      if (w < least) {
+        least = w;
+        best = x;
+      }
+    }
+    la[best] += a[k];
+    lb[best] += b[k];
+    of[k] = (uint8_t)best;
+  }
+  const double ma = *std::max_element(la, la + XCDS), mb = *std::max_element(lb, lb + XCDS);
+  if (ma * XCDS > 1.1 * sa || mb * XCDS > 1.1 * sb) of.clear();
+}
+
+void BatchBodies::init(const cc_body_desc* bodies, const cc_params* params, const std::vector<uint32_t>& cloth_n,
+                       uint32_t count, hipStream_t s) {
   std::vector<float> h_rest, h_p0, h_p1;
   std::vector<uint32_t> h_tris, h_capv;
   uint32_t nv_sum = 0, m_sum = 0, n_sum = 0, c_sum = 0, cv_sum = 0, p_sum = 0;
@@ -748,6 +575,11 @@ void BatchBodies::init(const cc_body_desc* bodies, const cc_params* params, uint
     phase.push_back(ph);
   }
   nb = (uint32_t)h.size();
+  {
+    std::vector<double> tri(count, 0.0), vert(cloth_n.begin(), cloth_n.end());
+    for (uint32_t j = 0; j < nb; ++j) tri[inst[j]] = h[j].m;
+    xcd.init(tri, vert);
+  }
   if (nb == 0) return;
   desc.upload(h.data(), nb, s);
   rest.upload(h_rest.data(), h_rest.size(), s);
@@ -801,15 +633,19 @@ void BatchBodies::init(const cc_body_desc* bodies, const cc_params* params, uint
       if (which == 0 || d.mode == CC_BODY_REBUILD) lsort.push_back(j);
       lbuild.push_back(j);
     }
-    upload_list(P.deform, P.n_deform, tdef, s);
-    upload_list(P.boxes, P.n_boxes, tbox, s);
-    upload_list(P.sort, P.n_sort, lsort, s);
-    const std::vector<std::vector<LvBlock>> t = build_level_tables(h, lbuild);
+    auto of_body = [&](const uint4& e) { return inst[e.x]; };
+    upload_list(P.deform, P.n_deform, xcd.arrange(tdef, of_body), s);
+    upload_list(P.boxes, P.n_boxes, xcd.arrange(tbox, of_body), s);
+    P.sort.init(h, lsort, s, [&](std::vector<uint4>& tl) { tl = xcd.arrange(tl, of_body); });
+    std::vector<std::vector<LvBlock>> t = build_level_tables(
+        h, lbuild, [&](uint32_t j) { return which == 0 || h[j].mode == CC_BODY_REBUILD; });
+    for (auto& lv : t) lv = xcd.arrange(lv, [&](const LvBlock& e) { return inst[e.body]; });
     for (int L = 0; L < BB_MAX_LEVELS; ++L) {
       P.n_level[L] = L < (int)t.size() ? (uint32_t)t[L].size() : 0u;
       if (P.n_level[L]) P.level[L].upload(t[L].data(), t[L].size(), s);
     }
   }
+  scratch.alloc(all.sort.ntiles, all.sort.nbig);
   // frame 0 for every body, in both slots
   upload_motion(0, 1, s);
   launch(all, 0, 0, s);
@@ -854,42 +690,18 @@ void BatchBodies::pre(const BodyPass& P, int k, int slot, hipStream_t s) {
 }
 
 void BatchBodies::sort(const BodyPass& P, int slot, hipStream_t s) {
-  if (nb == 0 || !P.n_sort) return;
-  k_bb_sort<<<P.n_sort, SB_THREADS, 0, s>>>(desc.p, P.sort.p, boxes.p, partial.p, kv[0].p, kv[1].p, keys.p,
-                                             leaf_tri[slot].p, tris.p, root[slot].p);
-  CC_LAUNCHED();
-}
-
-template <int EW, int TILE>
-static void launch_sort_step(BatchBodies& B, const BodyPass& P, int slot, const StepLaunch& st, hipStream_t s) {
-  const uint32_t per = SB_THREADS / TILE;
-  const uint32_t nstep = (st.nblocks + per - 1) / per;
-  k_bb_sort_step<EW, TILE><<<P.n_sort + nstep, SB_THREADS, 0, s>>>(
-      B.desc.p, P.sort.p, P.n_sort, B.boxes.p, B.partial.p, B.kv[0].p, B.kv[1].p, B.keys.p, B.leaf_tri[slot].p,
-      B.tris.p, B.root[slot].p, st);
-}
-
-void BatchBodies::sort_with_step(const BodyPass& P, int slot, const StepLaunch& st, hipStream_t s) {
-  CC_REQUIRE(st.tile == 64 || st.tile == 128 || st.tile == 256, "batch: step tile must be 64, 128 or 256");
-  if (st.ew == ELL_W) {
-    if (st.tile == 64) launch_sort_step<ELL_W, 64>(*this, P, slot, st, s);
-    else if (st.tile == 128) launch_sort_step<ELL_W, 128>(*this, P, slot, st, s);
-    else launch_sort_step<ELL_W, 256>(*this, P, slot, st, s);
-  } else {
-    if (st.tile == 64) launch_sort_step<0, 64>(*this, P, slot, st, s);
-    else if (st.tile == 128) launch_sort_step<0, 128>(*this, P, slot, st, s);
-    else launch_sort_step<0, 256>(*this, P, slot, st, s);
-  }
-  CC_LAUNCHED();
+  if (nb == 0) return;
+  const SortFrame f{boxes.p, partial.p, {kv[0].p, kv[1].p}, &scratch, keys.p, nullptr, root[slot].p};
+  launch_sort(desc.p, P.sort, tris.p, &f, 1, s);
 }
 
 void BatchBodies::post(const BodyPass& P, int slot, hipStream_t s) {
   if (nb == 0) return;
   const LvBlock* tabs[BB_MAX_LEVELS];
   for (int L = 0; L < BB_MAX_LEVELS; ++L) tabs[L] = P.level[L].p;
-  const LvFrame f{keys.p, boxes.p, {items[0].p, items[1].p}, {nitems[0].p, nitems[1].p},
+  const LvFrame f{keys.p, tris.p, boxes.p, leaf_tri[slot].p, {items[0].p, items[1].p}, {nitems[0].p, nitems[1].p},
                   nodes[slot].p, root[slot].p, leaf0[slot].p};
-  launch_build_levels(desc.p, tabs, P.n_level, &f, 1, s);
+  launch_build_levels(tabs, P.n_level, &f, 1, s);
 }
 
 void BatchBodies::export_tree(uint32_t j, int slot, float* verts3, uint64_t* okeys, uint32_t* order,

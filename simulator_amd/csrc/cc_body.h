@@ -8,6 +8,7 @@
 // own build scratch, so several frames can be updated at the same time.
 #pragma once
 
+#include <functional>
 #include <vector>
 
 #include "cc_internal.h"
@@ -67,6 +68,42 @@ struct BodyDesc {
   uint32_t pad;
 };
 
+// ---- Morton codes and their sort (sort.hip), of one body or of a batch's
+constexpr uint32_t BOX_BLOCK = 256;        // triangles per partial root box
+constexpr uint32_t SORT_TILE = 1024;       // keys per sort workgroup
+constexpr uint32_t SORT_SUM_TILES = 64;    // see sort.hip
+constexpr uint32_t SORT_SUM_MAX = SORT_SUM_TILES * SORT_TILE;
+inline uint32_t sort_tiles(uint32_t m) { return (m + SORT_TILE - 1) / SORT_TILE; }
+// Work table of a set of bodies: their tiles, and the bodies of more than
+// SORT_SUM_TILES tiles.
+struct SortTable {
+  DBuf<uint4> tiles, big;
+  uint32_t ntiles = 0, nbig = 0;
+  // arrange (optional): an order of the tiles
+  void init(const std::vector<BodyDesc>& h, const std::vector<uint32_t>& bodies, hipStream_t s,
+            const std::function<void(std::vector<uint4>&)>& arrange = {});
+};
+// Scratch of one sort in flight.
+struct SortScratch {
+  DBuf<uint32_t> counts;   // [tiles * 512] digit counts of each tile, 16-bit pairs
+  DBuf<uint32_t> first;    // [tiles * 1024] of big bodies: places of each tile's digits
+  DBuf<uint32_t> total;    // [big bodies * 1024] their keys per digit
+  void alloc(size_t tiles, size_t nbig);
+};
+struct SortFrame {
+  const float* boxes;      // [6 m] expanded boxes
+  const float* partial;    // root box of each BOX_BLOCK triangles
+  uint2* kv[2];            // [m] (code, primitive) ping-pong
+  SortScratch* sort;
+  uint64_t* keys;          // [m] out: sorted code << 32 | primitive
+  uint4* leaf_tri;         // [m] out: sorted leaves (null: the level build writes them)
+  float* root;             // [6 * bodies] out: root boxes
+};
+// Codes, sort, keys and leaves of the table's bodies; nframes frames in each
+// launch (grid.y).
+void launch_sort(const BodyDesc* desc, const SortTable& t, const uint32_t* tris, const SortFrame* frames, int nframes,
+                 hipStream_t s);
+
 // A node finished by one level of the bottom-up build and handed to the
 // next: its sorted-leaf range, Karras index, box, the key of its first leaf
 // and the deltas of the key pairs at its two boundaries (-1 at the ends of
@@ -82,7 +119,9 @@ static_assert(sizeof(BItem) == 64, "BItem must be 64 bytes");
 // One workgroup of a build level: chunk q of the body's level, input slots
 // from in_base (n_in of them; leaves at level 0), output slots at out_base.
 struct LvBlock {
-  uint32_t body, q, in_base, out_base, n_in, pad[3];
+  uint32_t body, q, in_base, out_base, n_in;
+  uint32_t t0, n0;          // as in the body's BodyDesc
+  uint32_t write_leaves;
 };
 
 constexpr int BB_MAX_LEVELS = 8;       // 2^30 leaves: 2^20 -> 2^17 -> ... -> 4 -> 1 chunks
@@ -93,13 +132,18 @@ constexpr uint32_t LV_MAX_LEAVES = 1u << 21;   // leaf indices of the bottom-up 
 // the number of level-0 chunks of m leaves, and the launches of all levels.
 // keys / boxes / nodes are indexed through each
 // body's t0 / n0; root and leaf0 hold 6 floats per body.
+// Level 0 also writes the sorted leaves of the bodies that are sorted anew
+// (write_leaves(body); their keys alone come out of the sort).
 std::vector<std::vector<LvBlock>> build_level_tables(const std::vector<BodyDesc>& h,
-                                                     const std::vector<uint32_t>& bodies);
+                                                     const std::vector<uint32_t>& bodies,
+                                                     const std::function<bool(uint32_t)>& write_leaves);
 size_t level_chunks0(uint32_t m);
 // The buffers of one frame of a level build.
 struct LvFrame {
   const uint64_t* keys;
+  const uint32_t* tris;
   const float* boxes;
+  uint4* leaf_tri;
   BItem* items[2];
   uint32_t* nitems[2];
   Node* nodes;
@@ -107,7 +151,7 @@ struct LvFrame {
   float* leaf0;
 };
 // nframes (1..MAX_FRAMES) frames of the same tables in each launch (grid.y)
-void launch_build_levels(const BodyDesc* desc, const LvBlock* const* level, const uint32_t* n_level,
+void launch_build_levels(const LvBlock* const* level, const uint32_t* n_level,
                          const LvFrame* frames, int nframes, hipStream_t s);
 
 // One frame of the body as the collision query reads it.
@@ -129,9 +173,8 @@ struct Lane {
   uint32_t nblk_box = 0;
   DBuf<float> boxes;                // [6*m] unsorted expanded boxes
   DBuf<float> partial;              // [6*nblk_box] per-block root boxes
-  DBuf<uint32_t> code[2], idx[2];   // radix sort ping-pong
-  DBuf<uint32_t> hist;              // [256 * sort blocks]
-  DBuf<uint32_t> digit_total;       // [1024] keys per digit of the current pass
+  DBuf<uint2> kv[2];                // radix sort ping-pong
+  SortScratch sort;
   DBuf<uint64_t> keys;              // [m] sorted morton << 32 | primitive
   DBuf<int32_t> leaf_parent;        // [m]
   // refit description: internal nodes whose leaf range crosses a chunk
@@ -178,8 +221,9 @@ struct Body {
   // A rebuilt body of 2..2^21 triangles builds its tree and boxes bottom-up
   // (the batched build's level kernels) instead of the Karras searches, the
   // refit description and the refit.
+  DBuf<BodyDesc> desc;              // [1] offsets 0
+  SortTable sort_table;
   bool bottom_up = false;
-  DBuf<BodyDesc> bu_desc;           // [1] offsets 0
   DBuf<LvBlock> bu_level[BB_MAX_LEVELS];
   uint32_t bu_n[BB_MAX_LEVELS] = {};
 

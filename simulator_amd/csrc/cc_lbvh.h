@@ -27,6 +27,23 @@ __device__ inline void unite(float* mn, float* mx, const float* b6) {
   }
 }
 
+// Component threadIdx.x (0..5) of the block's box, in its first six threads:
+// lanes reduce by shuffles, waves through red.
+template <int WAVES>
+__device__ inline float block_box(float* mn, float* mx, float (&red)[WAVES][6]) {
+  for (int off = 32; off > 0; off >>= 1)
+    for (int c = 0; c < 3; ++c) {
+      mn[c] = fminf(mn[c], __shfl_xor(mn[c], off, 64));
+      mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], off, 64));
+    }
+  if ((threadIdx.x & 63u) == 0) put6(red[threadIdx.x >> 6], mn, mx);
+  __syncthreads();
+  const uint32_t c = threadIdx.x < 6 ? threadIdx.x : 0;
+  float v = red[0][c];
+  for (int w = 1; w < WAVES; ++w) v = c < 3 ? fminf(v, red[w][c]) : fmaxf(v, red[w][c]);
+  return v;
+}
+
 // A box of the four-wide form: entry d = {record * 4 + entry, link}, ~0 for
 // none.  An entry is one 32-byte sector {min xyz, max x | max yz, link, 0}
 // written whole by one thread (two 16-byte stores).

@@ -1,7 +1,6 @@
 // lbvh.hip -- body deformation and the Karras LBVH on gfx950: expanded
-// triangle boxes, 30-bit Morton codes, LSD radix sort (LDS histogram +
-// wavefront-ballot ranking) and the clz64 radix-tree build; the box refit
-// lives in refit.hip.
+// triangle boxes and the clz64 radix-tree build; the codes and their sort
+// live in sort.hip, the box refit in refit.hip.
 //
 // Reference path: BVHAccel (bvh.cu:154-297) computes boxes and codes on the
 // GPU, sorts on the host (Utilities.h:22-67) and builds the tree with
@@ -67,23 +66,7 @@ __global__ __launch_bounds__(256) void k_deform(const float* __restrict__ rest, 
 
 // ------------------------------------------------------------ boxes + codes
 constexpr int BOX_THREADS = 256;
-
-// Component threadIdx.x (0..5) of the block's box, in its first six threads:
-// lanes reduce by shuffles, waves through red.
-template <int WAVES>
-__device__ inline float block_box(float* mn, float* mx, float (&red)[WAVES][6]) {
-  for (int off = 32; off > 0; off >>= 1)
-    for (int c = 0; c < 3; ++c) {
-      mn[c] = fminf(mn[c], __shfl_xor(mn[c], off, 64));
-      mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], off, 64));
-    }
-  if ((threadIdx.x & 63u) == 0) put6(red[threadIdx.x >> 6], mn, mx);
-  __syncthreads();
-  const uint32_t c = threadIdx.x < 6 ? threadIdx.x : 0;
-  float v = red[0][c];
-  for (int w = 1; w < WAVES; ++w) v = c < 3 ? fminf(v, red[w][c]) : fmaxf(v, red[w][c]);
-  return v;
-}
+static_assert(BOX_THREADS == BOX_BLOCK, "one partial root box per BOX_BLOCK triangles");
 
 // expanded box per triangle + one partial root box per block
 __global__ __launch_bounds__(BOX_THREADS) void k_prim_boxes(PF<const float> verts_f,
@@ -104,261 +87,6 @@ __global__ __launch_bounds__(BOX_THREADS) void k_prim_boxes(PF<const float> vert
   }
   const float v = block_box<BOX_THREADS / 64>(mn, mx, red);
   if (threadIdx.x < 6) partial[6 * (size_t)blockIdx.x + threadIdx.x] = v;
-}
-
-// ------------------------------------------------------------ radix sort
-// Stable LSD sort of (code, index) pairs by code, three passes of 10-bit
-// digits (the Morton codes have 30 bits).  Because the indices enter in
-// ascending order and every pass is stable, the result is ordered by the
-// full 64-bit key (code << 32 | index).
-//
-// A pass cuts the keys into tiles of SORT_TILE, one workgroup each: the tile's
-// digit counts (by k_morton for the first pass, k_radix_hist for the others),
-// then k_radix_scatter.  A body of up to SORT_SCAN_BLOCKS tiles has no scan
-// launch between the two: the counts lie tile after tile and every scatter
-// workgroup sums the ones before it and all of them itself (at most 64 x 4
-// KB, coalesced); a larger body's counts lie digit after digit and are
-// scanned by k_radix_rowscan first, because the tiles' own sums grow with
-// the square of their number.  The chain of small launches is what a rebuild
-// of a garment-sized body costs (its lanes run beside the step, and other
-// simulators' work queues behind them).  50,688 triangles, three frames in a
-// chain: 37 us from codes to sorted leaves in six launches, against 68 us in
-// eleven (separate counts of the first pass, scans and key / leaf writing;
-// one row of 256 keys at a time between barriers).  Four rows per wave
-// instead of two: 33 us of scatters against 27.
-constexpr int SORT_THREADS = 512;
-constexpr int SORT_WAVES = SORT_THREADS / 64;
-constexpr int SORT_ROWS = 2;              // rows of 64 consecutive keys per wave
-constexpr int SORT_TILE = SORT_THREADS * SORT_ROWS;
-constexpr int RADIX_BITS = 10;
-constexpr int RADIX_DIGITS = 1 << RADIX_BITS;
-constexpr int RADIX_PASSES = 3;
-constexpr uint32_t SORT_SCAN_BLOCKS = 64;
-// counts tile after tile are 16-bit pairs; a workgroup reads them in
-// SORT_GROUPS groups of lanes, each summing every SORT_GROUPS-th tile
-constexpr int SORT_WORDS = RADIX_DIGITS / 2;
-constexpr int SORT_GROUPS = SORT_THREADS * 4 / SORT_WORDS;
-constexpr int SORT_LOADS = SORT_SCAN_BLOCKS / SORT_GROUPS;
-static_assert(SORT_THREADS * 2 == RADIX_DIGITS, "two digits per thread");
-static_assert(SORT_LOADS * SORT_TILE < 65536, "a group's sums fit 16 bits");
-
-// The workgroup's counts h to its tile's place: tile after tile (by_tile) or
-// digit after digit.
-__device__ inline void put_counts(const uint32_t* h, uint32_t* __restrict__ hist, uint32_t nblk, bool by_tile) {
-  const uint32_t t = threadIdx.x;
-  if (by_tile) {
-    hist[(size_t)blockIdx.x * SORT_WORDS + t] = h[2 * t] | (h[2 * t + 1] << 16);
-  } else {
-    hist[(size_t)(2 * t) * nblk + blockIdx.x] = h[2 * t];
-    hist[(size_t)(2 * t + 1) * nblk + blockIdx.x] = h[2 * t + 1];
-  }
-}
-
-// root box (sentinel U all partials, recomputed per block), then the code of
-// each box centroid (compute_morton_bbox, bvh.cu:71-79) of a sort tile and
-// the first pass's digit counts
-__global__ __launch_bounds__(SORT_THREADS) void k_morton(PF<const float> boxes_f, uint32_t m,
-                                                         PF<const float> partial_f, uint32_t npart,
-                                                         PF<uint32_t> codes_f, PF<uint32_t> hist_f, uint32_t nblk,
-                                                         bool by_tile, PF<float> root_f) {
-  __shared__ float red[SORT_WAVES][6], sroot[6];
-  __shared__ uint32_t h[RADIX_DIGITS];
-  const float* __restrict__ boxes = pick(boxes_f);
-  const float* __restrict__ partial = pick(partial_f);
-  uint32_t* __restrict__ codes = pick(codes_f);
-  float* __restrict__ root_out = pick(root_f);
-  const uint32_t tid = threadIdx.x, base = blockIdx.x * SORT_TILE;
-  float bx[SORT_ROWS][6];
-#pragma unroll
-  for (int r = 0; r < SORT_ROWS; ++r) {
-    const float* b = boxes + 6 * (size_t)min(base + r * SORT_THREADS + tid, m - 1);
-#pragma unroll
-    for (int c = 0; c < 6; ++c) bx[r][c] = b[c];
-  }
-  float mn[3], mx[3];
-  box_sentinel(mn, mx);
-  for (uint32_t q = tid; q < npart; q += SORT_THREADS) unite(mn, mx, partial + 6 * (size_t)q);
-  h[tid] = h[tid + SORT_THREADS] = 0;
-  const float v = block_box<SORT_WAVES>(mn, mx, red);
-  if (tid < 6) {
-    sroot[tid] = v;
-    if (blockIdx.x == 0) root_out[tid] = v;
-  }
-  __syncthreads();
-  const float rmin[3] = {sroot[0], sroot[1], sroot[2]};
-  const float rext[3] = {sroot[3] - sroot[0], sroot[4] - sroot[1], sroot[5] - sroot[2]};
-#pragma unroll
-  for (int r = 0; r < SORT_ROWS; ++r) {
-    const uint32_t i = base + r * SORT_THREADS + tid;
-    if (i >= m) continue;
-    const uint32_t c = box_morton(bx[r], bx[r] + 3, rmin, rext);
-    codes[i] = c;
-    atomicAdd(&h[c & (RADIX_DIGITS - 1)], 1u);
-  }
-  __syncthreads();
-  put_counts(h, pick(hist_f), nblk, by_tile);
-}
-
-__global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(PF<const uint32_t> keys_f, uint32_t n, int shift,
-                                                             PF<uint32_t> hist_f, uint32_t nblk, bool by_tile) {
-  __shared__ uint32_t h[RADIX_DIGITS];
-  const uint32_t* __restrict__ keys = pick(keys_f);
-  const uint32_t base = blockIdx.x * SORT_TILE;
-  uint32_t k[SORT_ROWS];
-#pragma unroll
-  for (int r = 0; r < SORT_ROWS; ++r) k[r] = keys[min(base + r * SORT_THREADS + threadIdx.x, n - 1)];
-  h[threadIdx.x] = h[threadIdx.x + SORT_THREADS] = 0;
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < SORT_ROWS; ++r)
-    if (base + r * SORT_THREADS + threadIdx.x < n) atomicAdd(&h[(k[r] >> shift) & (RADIX_DIGITS - 1)], 1u);
-  __syncthreads();
-  put_counts(h, pick(hist_f), nblk, by_tile);
-}
-
-// Counts digit after digit: per digit, the exclusive prefix over tiles (in
-// place) and the digit's total: one wave per digit, 64 tiles per round.
-__global__ __launch_bounds__(256) void k_radix_rowscan(PF<uint32_t> hist_f, uint32_t nblk, PF<uint32_t> total_f) {
-  uint32_t* __restrict__ hist = pick(hist_f);
-  uint32_t* __restrict__ total = pick(total_f);
-  const uint32_t lane = threadIdx.x & 63u, d = blockIdx.x * 4 + (threadIdx.x >> 6);
-  uint32_t* row = hist + (size_t)d * nblk;
-  uint32_t carry = 0;
-  for (uint32_t b0 = 0; b0 < nblk; b0 += 64) {
-    const uint32_t b = b0 + lane;
-    const uint32_t v = b < nblk ? row[b] : 0u;
-    uint32_t incl = v;
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t u = __shfl_up(incl, off, 64);
-      if (lane >= (uint32_t)off) incl += u;
-    }
-    if (b < nblk) row[b] = carry + incl - v;
-    carry += __shfl(incl, 63, 64);
-  }
-  if (lane == 0) total[d] = carry;
-}
-
-// Scatter with stable ranks.  Wave w owns SORT_ROWS rows of 64 consecutive
-// keys; within a row the lanes of a digit are matched with RADIX_BITS
-// ballots, and a running per-digit count of the wave's rows is kept in LDS,
-// so a tile takes three barriers.  Element order = (wave, row, lane) order.
-// FIRST: the values are the indices themselves.  LAST: the sorted keys and
-// leaf triangles are written instead of the pairs.
-template <bool FIRST, bool LAST>
-__global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(PF<const uint32_t> kin_f, PF<const uint32_t> vin_f,
-                                                                uint32_t n, int shift, PF<const uint32_t> hist_f,
-                                                                PF<const uint32_t> total_f, uint32_t nblk,
-                                                                bool by_tile, PF<uint32_t> kout_f,
-                                                                PF<uint32_t> vout_f, const uint32_t* __restrict__ tris,
-                                                                PF<uint64_t> keys_f, PF<uint4> leaf_tri_f) {
-  __shared__ __align__(16) uint32_t wcnt[SORT_WAVES][RADIX_DIGITS];
-  __shared__ uint32_t wsum[SORT_WAVES];
-  const uint32_t* __restrict__ kin = pick(kin_f);
-  const uint32_t* __restrict__ hist = pick(hist_f);
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-  const uint32_t base = blockIdx.x * SORT_TILE;
-  uint32_t key[SORT_ROWS], val[SORT_ROWS], loc[SORT_ROWS];
-  bool ok[SORT_ROWS];
-#pragma unroll
-  for (int r = 0; r < SORT_ROWS; ++r) {
-    const uint32_t e = base + (w * SORT_ROWS + r) * 64 + lane;
-    ok[r] = e < n;
-    key[r] = kin[min(e, n - 1)];
-    val[r] = FIRST ? e : pick(vin_f)[min(e, n - 1)];
-  }
-
-  // the tile's first place of each of the thread's digits 2 tid, 2 tid + 1
-  uint32_t tot[2], first[2];
-  if (by_tile) {
-    // all loads of a lane in flight at once; sums of 16-bit pairs
-    uint4* part = reinterpret_cast<uint4*>(&wcnt[0][0]);      // [2][SORT_GROUPS][SORT_WORDS] words
-    const uint32_t g = tid / (SORT_WORDS / 4), q = tid % (SORT_WORDS / 4);
-    const uint4* h4 = reinterpret_cast<const uint4*>(hist) + q;
-    uint4 c[SORT_LOADS];
-#pragma unroll
-    for (int j = 0; j < SORT_LOADS; ++j)
-      c[j] = h4[(size_t)min(g + (uint32_t)(j * SORT_GROUPS), nblk - 1) * (SORT_WORDS / 4)];
-    uint4 all = make_uint4(0, 0, 0, 0), pre = make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < SORT_LOADS; ++j) {
-      const uint32_t b = g + (uint32_t)(j * SORT_GROUPS);
-      const uint32_t in = b < nblk ? ~0u : 0u, be = b < blockIdx.x ? ~0u : 0u;
-      all.x += c[j].x & in; all.y += c[j].y & in; all.z += c[j].z & in; all.w += c[j].w & in;
-      pre.x += c[j].x & be; pre.y += c[j].y & be; pre.z += c[j].z & be; pre.w += c[j].w & be;
-    }
-    part[g * (SORT_WORDS / 4) + q] = all;
-    part[(SORT_GROUPS + g) * (SORT_WORDS / 4) + q] = pre;
-    __syncthreads();
-    const uint32_t* pw = &wcnt[0][0] + tid;
-    tot[0] = tot[1] = first[0] = first[1] = 0;
-#pragma unroll
-    for (int k = 0; k < SORT_GROUPS; ++k) {
-      const uint32_t a = pw[k * SORT_WORDS], p = pw[(SORT_GROUPS + k) * SORT_WORDS];
-      tot[0] += a & 0xffffu; tot[1] += a >> 16;
-      first[0] += p & 0xffffu; first[1] += p >> 16;
-    }
-  } else {
-    const uint2 t2 = reinterpret_cast<const uint2*>(pick(total_f))[tid];
-    tot[0] = t2.x; tot[1] = t2.y;
-    for (int q = 0; q < 2; ++q) first[q] = hist[(size_t)(2 * tid + q) * nblk + blockIdx.x];
-  }
-  {
-    const uint32_t v = tot[0] + tot[1];
-    uint32_t incl = v;
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t u = __shfl_up(incl, off, 64);
-      if (lane >= (uint32_t)off) incl += u;
-    }
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();                       // also: the parts have been read
-    uint32_t s = incl - v;
-    for (uint32_t q = 0; q < w; ++q) s += wsum[q];
-    first[0] += s;
-    first[1] += s + tot[0];
-  }
-  for (uint32_t d = lane; d < (uint32_t)RADIX_DIGITS / 4; d += 64)
-    reinterpret_cast<uint4*>(wcnt[w])[d] = make_uint4(0, 0, 0, 0);
-
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-#pragma unroll
-  for (int r = 0; r < SORT_ROWS; ++r) {
-    const uint32_t d = (key[r] >> shift) & (RADIX_DIGITS - 1);
-    uint64_t msk = __ballot(ok[r]);
-#pragma unroll
-    for (int b = 0; b < RADIX_BITS; ++b) {
-      const bool on = (d >> b) & 1u;
-      const uint64_t bb = __ballot(on);
-      msk &= on ? bb : ~bb;
-    }
-    // the wave's count of this digit in its earlier rows, then this row's
-    // lanes of the digit; the lowest such lane adds the row's count
-    const uint32_t prior = wcnt[w][d], rank = __popcll(msk & lt);
-    loc[r] = prior + rank;
-    if (ok[r] && rank == 0) wcnt[w][d] = prior + (uint32_t)__popcll(msk);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int v = 0; v < SORT_WAVES; ++v) {   // per digit: offsets of the waves' runs
-    uint2& p = reinterpret_cast<uint2*>(wcnt[v])[tid];
-    const uint2 c = p;
-    p = make_uint2(first[0], first[1]);
-    first[0] += c.x;
-    first[1] += c.y;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < SORT_ROWS; ++r) {
-    if (!ok[r]) continue;
-    const uint32_t pos = wcnt[w][(key[r] >> shift) & (RADIX_DIGITS - 1)] + loc[r];
-    if constexpr (LAST) {
-      pick(keys_f)[pos] = ((uint64_t)key[r] << 32) | val[r];
-      const uint32_t* t = tris + 3 * (size_t)val[r];
-      pick(leaf_tri_f)[pos] = make_uint4(t[0], t[1], t[2], val[r]);
-    } else {
-      pick(kout_f)[pos] = key[r];
-      pick(vout_f)[pos] = val[r];
-    }
-  }
 }
 
 // ------------------------------------------------------------ Karras build
@@ -386,10 +114,10 @@ void Body::build_levels(int F, const int* ks, const int* ls, hipStream_t s) {
   for (int f = 0; f < F; ++f) {
     Lane& L = lane[ls[f]];
     Slot& S = slot[ks[f]];
-    fr[f] = LvFrame{L.keys.p, L.boxes.p, {L.items[0].p, L.items[1].p},
+    fr[f] = LvFrame{L.keys.p, tris.p, L.boxes.p, leaf_tri_of(ks[f]), {L.items[0].p, L.items[1].p},
                     {L.nitems[0].p, L.nitems[1].p}, S.nodes.p, S.root.p, S.leaf0_box.p};
   }
-  launch_build_levels(bu_desc.p, tabs, bu_n, fr, F, s);
+  launch_build_levels(tabs, bu_n, fr, F, s);
 }
 
 void Lane::alloc(uint32_t m, bool full_lane, bool bottom_up, hipStream_t s) {
@@ -401,12 +129,8 @@ void Lane::alloc(uint32_t m, bool full_lane, bool bottom_up, hipStream_t s) {
   nblk_box = grid_for(m, BOX_THREADS);
   boxes.alloc(6 * (size_t)m);
   partial.alloc(6 * (size_t)nblk_box);
-  for (int b = 0; b < 2; ++b) {
-    code[b].alloc(m);
-    idx[b].alloc(m);
-  }
-  hist.alloc(RADIX_DIGITS * (size_t)grid_for(m, SORT_TILE));
-  digit_total.alloc(RADIX_DIGITS);
+  for (auto& b : kv) b.alloc(m);
+  sort.alloc(sort_tiles(m), m > SORT_SUM_MAX ? 1 : 0);
   if (bottom_up) {
     const size_t c0 = level_chunks0(m);
     for (int q = 0; q < 2; ++q) {
@@ -486,14 +210,15 @@ void Body::init(const float* v3, uint32_t nv_, const uint32_t* t3, uint32_t nf, 
     S.motion.zero(s);
   }
   bottom_up = mode == CC_BODY_REBUILD && m >= 2 && m <= LV_MAX_LEAVES && allow_bottom_up;
+  BodyDesc d{};
+  d.nv = nv;
+  d.m = m;
+  d.mode = mode;
+  d.depth = depth;
+  desc.upload(&d, 1, s);
+  sort_table.init({d}, {0u}, s);
   if (bottom_up) {
-    BodyDesc d{};
-    d.nv = nv;
-    d.m = m;
-    d.mode = mode;
-    d.depth = depth;
-    bu_desc.upload(&d, 1, s);
-    const std::vector<std::vector<LvBlock>> t = build_level_tables(std::vector<BodyDesc>{d}, {0u});
+    const std::vector<std::vector<LvBlock>> t = build_level_tables({d}, {0u}, [](uint32_t) { return true; });
     for (int q = 0; q < BB_MAX_LEVELS; ++q) {
       bu_n[q] = q < (int)t.size() ? (uint32_t)t[q].size() : 0u;
       if (bu_n[q]) bu_level[q].upload(t[q].data(), t[q].size(), s);
@@ -531,54 +256,23 @@ void Body::deform(int k, uint64_t frame, hipStream_t s) { deform_frames(1, &k, &
 void Body::build_frames(int F, const int* ks, const int* ls, hipStream_t s) {
   if (mode == CC_BODY_NONE || m == 0) return;
   CC_REQUIRE(F >= 1 && F <= MAX_FRAMES && (F == 1 || bottom_up), "body: frames per build chain");
-  PF<const float> verts{}, boxes_c{}, partial_c{};
-  PF<float> boxes{}, partial{}, root{};
-  PF<uint32_t> code[2] = {}, idx[2] = {}, hist{}, total{};
-  PF<const uint32_t> code_c[2] = {}, idx_c[2] = {}, hist_c{}, total_c{};
-  PF<uint64_t> keys{};
-  PF<uint4> leaf{};
+  PF<const float> verts{};
+  PF<float> boxes{}, partial{};
+  SortFrame sf[MAX_FRAMES];
   for (int f = 0; f < F; ++f) {
     Lane& L = lane[ls[f]];
     CC_REQUIRE(L.full, "body: build on a refit-only lane");
     Slot& S = slot[ks[f]];
     verts.p[f] = S.verts.p;
     boxes.p[f] = L.boxes.p;
-    boxes_c.p[f] = L.boxes.p;
     partial.p[f] = L.partial.p;
-    partial_c.p[f] = L.partial.p;
-    root.p[f] = S.root.p;
-    for (int b = 0; b < 2; ++b) {
-      code[b].p[f] = L.code[b].p;
-      code_c[b].p[f] = L.code[b].p;
-      idx[b].p[f] = L.idx[b].p;
-      idx_c[b].p[f] = L.idx[b].p;
-    }
-    hist.p[f] = L.hist.p;
-    hist_c.p[f] = L.hist.p;
-    total.p[f] = L.digit_total.p;
-    total_c.p[f] = L.digit_total.p;
-    keys.p[f] = L.keys.p;
-    leaf.p[f] = leaf_tri_of(ks[f]);
+    sf[f] = SortFrame{L.boxes.p, L.partial.p, {L.kv[0].p, L.kv[1].p}, &L.sort, L.keys.p,
+                      bottom_up ? nullptr : leaf_tri_of(ks[f]), S.root.p};
   }
-  const unsigned nf = (unsigned)F;
   const uint32_t nblk_box = lane[ls[0]].nblk_box;
-  k_prim_boxes<<<dim3(nblk_box, nf), BOX_THREADS, 0, s>>>(verts, tris.p, m, depth, boxes, partial);
+  k_prim_boxes<<<dim3(nblk_box, (unsigned)F), BOX_THREADS, 0, s>>>(verts, tris.p, m, depth, boxes, partial);
   CC_LAUNCHED();
-  const uint32_t nblk = grid_for(m, SORT_TILE);
-  const bool by_tile = nblk <= SORT_SCAN_BLOCKS;
-  const dim3 tiles(nblk, nf);
-  k_morton<<<tiles, SORT_THREADS, 0, s>>>(boxes_c, m, partial_c, nblk_box, code[0], hist, nblk, by_tile, root);
-  CC_LAUNCHED();
-  for (int pass = 0, shift = 0; pass < RADIX_PASSES; ++pass, shift += RADIX_BITS) {
-    const int src = pass & 1, dst = src ^ 1;
-    if (pass) k_radix_hist<<<tiles, SORT_THREADS, 0, s>>>(code_c[src], m, shift, hist, nblk, by_tile);
-    if (!by_tile) k_radix_rowscan<<<dim3(RADIX_DIGITS / 4, nf), 256, 0, s>>>(hist, nblk, total);
-    auto scatter = pass == 0 ? k_radix_scatter<true, false>
-                   : pass + 1 < RADIX_PASSES ? k_radix_scatter<false, false> : k_radix_scatter<false, true>;
-    scatter<<<tiles, SORT_THREADS, 0, s>>>(code_c[src], idx_c[src], m, shift, hist_c, total_c, nblk, by_tile, code[dst],
-                                           idx[dst], tris.p, keys, leaf);
-    CC_LAUNCHED();
-  }
+  launch_sort(desc.p, sort_table, tris.p, sf, F, s);
   if (bottom_up) {                      // tree, parent links and boxes, bottom-up
     build_levels(F, ks, ls, s);
     fold_frames(F, ks, s);
