@@ -199,6 +199,7 @@ struct Lane {
   DBuf<uint32_t> nitems[2];
 
   void alloc(uint32_t m, bool full_lane, bool bottom_up, hipStream_t s);
+  void alloc_levels(uint32_t m, hipStream_t s);
 };
 
 // Host copy of a built tree in the reference encoding (see cc_bvh_export):
@@ -284,6 +285,16 @@ struct Body {
   void init(const float* verts3, uint32_t nv, const uint32_t* tris, uint32_t nf, uint32_t mode, float depth,
             const cc_capsules* caps, const MotionParams& mp, int slots, int lanes, hipStream_t s,
             int chain = 1, bool allow_bottom_up = true);
+
+  // A static body whose vertices its owner replaces: from here on its tree
+  // is built and its wide records are folded on the device, as a rebuilt
+  // body's are (2 <= m <= 2^21; otherwise nothing changes).  The tree is the
+  // same; the host layout of wide_setup (some 2 ms at 50,688 triangles: the
+  // nodes copied to the host, laid out breadth-first and sorted, a dozen
+  // buffers made) pays only for a body that stays, whose walk it makes 3%
+  // shorter.
+  void rebuild_on_device(hipStream_t s);
+  void level_setup(hipStream_t s);    // work tables and scratch of the build by levels, lane 0..
 
   // launches, asynchronous on s
   void deform(int k, uint64_t frame, hipStream_t s);   // rest -> slot k pose of `frame`

@@ -198,6 +198,24 @@ struct Sim {
     CC_HIP(hipStreamSynchronize(stream));
   }
 
+  // A new tree over slot k's vertices, shared with the other slots of a
+  // refitted body.  Captured blocks hold the body's views: they go where one
+  // changed (its four-wide records in another buffer).
+  void rebuild_body(int k) {
+    std::vector<BvhView> before;
+    for (int q = 0; q < body.nslots; ++q) before.push_back(body.view(q));
+    body.rebuild_on_device(stream);
+    body.build(k, 0, stream);
+    body.share_topology(k, stream);
+    for (int q = 0; q < body.nslots; ++q) {
+      const BvhView v = body.view(q);
+      if (v.wide != before[q].wide || v.grouped != before[q].grouped) {
+        drop_graphs();
+        return;
+      }
+    }
+  }
+
   hipGraphExec_t end_capture(int cur0) {
     cur = cur0;
     hipGraph_t graph = nullptr;

@@ -131,14 +131,7 @@ void Lane::alloc(uint32_t m, bool full_lane, bool bottom_up, hipStream_t s) {
   partial.alloc(6 * (size_t)nblk_box);
   for (auto& b : kv) b.alloc(m);
   sort.alloc(sort_tiles(m), m > SORT_SUM_MAX ? 1 : 0);
-  if (bottom_up) {
-    const size_t c0 = level_chunks0(m);
-    for (int q = 0; q < 2; ++q) {
-      items[q].alloc(c0 * 128);
-      nitems[q].alloc(c0);
-      nitems[q].zero(s);
-    }
-  }
+  if (bottom_up) alloc_levels(m, s);
   keys.alloc(m);
   leaf_parent.alloc(m);
   leaf_parent.zero(s);
@@ -160,6 +153,42 @@ void Lane::alloc(uint32_t m, bool full_lane, bool bottom_up, hipStream_t s) {
   lflag.zero(s);
   chunk_h.alloc(grid_for(std::max<uint32_t>(m, 1), REFIT_CHUNK));
   chunk_h.zero(s);
+}
+
+void Lane::alloc_levels(uint32_t m, hipStream_t s) {
+  const size_t c0 = level_chunks0(m);
+  for (int q = 0; q < 2; ++q) {
+    items[q].alloc(c0 * 128);
+    nitems[q].alloc(c0);
+    nitems[q].zero(s);
+  }
+}
+
+void Body::level_setup(hipStream_t s) {
+  BodyDesc d{};
+  d.nv = nv;
+  d.m = m;
+  d.mode = mode;
+  d.depth = depth;
+  const std::vector<std::vector<LvBlock>> t = build_level_tables({d}, {0u}, [](uint32_t) { return true; });
+  for (int q = 0; q < BB_MAX_LEVELS; ++q) {
+    bu_n[q] = q < (int)t.size() ? (uint32_t)t[q].size() : 0u;
+    if (bu_n[q]) bu_level[q].upload(t[q].data(), t[q].size(), s);
+  }
+  CC_HIP(hipStreamSynchronize(s));   // the tables' host copies end here
+}
+
+void Body::rebuild_on_device(hipStream_t s) {
+  if (mode != CC_BODY_STATIC || bottom_up || m < 2 || m > LV_MAX_LEAVES) return;
+  lane[0].alloc_levels(m, s);
+  level_setup(s);
+  slot[0].wide.alloc(8 * (size_t)(m - 1));
+  w_src.release();
+  w_link.release();
+  w_dst.release();
+  nwide = m - 1;
+  wide_stack = STACK_LIMIT;
+  grouped = bottom_up = true;
 }
 
 void Body::init(const float* v3, uint32_t nv_, const uint32_t* t3, uint32_t nf, uint32_t mode_, float depth_,
@@ -217,13 +246,7 @@ void Body::init(const float* v3, uint32_t nv_, const uint32_t* t3, uint32_t nf, 
   d.depth = depth;
   desc.upload(&d, 1, s);
   sort_table.init({d}, {0u}, s);
-  if (bottom_up) {
-    const std::vector<std::vector<LvBlock>> t = build_level_tables({d}, {0u}, [](uint32_t) { return true; });
-    for (int q = 0; q < BB_MAX_LEVELS; ++q) {
-      bu_n[q] = q < (int)t.size() ? (uint32_t)t[q].size() : 0u;
-      if (bu_n[q]) bu_level[q].upload(t[q].data(), t[q].size(), s);
-    }
-  }
+  if (bottom_up) level_setup(s);
   if (mode == CC_BODY_REBUILD && !bottom_up) chain = 1;
   for (int l = 0; l < nlanes * chain; ++l) lane[l].alloc(m, l == 0 || mode == CC_BODY_REBUILD, bottom_up, s);
   // A rebuilt body is walked through wide records folded after each build,

@@ -835,12 +835,16 @@ int cc_body_set_vertices(cc_sim* sim, const float* verts3) {
     CC_HIP(hipDeviceSynchronize());
     Sim& S = sim->s;
     const int k = B.slot_of(S.frame);
-    copy_on(B.rest.p, verts3, 3 * (size_t)B.nv * 4, hipMemcpyHostToDevice, sim->s.stream);
-    copy_on(B.slot[k].verts.p, verts3, 3 * (size_t)B.nv * 4, hipMemcpyHostToDevice, sim->s.stream);
-    // new rest pose: the topology from it as given, then the current frame's pose
-    B.build(k, 0, S.stream);
-    B.share_topology(k, S.stream);
-    S.refresh_body();
+    const size_t bytes = 3 * (size_t)B.nv * 4;
+    CC_HIP(hipMemcpyAsync(B.rest.p, verts3, bytes, hipMemcpyHostToDevice, S.stream));
+    CC_HIP(hipMemcpyAsync(B.slot[k].verts.p, B.rest.p, bytes, hipMemcpyDeviceToDevice, S.stream));
+    // new rest pose: the topology from it as given, then the current frame's
+    // pose (a static body's is the one just built)
+    S.rebuild_body(k);
+    if (B.moving())
+      S.refresh_body();
+    else
+      CC_HIP(hipStreamSynchronize(S.stream));
   });
 }
 
@@ -874,8 +878,7 @@ int cc_bvh_rebuild(cc_sim* sim) {
     CC_HIP(hipDeviceSynchronize());
     Sim& S = sim->s;
     const int k = S.body.slot_of(S.frame);
-    S.body.build(k, 0, S.stream);
-    S.body.share_topology(k, S.stream);
+    S.rebuild_body(k);
     S.ready = S.frame + 1;    // poses computed ahead keep the old boxes
     CC_HIP(hipStreamSynchronize(S.stream));
   });
