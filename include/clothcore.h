@@ -448,8 +448,10 @@ int cc_fault_inject(int kind, int64_t count);
    projected in a step is moved by that fixed plane projection, and the
    contact normal entering the next step's force projection is a constant.
    The spring set must be symmetric (each i->j with a j->i of the same type
-   and rest length).  States are checkpointed every ckpt_every steps and
-   recomputed in the backward pass.  sim must outlive the handle. */
+   and rest length).  A rollout of up to 1 GiB (36 bytes per vertex and step)
+   keeps every state; states of a longer one (or where that memory is not to
+   be had) are checkpointed every ckpt_every steps and recomputed in the
+   backward pass, with the same results.  sim must outlive the handle. */
 typedef struct cc_adj cc_adj;
 int cc_adj_create(cc_sim* sim, uint32_t nsteps, uint32_t ckpt_every, cc_adj** out);
 int cc_adj_destroy(cc_adj* adj);

@@ -16,15 +16,20 @@
 //   lP += 2 lu, lQ -= lu, lF = w (I - c c^T) lu,
 //   F = g m + damp v + sum_j f(d, dv), v = (P - Q)/dt, d = P_i - P_j + eps,
 //   f = alpha d/L, alpha = -k (L - rest) + kd (dv . d)/L.
-// Two kernels: k_adj_force (lu, lF and the vertex-local terms) and
-// k_adj_springs (the spring terms, gathered per vertex: for a spring i->j
-// the side of f_ij weighted by lF_i and, by the symmetry of the spring set
-// (checked at creation), the side of f_ji weighted by lF_j).
+// A step back has two parts: the force part (lu, lF and the vertex-local terms;
+// no neighbour needed) and the spring part (the spring terms, gathered per
+// vertex: for a spring i->j the side of f_ij weighted by lF_i and, by the
+// symmetry of the spring set (checked at creation), the side of f_ji weighted
+// by lF_j).  One launch takes the spring part of step t and the force part of
+// step t - 1, which needs only what this vertex has just finished
+// (k_adj_step); k_adj_force opens a run of steps.
 //
-// Checkpoints every `ckpt` steps; each segment is recomputed forward with
-// its per-step states kept, then stepped back.  Parameter gradients: FP32
-// block sums per step, accumulated per block in FP64, reduced in FP64 on
-// the GPU at the end.
+// A trajectory of up to ADJ_KEEP_BYTES keeps every state of the forward, and
+// the backward steps through them.  A longer one keeps checkpoints every
+// `ckpt` steps; each segment is recomputed forward with its per-step states
+// kept, then stepped back.  The states are the same either way.  Parameter
+// gradients: FP32 sums per step and block of 256 vertices, accumulated per
+// block in FP64 (k_adj_acc), reduced in FP64 on the GPU at the end.
 #include <cstring>
 #include <memory>
 
@@ -35,6 +40,10 @@ namespace cc {
 
 constexpr int ADJ_THREADS = 256;
 constexpr int NPARAM = 5;   // k0, k1, k2, damp, rest_scale
+// All states of a rollout are kept up to this size (36 bytes per vertex and
+// step): 128 x 128 vertices over 200 steps take 118 MB, and recomputing them
+// took 1.1 of the 3.6 ms of their backward.  1 GiB is a 1/288 of the card.
+constexpr size_t ADJ_KEEP_BYTES = (size_t)1 << 30;
 
 struct AdjArgs {
   float dt, inv_dt, w, damp, kd, k0, k1, k2, rest_scale, eps;
@@ -61,162 +70,259 @@ __device__ inline void spring_vjp(f3 d, f3 dv, float ks, float rest, float kd, f
   dl = l;
 }
 
-// Sum v over the block (64-wide waves, ADJ_THREADS / 64 of them); the
-// result is valid in thread 0.
+// Sum over a wave of 64 vertices (one per lane), valid in lane 0.
 template <int K>
-__device__ inline void block_sum(float (&v)[K]) {
-  __shared__ float part[ADJ_THREADS / 64][K];
+__device__ inline void wave_sum(float (&v)[K]) {
 #pragma unroll
   for (int k = 0; k < K; ++k)
     for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int k = 0; k < K; ++k) part[threadIdx.x >> 6][k] = v[k];
-  __syncthreads();
-  if (threadIdx.x == 0)
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      float s = 0.0f;
-      for (int w = 0; w < ADJ_THREADS / 64; ++w) s += part[w][k];
-      v[k] = s;
-    }
+}
+
+// The force part of a step for one vertex: its adjoint lP, lQ after the step,
+// the contact normals before (c) and after (nn) it, its state s before it.
+struct AdjForce {
+  f3 lF, gp, gq;     // lF, and the vertex-local terms of lP, lQ before the step
+  float damp;        // lF . vel
+};
+__device__ inline AdjForce adj_force(f3 lP, f3 lQ, bool pinned, f3 c, f3 nn, f3 sp, f3 sq, const AdjArgs& a) {
+  AdjForce r{mk(0.0f, 0.0f, 0.0f), mk(0.0f, 0.0f, 0.0f), mk(0.0f, 0.0f, 0.0f), 0.0f};
+  if (pinned) {
+    r.gp = lP + lQ;
+    return r;
+  }
+  f3 lu;
+  if (nn.x != 0.0f || nn.y != 0.0f || nn.z != 0.0f) {
+    const f3 s2 = lP + lQ;
+    const float ns = fmaf(nn.z, s2.z, fmaf(nn.y, s2.y, nn.x * s2.x));
+    lu = mk(fmaf(-nn.x, ns, s2.x), fmaf(-nn.y, ns, s2.y), fmaf(-nn.z, ns, s2.z));
+  } else {
+    lu = lP;
+    r.gp = lQ;
+  }
+  r.gp = mk(fmaf(2.0f, lu.x, r.gp.x), fmaf(2.0f, lu.y, r.gp.y), fmaf(2.0f, lu.z, r.gp.z));
+  r.gq = mk(-lu.x, -lu.y, -lu.z);
+  const float cl = fmaf(c.z, lu.z, fmaf(c.y, lu.y, c.x * lu.x));
+  r.lF = mk(a.w * fmaf(-c.x, cl, lu.x), a.w * fmaf(-c.y, cl, lu.y), a.w * fmaf(-c.z, cl, lu.z));
+  const f3 vel = mk((sp.x - sq.x) * a.inv_dt, (sp.y - sq.y) * a.inv_dt, (sp.z - sq.z) * a.inv_dt);
+  r.damp = fmaf(r.lF.z, vel.z, fmaf(r.lF.y, vel.y, r.lF.x * vel.x));   // F += damp * vel
+  const float dd = a.damp * a.inv_dt;
+  r.gp = mk(fmaf(dd, r.lF.x, r.gp.x), fmaf(dd, r.lF.y, r.gp.y), fmaf(dd, r.lF.z, r.gp.z));
+  r.gq = mk(fmaf(-dd, r.lF.x, r.gq.x), fmaf(-dd, r.lF.y, r.gq.y), fmaf(-dd, r.lF.z, r.gq.z));
+  return r;
 }
 
 __global__ __launch_bounds__(ADJ_THREADS) void k_adj_force(
     uint32_t n, const uint32_t* __restrict__ row, const float* __restrict__ state,
     const float* __restrict__ c_in, const float* __restrict__ c_out, const float* __restrict__ lp,
     const float* __restrict__ lq, AdjArgs a, float* __restrict__ lf, float* __restrict__ locp,
-    float* __restrict__ locq, double* __restrict__ acc) {
+    float* __restrict__ locq, float* __restrict__ part) {
   const uint32_t i = blockIdx.x * ADJ_THREADS + threadIdx.x;
   float g[1] = {0.0f};
   if (i < n) {
-    const f3 lP = ld3(lp + 3 * (size_t)i), lQ = ld3(lq + 3 * (size_t)i);
-    f3 gp = mk(0.0f, 0.0f, 0.0f), gq = mk(0.0f, 0.0f, 0.0f), lF = mk(0.0f, 0.0f, 0.0f);
-    if (row[i] & PIN_BIT) {
-      gp = lP + lQ;
-    } else {
-      const f3 nn = ld3(c_out + 3 * (size_t)i);
-      f3 lu;
-      if (nn.x != 0.0f || nn.y != 0.0f || nn.z != 0.0f) {
-        const f3 s2 = lP + lQ;
-        const float ns = fmaf(nn.z, s2.z, fmaf(nn.y, s2.y, nn.x * s2.x));
-        lu = mk(fmaf(-nn.x, ns, s2.x), fmaf(-nn.y, ns, s2.y), fmaf(-nn.z, ns, s2.z));
-      } else {
-        lu = lP;
-        gp = lQ;
-      }
-      gp = mk(fmaf(2.0f, lu.x, gp.x), fmaf(2.0f, lu.y, gp.y), fmaf(2.0f, lu.z, gp.z));
-      gq = mk(-lu.x, -lu.y, -lu.z);
-      const f3 c = ld3(c_in + 3 * (size_t)i);
-      const float cl = fmaf(c.z, lu.z, fmaf(c.y, lu.y, c.x * lu.x));
-      lF = mk(a.w * fmaf(-c.x, cl, lu.x), a.w * fmaf(-c.y, cl, lu.y), a.w * fmaf(-c.z, cl, lu.z));
-      const float* s = state + 6 * (size_t)i;
-      const f3 vel = mk((s[0] - s[3]) * a.inv_dt, (s[1] - s[4]) * a.inv_dt, (s[2] - s[5]) * a.inv_dt);
-      g[0] = fmaf(lF.z, vel.z, fmaf(lF.y, vel.y, lF.x * vel.x));   // F += damp * vel
-      const float dd = a.damp * a.inv_dt;
-      gp = mk(fmaf(dd, lF.x, gp.x), fmaf(dd, lF.y, gp.y), fmaf(dd, lF.z, gp.z));
-      gq = mk(fmaf(-dd, lF.x, gq.x), fmaf(-dd, lF.y, gq.y), fmaf(-dd, lF.z, gq.z));
-    }
-    st3(lf + 3 * (size_t)i, lF);
-    st3(locp + 3 * (size_t)i, gp);
-    st3(locq + 3 * (size_t)i, gq);
+    const size_t o = 3 * (size_t)i;
+    const AdjForce r = adj_force(ld3(lp + o), ld3(lq + o), (row[i] & PIN_BIT) != 0, ld3(c_in + o), ld3(c_out + o),
+                                 ld3(state + 2 * o), ld3(state + 2 * o + 3), a);
+    st3(lf + o, r.lF);
+    st3(locp + o, r.gp);
+    st3(locq + o, r.gq);
+    g[0] = r.damp;
   }
-  block_sum(g);
-  if (threadIdx.x == 0) acc[NPARAM * blockIdx.x + 3] += (double)g[0];
+  wave_sum(g);
+  if ((threadIdx.x & 63u) == 0 && i < n) part[NPARAM * (size_t)(i >> 6) + 3] = g[0];
 }
 
-// One spring's adjoint terms (the forward's f_ij in F_i and f_ji in F_j)
-// added to gp, gq and the parameter gradients g.
-__device__ inline void adj_spring_term(f3 pi, f3 vi, f3 lFi, f3 pj, f3 vj, f3 lFj, uint2 r, const AdjArgs& a, f3& gp,
-                                       f3& gq, float (&g)[4]) {
-  const uint32_t t = r.x >> 30;
+// One spring's adjoint terms (the forward's f_ij in F_i and f_ji in F_j):
+// gp += a1, gq -= v1 / dt, gp -= a2, gq += v2 / dt, in that order, and its
+// parts gk, gr of the gradients of its type's stiffness and of rest_scale.
+// All zero for an empty slot.
+struct AdjTerm {
+  f3 a1, v1, a2, v2;
+  float gk, gr;
+  uint32_t t;
+};
+__device__ inline AdjTerm adj_spring(f3 pi, f3 vi, f3 lFi, f3 pj, f3 vj, f3 lFj, uint2 r, bool real,
+                                     const AdjArgs& a) {
+  AdjTerm o;
+  o.t = r.x >> 30;
   const float rest0 = __uint_as_float(r.y), rest = rest0 * a.rest_scale;
-  const float ks = t == 0 ? a.k0 : (t == 1 ? a.k1 : a.k2);
-  f3 gd, gdv;
+  const float ks = o.t == 0 ? a.k0 : (o.t == 1 ? a.k1 : a.k2);
+  f3 gd;
   float dl, L;
   // f_ij, in F_i
   spring_vjp(mk((pi.x - pj.x) + a.eps, (pi.y - pj.y) + a.eps, (pi.z - pj.z) + a.eps), vi - vj, ks, rest, a.kd, lFi,
-             gd, gdv, dl, L);
-  gp = mk(gp.x + fmaf(gdv.x, a.inv_dt, gd.x), gp.y + fmaf(gdv.y, a.inv_dt, gd.y), gp.z + fmaf(gdv.z, a.inv_dt, gd.z));
-  gq = mk(fmaf(-gdv.x, a.inv_dt, gq.x), fmaf(-gdv.y, a.inv_dt, gq.y), fmaf(-gdv.z, a.inv_dt, gq.z));
-  const float gk = -(L - rest) * dl;
-  g[0] += t == 0 ? gk : 0.0f;
-  g[1] += t == 1 ? gk : 0.0f;
-  g[2] += t == 2 ? gk : 0.0f;
-  g[3] += ks * rest0 * dl;
+             gd, o.v1, dl, L);
+  o.a1 = mk(fmaf(o.v1.x, a.inv_dt, gd.x), fmaf(o.v1.y, a.inv_dt, gd.y), fmaf(o.v1.z, a.inv_dt, gd.z));
+  o.gk = -(L - rest) * dl;
+  o.gr = ks * rest0 * dl;
   // f_ji, in F_j (the same type and rest length)
   spring_vjp(mk((pj.x - pi.x) + a.eps, (pj.y - pi.y) + a.eps, (pj.z - pi.z) + a.eps), vj - vi, ks, rest, a.kd, lFj,
-             gd, gdv, dl, L);
-  gp = mk(gp.x - fmaf(gdv.x, a.inv_dt, gd.x), gp.y - fmaf(gdv.y, a.inv_dt, gd.y), gp.z - fmaf(gdv.z, a.inv_dt, gd.z));
-  gq = mk(fmaf(gdv.x, a.inv_dt, gq.x), fmaf(gdv.y, a.inv_dt, gq.y), fmaf(gdv.z, a.inv_dt, gq.z));
+             gd, o.v2, dl, L);
+  o.a2 = mk(fmaf(o.v2.x, a.inv_dt, gd.x), fmaf(o.v2.y, a.inv_dt, gd.y), fmaf(o.v2.z, a.inv_dt, gd.z));
+  if (!real) {
+    const f3 z = mk(0.0f, 0.0f, 0.0f);
+    o = AdjTerm{z, z, z, z, 0.0f, 0.0f, 3u};
+  }
+  return o;
+}
+// Its sum into gp, gq and the parameter gradients g = {k0, k1, k2, -, rest_scale}.
+__device__ inline void adj_add(const AdjTerm& o, float inv_dt, f3& gp, f3& gq, float (&g)[NPARAM]) {
+  gp = gp + o.a1;
+  gq = mk(fmaf(-o.v1.x, inv_dt, gq.x), fmaf(-o.v1.y, inv_dt, gq.y), fmaf(-o.v1.z, inv_dt, gq.z));
+  g[0] += o.t == 0 ? o.gk : 0.0f;
+  g[1] += o.t == 1 ? o.gk : 0.0f;
+  g[2] += o.t == 2 ? o.gk : 0.0f;
+  g[4] += o.gr;
+  gp = gp - o.a2;
+  gq = mk(fmaf(o.v2.x, inv_dt, gq.x), fmaf(o.v2.y, inv_dt, gq.y), fmaf(o.v2.z, inv_dt, gq.z));
+}
+template <int K>
+__device__ inline f3 quad_bcast3(f3 v) {
+  return mk(quad_bcast<K>(v.x), quad_bcast<K>(v.y), quad_bcast<K>(v.z));
+}
+// lane K's terms added in every lane of the quad, in their order
+template <int K, int NB>
+__device__ inline void quad_adj_add(const AdjTerm (&t)[NB], float inv_dt, f3& gp, f3& gq, float (&g)[NPARAM]) {
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const AdjTerm o{quad_bcast3<K>(t[k].a1), quad_bcast3<K>(t[k].v1), quad_bcast3<K>(t[k].a2),
+                    quad_bcast3<K>(t[k].v2), quad_bcast<K>(t[k].gk),  quad_bcast<K>(t[k].gr),
+                    (uint32_t)quad_perm<K * 0x55>((int32_t)t[k].t)};
+    adj_add(o, inv_dt, gp, gq, g);
+  }
 }
 
-// EW > 0: `rec` holds EW records per vertex (the forward's fixed-width rows,
-// empty slots of type 3 skipped), loaded with the vertex's own data and
-// gathered six at a time; EW == 0: the merged CSR at `row`, one spring after
-// another.  The same springs in the same order either way.
-template <int EW>
-__global__ __launch_bounds__(ADJ_THREADS) void k_adj_springs(
-    uint32_t n, const uint32_t* __restrict__ row, const uint2* __restrict__ rec, const float* __restrict__ state,
-    const float* __restrict__ lf, const float* __restrict__ locp, const float* __restrict__ locq, AdjArgs a,
-    float* __restrict__ lp_out, float* __restrict__ lq_out, double* __restrict__ acc) {
-  const uint32_t i = blockIdx.x * ADJ_THREADS + threadIdx.x;
-  float g[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // k0, k1, k2, rest_scale
+// What a launch of k_adj_step reads and writes: step t's records and springs,
+// and for the force part of step t - 1 its state and contact normals (state1
+// null: the first step of a run, whose adjoint goes to lp, lq).
+struct AdjStep {
+  const float *state, *lf, *locp, *locq;          // of step t
+  const float *state1, *c_in1, *c_out1;           // of step t - 1
+  float *lf1, *locp1, *locq1;                     // out: the force part of step t - 1
+  float *lp, *lq;                                 // out: dL/dx_cur, dL/dx_prev before step t
+  float *part, *part1;                            // out: parameter sums of 64 vertices each, of steps t, t - 1
+};
+
+// The spring part of step t and the force part of step t - 1.  LANES lanes per
+// vertex (4: a quad, each lane a quarter of the springs, their terms added in
+// row order in every lane); the parameter sums go out per 64 vertices, so they
+// add the same numbers in the same order either way.  EW > 0: `rec` holds EW
+// records per vertex (the forward's fixed-width rows); EW == 0: the merged CSR
+// at `row`.  Bound by the chain from the records to the gathers and the terms
+// (two square roots and divisions each) on a chip that one lane per vertex
+// fills to a quarter at 128 x 128: 200 steps back take 1.3 ms (6.1 us a step,
+// 101 VGPRs), against 3.6 with two launches a step (9.2 + 2.9), one lane per
+// vertex and the states recomputed (5.3).
+template <int EW, int LANES>
+__global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint32_t* __restrict__ row,
+                                                          const uint2* __restrict__ rec, AdjStep S, AdjArgs a) {
+  constexpr bool QUAD = LANES == 4;
+  constexpr int NB = EW && QUAD ? EW / 4 : (QUAD ? 3 : (EW ? 6 : 4));   // springs of a lane at a time
+  constexpr uint32_t VERTS = ADJ_THREADS / LANES;
+  __shared__ float sg[QUAD ? VERTS : 1][NPARAM];
+  const uint32_t v = threadIdx.x / LANES, i = blockIdx.x * VERTS + v;
+  const int e = (int)(threadIdx.x % LANES);
+  float g[NPARAM] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   if (i < n) {
-    uint2 er[EW ? EW : 1];
-    if constexpr (EW > 0) {
-#pragma unroll
-      for (int k = 0; k < EW; ++k) er[k] = rec[(size_t)i * EW + k];
+    const size_t o = 3 * (size_t)i;
+    const uint32_t r0raw = row[i], r1raw = EW ? 0u : row[i + 1];
+    const f3 pi = ld3(S.state + 2 * o), qi = ld3(S.state + 2 * o + 3);
+    const f3 lFi = ld3(S.lf + o);
+    f3 gp = ld3(S.locp + o), gq = ld3(S.locq + o);
+    // the force part's own loads, early
+    f3 c1 = mk(0.0f, 0.0f, 0.0f), n1 = c1, p1 = c1, q1 = c1;
+    if (S.state1) {
+      c1 = ld3(S.c_in1 + o);
+      n1 = ld3(S.c_out1 + o);
+      p1 = ld3(S.state1 + 2 * o);
+      q1 = ld3(S.state1 + 2 * o + 3);
     }
-    const float* s = state + 6 * (size_t)i;
-    const f3 pi = mk(s[0], s[1], s[2]);
-    const f3 vi = mk((s[0] - s[3]) * a.inv_dt, (s[1] - s[4]) * a.inv_dt, (s[2] - s[5]) * a.inv_dt);
-    const f3 lFi = ld3(lf + 3 * (size_t)i);
-    f3 gp = ld3(locp + 3 * (size_t)i), gq = ld3(locq + 3 * (size_t)i);
-    if constexpr (EW > 0) {
-      constexpr int GB = 6;
+    const f3 vi = mk((pi.x - qi.x) * a.inv_dt, (pi.y - qi.y) * a.inv_dt, (pi.z - qi.z) * a.inv_dt);
+    const uint32_t r0 = EW ? i * (uint32_t)EW : r0raw & ROW_MASK, r1 = EW ? r0 + EW : r1raw & ROW_MASK;
+    for (uint32_t k0 = r0; k0 < r1; k0 += NB * LANES) {
+      uint2 er[NB];
+      bool real[NB];
+      float sj[NB][6], lj[NB][3];
 #pragma unroll
-      for (int b0 = 0; b0 < EW; b0 += GB) {
-        float sj[GB][6], lj[GB][3];
-#pragma unroll
-        for (int k = 0; k < GB; ++k) {
-          const uint32_t j = er[b0 + k].x & END_MASK;
-          const float2* s2 = reinterpret_cast<const float2*>(state + 6 * (size_t)j);
-          const float2 u = s2[0], v = s2[1], w = s2[2];
-          sj[k][0] = u.x; sj[k][1] = u.y; sj[k][2] = v.x; sj[k][3] = v.y; sj[k][4] = w.x; sj[k][5] = w.y;
-          lj[k][0] = lf[3 * (size_t)j]; lj[k][1] = lf[3 * (size_t)j + 1]; lj[k][2] = lf[3 * (size_t)j + 2];
-        }
-#pragma unroll
-        for (int k = 0; k < GB; ++k) {
-          if ((er[b0 + k].x & PAD_TYPE) == PAD_TYPE) continue;
-          const f3 pj = mk(sj[k][0], sj[k][1], sj[k][2]);
-          const f3 vj = mk((sj[k][0] - sj[k][3]) * a.inv_dt, (sj[k][1] - sj[k][4]) * a.inv_dt,
-                           (sj[k][2] - sj[k][5]) * a.inv_dt);
-          adj_spring_term(pi, vi, lFi, pj, vj, mk(lj[k][0], lj[k][1], lj[k][2]), er[b0 + k], a, gp, gq, g);
-        }
+      for (int k = 0; k < NB; ++k) {
+        const uint32_t at = k0 + (uint32_t)(e * NB + k);
+        er[k] = rec[EW ? at : min(at, r1 - 1)];
+        real[k] = EW ? (er[k].x & PAD_TYPE) != PAD_TYPE : at < r1;
+        if (!EW && !real[k]) er[k] = make_uint2(i | PAD_TYPE, 0u);
       }
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const uint32_t j = er[k].x & END_MASK;
+        const float2* s2 = reinterpret_cast<const float2*>(S.state + 6 * (size_t)j);
+        const float2 u = s2[0], w = s2[1], x = s2[2];
+        sj[k][0] = u.x; sj[k][1] = u.y; sj[k][2] = w.x; sj[k][3] = w.y; sj[k][4] = x.x; sj[k][5] = x.y;
+        for (int c = 0; c < 3; ++c) lj[k][c] = S.lf[3 * (size_t)j + c];
+      }
+      AdjTerm t[NB];
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const f3 pj = mk(sj[k][0], sj[k][1], sj[k][2]);
+        const f3 vj = mk((sj[k][0] - sj[k][3]) * a.inv_dt, (sj[k][1] - sj[k][4]) * a.inv_dt,
+                         (sj[k][2] - sj[k][5]) * a.inv_dt);
+        t[k] = adj_spring(pi, vi, lFi, pj, vj, mk(lj[k][0], lj[k][1], lj[k][2]), er[k], real[k], a);
+        if constexpr (!QUAD) adj_add(t[k], a.inv_dt, gp, gq, g);
+      }
+      if constexpr (QUAD) {
+        quad_adj_add<0>(t, a.inv_dt, gp, gq, g);
+        quad_adj_add<1>(t, a.inv_dt, gp, gq, g);
+        quad_adj_add<2>(t, a.inv_dt, gp, gq, g);
+        quad_adj_add<3>(t, a.inv_dt, gp, gq, g);
+      }
+    }
+    if (S.state1) {
+      const AdjForce r = adj_force(gp, gq, (r0raw & PIN_BIT) != 0, c1, n1, p1, q1, a);
+      g[3] = r.damp;
+      if (!QUAD || e == 0) st3(S.lf1 + o, r.lF);
+      if (!QUAD || e == 1) st3(S.locp1 + o, r.gp);
+      if (!QUAD || e == 2) st3(S.locq1 + o, r.gq);
     } else {
-      const uint32_t r0 = row[i] & ROW_MASK, r1 = row[i + 1] & ROW_MASK;
-      for (uint32_t k = r0; k < r1; ++k) {
-        const uint2 r = rec[k];
-        const uint32_t j = r.x & END_MASK;
-        const float* sj = state + 6 * (size_t)j;
-        const f3 pj = mk(sj[0], sj[1], sj[2]);
-        const f3 vj = mk((sj[0] - sj[3]) * a.inv_dt, (sj[1] - sj[4]) * a.inv_dt, (sj[2] - sj[5]) * a.inv_dt);
-        adj_spring_term(pi, vi, lFi, pj, vj, ld3(lf + 3 * (size_t)j), r, a, gp, gq, g);
-      }
+      if (!QUAD || e == 0) st3(S.lp + o, gp);
+      if (!QUAD || e == 1) st3(S.lq + o, gq);
     }
-    st3(lp_out + 3 * (size_t)i, gp);
-    st3(lq_out + 3 * (size_t)i, gq);
+    if (QUAD && e == 3)
+      for (int k = 0; k < NPARAM; ++k) sg[v][k] = g[k];
   }
-  block_sum(g);
-  if (threadIdx.x == 0) {
-    double* ab = acc + NPARAM * (size_t)blockIdx.x;
-    ab[0] += (double)g[0];
-    ab[1] += (double)g[1];
-    ab[2] += (double)g[2];
-    ab[4] += (double)g[3];
+  uint32_t v0 = i;                       // this lane's vertex in the sums
+  if constexpr (QUAD) {                  // one vertex per lane again, in the first wave
+    static_assert(VERTS == 64, "one wave of vertices per block");
+    __syncthreads();
+    if (threadIdx.x >= VERTS) return;
+    v0 = blockIdx.x * VERTS + threadIdx.x;
+    for (int k = 0; k < NPARAM; ++k) g[k] = v0 < n ? sg[threadIdx.x][k] : 0.0f;
   }
+  wave_sum(g);
+  if ((threadIdx.x & 63u) == 0 && v0 < n) {
+    const size_t w = NPARAM * (size_t)(v0 >> 6);
+    for (int k = 0; k < NPARAM; ++k)
+      if (k != 3) S.part[w + k] = g[k];
+    if (S.state1) S.part1[w + 3] = g[3];
+  }
+}
+
+// acc[b] += the sums of L steps, last step first, over blocks of ADJ_THREADS
+// vertices (four waves each, added in order in FP32): thread = block and
+// parameter.
+__global__ __launch_bounds__(256) void k_adj_acc(const float* __restrict__ part, uint32_t L, uint32_t nw,
+                                                 uint32_t nblk, double* __restrict__ acc) {
+  const uint32_t q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= NPARAM * nblk) return;
+  const uint32_t b = q / NPARAM, p = q % NPARAM, w0 = 4 * b;
+  double s = acc[q];
+#pragma unroll 8
+  for (uint32_t t = L; t-- > 0;) {
+    const float* x = part + NPARAM * ((size_t)t * nw + w0) + p;
+    float f = 0.0f;
+    f += x[0];
+    f += w0 + 1 < nw ? x[NPARAM] : 0.0f;
+    f += w0 + 2 < nw ? x[2 * NPARAM] : 0.0f;
+    f += w0 + 3 < nw ? x[3 * NPARAM] : 0.0f;
+    s += (double)f;
+  }
+  acc[q] = s;
 }
 
 // out[p] = sum over blocks of acc[p], in FP64 (one workgroup)
@@ -244,10 +350,12 @@ struct Adj {
   StepArgs sa{};
   AdjArgs aa{};
   bool have_forward = false;
+  bool keep = false;                     // seg_state / seg_contact hold every state of the forward
   DBuf<float> st[2], contact;
   DBuf<float> ck_state, ck_contact;      // [nck][6n], [nck][3n]
   DBuf<float> seg_state, seg_contact;    // [ckpt+1][6n], [ckpt+1][3n]
-  DBuf<float> lp[2], lq[2], lf, locp, locq;
+  DBuf<float> lp, lq, lf[2], locp[2], locq[2];
+  DBuf<float> part;                      // [ckpt][ceil(n / 64)][NPARAM]
   DBuf<double> acc, out;
   ~Adj() {
     if (S && S->stream) (void)hipStreamSynchronize(S->stream);   // before the buffers are freed
@@ -296,19 +404,34 @@ int cc_adj_create(cc_sim* sim, uint32_t nsteps, uint32_t ckpt_every, cc_adj** ou
     A.nck = (nsteps + A.ckpt - 1) / A.ckpt;
     A.nblk = grid_for(S.n, ADJ_THREADS);
     const size_t n3 = 3 * (size_t)S.n, n6 = 6 * (size_t)S.n;
-    for (int b = 0; b < 2; ++b) {
-      A.st[b].alloc(n6);
-      A.lp[b].alloc(n3);
-      A.lq[b].alloc(n3);
+    // Every state where that takes little memory, checkpoints otherwise (also
+    // when that memory is not to be had).
+    if (((size_t)nsteps + 1) * (n6 + n3) * sizeof(float) <= ADJ_KEEP_BYTES) try {
+        A.seg_state.alloc(((size_t)nsteps + 1) * n6);
+        A.seg_contact.alloc(((size_t)nsteps + 1) * n3);
+        A.keep = true;
+        A.ckpt = nsteps;
+        A.nck = 1;
+      } catch (const Error& e) {
+        if (e.code != CC_ERR_ALLOC) throw;
+        A.seg_state.release();
+      }
+    if (!A.keep) {
+      for (int b = 0; b < 2; ++b) A.st[b].alloc(n6);
+      A.contact.alloc(n3);
+      A.ck_state.alloc(A.nck * n6);
+      A.ck_contact.alloc(A.nck * n3);
+      A.seg_state.alloc((A.ckpt + 1) * n6);
+      A.seg_contact.alloc((A.ckpt + 1) * n3);
     }
-    A.contact.alloc(n3);
-    A.ck_state.alloc(A.nck * n6);
-    A.ck_contact.alloc(A.nck * n3);
-    A.seg_state.alloc((A.ckpt + 1) * n6);
-    A.seg_contact.alloc((A.ckpt + 1) * n3);
-    A.lf.alloc(n3);
-    A.locp.alloc(n3);
-    A.locq.alloc(n3);
+    A.lp.alloc(n3);
+    A.lq.alloc(n3);
+    for (int b = 0; b < 2; ++b) {
+      A.lf[b].alloc(n3);
+      A.locp[b].alloc(n3);
+      A.locq[b].alloc(n3);
+    }
+    A.part.alloc((size_t)A.ckpt * grid_for(S.n, 64) * NPARAM);
     A.acc.alloc(NPARAM * (size_t)A.nblk);
     A.out.alloc(NPARAM);
     *out = h.release();
@@ -353,20 +476,31 @@ int cc_adj_forward(cc_adj* adj, const float* x0, const float* v0, const double t
         packed[6 * (size_t)i + c] = x;
         packed[6 * (size_t)i + 3 + c] = x - v * A.prm.dt;
       }
-    CC_HIP(hipMemcpyAsync(A.st[0].p, packed.data(), n6 * sizeof(float), hipMemcpyHostToDevice, s));
-    A.contact.zero(s);
-    int cur = 0;
-    for (uint32_t t = 0; t < A.nsteps; ++t) {
-      if (t % A.ckpt == 0) {
-        const uint32_t c = t / A.ckpt;
-        CC_HIP(hipMemcpyAsync(A.ck_state.p + c * n6, A.st[cur].p, n6 * sizeof(float), hipMemcpyDeviceToDevice, s));
-        CC_HIP(hipMemcpyAsync(A.ck_contact.p + c * n3, A.contact.p, n3 * sizeof(float), hipMemcpyDeviceToDevice, s));
+    float* const x_in = A.keep ? A.seg_state.p : A.st[0].p;
+    float* const c_in = A.keep ? A.seg_contact.p : A.contact.p;
+    CC_HIP(hipMemcpyAsync(x_in, packed.data(), n6 * sizeof(float), hipMemcpyHostToDevice, s));
+    CC_HIP(hipMemsetAsync(c_in, 0, n3 * sizeof(float), s));
+    const float* x_out = nullptr;
+    if (A.keep) {
+      for (uint32_t t = 0; t < A.nsteps; ++t)
+        S.launch_step(A.seg_state.p + t * n6, A.seg_state.p + (t + 1) * n6, A.seg_contact.p + t * n3,
+                      A.seg_contact.p + (t + 1) * n3, A.sa, 0, s);
+      x_out = A.seg_state.p + A.nsteps * n6;
+    } else {
+      int cur = 0;
+      for (uint32_t t = 0; t < A.nsteps; ++t) {
+        if (t % A.ckpt == 0) {
+          const uint32_t c = t / A.ckpt;
+          CC_HIP(hipMemcpyAsync(A.ck_state.p + c * n6, A.st[cur].p, n6 * sizeof(float), hipMemcpyDeviceToDevice, s));
+          CC_HIP(hipMemcpyAsync(A.ck_contact.p + c * n3, A.contact.p, n3 * sizeof(float), hipMemcpyDeviceToDevice, s));
+        }
+        S.launch_step(A.st[cur].p, A.st[cur ^ 1].p, A.contact.p, A.contact.p, A.sa, 0, s);
+        cur ^= 1;
       }
-      S.launch_step(A.st[cur].p, A.st[cur ^ 1].p, A.contact.p, A.contact.p, A.sa, 0, s);
-      cur ^= 1;
+      x_out = A.st[cur].p;
     }
     if (x_final) {
-      CC_HIP(hipMemcpyAsync(packed.data(), A.st[cur].p, n6 * sizeof(float), hipMemcpyDeviceToHost, s));
+      CC_HIP(hipMemcpyAsync(packed.data(), x_out, n6 * sizeof(float), hipMemcpyDeviceToHost, s));
       CC_HIP(hipStreamSynchronize(s));
       for (uint32_t i = 0; i < A.n; ++i)
         for (int c = 0; c < 3; ++c) x_final[3 * (size_t)i + c] = packed[6 * (size_t)i + c];
@@ -384,42 +518,66 @@ int cc_adj_backward(cc_adj* adj, const float* dl_dx_final, double dl_dtheta[5], 
     Sim& S = *A.S;
     hipStream_t s = S.stream;
     const size_t n3 = 3 * (size_t)A.n, n6 = 6 * (size_t)A.n;
-    CC_HIP(hipMemcpyAsync(A.lp[0].p, dl_dx_final, n3 * sizeof(float), hipMemcpyHostToDevice, s));
-    A.lq[0].zero(s);
+    CC_HIP(hipMemcpyAsync(A.lp.p, dl_dx_final, n3 * sizeof(float), hipMemcpyHostToDevice, s));
+    A.lq.zero(s);
     A.acc.zero(s);
-    int cur = 0;
+    // four lanes per vertex up to the size where the forward's step takes them
+    const bool quads = A.n <= QUAD_MAX_N, ell = S.ell_w == ELL_W;
+    const uint2* recs = ell ? S.ell.p : S.rec.p;
+    auto kern = ell ? (quads ? k_adj_step<ELL_W, 4> : k_adj_step<ELL_W, 1>)
+                    : (quads ? k_adj_step<0, 4> : k_adj_step<0, 1>);
+    const unsigned grid = grid_for(A.n, quads ? ADJ_THREADS / 4 : ADJ_THREADS);
+    const uint32_t nw = grid_for(A.n, 64);
+    auto part = [&](uint32_t j) { return A.part.p + (size_t)j * nw * NPARAM; };
     for (uint32_t c = A.nck; c-- > 0;) {
       const uint32_t t0 = c * A.ckpt, t1 = std::min(t0 + A.ckpt, A.nsteps), L = t1 - t0;
-      // the segment forward again, keeping every state
-      CC_HIP(hipMemcpyAsync(A.seg_state.p, A.ck_state.p + c * n6, n6 * sizeof(float), hipMemcpyDeviceToDevice, s));
-      CC_HIP(hipMemcpyAsync(A.seg_contact.p, A.ck_contact.p + c * n3, n3 * sizeof(float), hipMemcpyDeviceToDevice,
-                            s));
-      for (uint32_t j = 0; j < L; ++j)   // contact normals of step j in, of step j + 1 out
-        S.launch_step(A.seg_state.p + j * n6, A.seg_state.p + (j + 1) * n6, A.seg_contact.p + j * n3,
-                      A.seg_contact.p + (j + 1) * n3, A.sa, 0, s);
+      if (!A.keep) {
+        // the segment forward again, keeping every state
+        CC_HIP(hipMemcpyAsync(A.seg_state.p, A.ck_state.p + c * n6, n6 * sizeof(float), hipMemcpyDeviceToDevice, s));
+        CC_HIP(hipMemcpyAsync(A.seg_contact.p, A.ck_contact.p + c * n3, n3 * sizeof(float), hipMemcpyDeviceToDevice,
+                              s));
+        for (uint32_t j = 0; j < L; ++j)   // contact normals of step j in, of step j + 1 out
+          S.launch_step(A.seg_state.p + j * n6, A.seg_state.p + (j + 1) * n6, A.seg_contact.p + j * n3,
+                        A.seg_contact.p + (j + 1) * n3, A.sa, 0, s);
+      }
+      auto st = [&](uint32_t j) { return A.seg_state.p + j * n6; };
+      auto ct = [&](uint32_t j) { return A.seg_contact.p + j * n3; };
+      int cur = 0;
+      k_adj_force<<<A.nblk, ADJ_THREADS, 0, s>>>(A.n, S.row.p, st(L - 1), ct(L - 1), ct(L), A.lp.p, A.lq.p, A.aa,
+                                                 A.lf[0].p, A.locp[0].p, A.locq[0].p, part(L - 1));
+      CC_LAUNCHED();
       for (uint32_t j = L; j-- > 0;) {
-        const float* stj = A.seg_state.p + j * n6;
-        k_adj_force<<<A.nblk, ADJ_THREADS, 0, s>>>(A.n, S.row.p, stj, A.seg_contact.p + j * n3,
-                                                   A.seg_contact.p + (j + 1) * n3, A.lp[cur].p, A.lq[cur].p, A.aa,
-                                                   A.lf.p, A.locp.p, A.locq.p, A.acc.p);
-        CC_LAUNCHED();
-        if (S.ell_w == ELL_W)
-          k_adj_springs<ELL_W><<<A.nblk, ADJ_THREADS, 0, s>>>(A.n, S.row.p, S.ell.p, stj, A.lf.p, A.locp.p,
-                                                              A.locq.p, A.aa, A.lp[cur ^ 1].p, A.lq[cur ^ 1].p,
-                                                              A.acc.p);
-        else
-          k_adj_springs<0><<<A.nblk, ADJ_THREADS, 0, s>>>(A.n, S.row.p, S.rec.p, stj, A.lf.p, A.locp.p, A.locq.p,
-                                                          A.aa, A.lp[cur ^ 1].p, A.lq[cur ^ 1].p, A.acc.p);
+        AdjStep D{};
+        D.state = st(j);
+        D.lf = A.lf[cur].p;
+        D.locp = A.locp[cur].p;
+        D.locq = A.locq[cur].p;
+        D.part = part(j);
+        if (j > 0) {
+          D.part1 = part(j - 1);
+          D.state1 = st(j - 1);
+          D.c_in1 = ct(j - 1);
+          D.c_out1 = ct(j);
+          D.lf1 = A.lf[cur ^ 1].p;
+          D.locp1 = A.locp[cur ^ 1].p;
+          D.locq1 = A.locq[cur ^ 1].p;
+        } else {
+          D.lp = A.lp.p;
+          D.lq = A.lq.p;
+        }
+        kern<<<grid, ADJ_THREADS, 0, s>>>(A.n, S.row.p, recs, D, A.aa);
         CC_LAUNCHED();
         cur ^= 1;
       }
+      k_adj_acc<<<grid_for(NPARAM * (size_t)A.nblk, 256), 256, 0, s>>>(A.part.p, L, nw, A.nblk, A.acc.p);
+      CC_LAUNCHED();
     }
     k_reduce_f64<<<1, 256, 0, s>>>(A.acc.p, A.nblk, A.out.p);
     CC_LAUNCHED();
     std::vector<float> lp(n3), lq(n3);
     double g[NPARAM];
-    CC_HIP(hipMemcpyAsync(lp.data(), A.lp[cur].p, n3 * sizeof(float), hipMemcpyDeviceToHost, s));
-    CC_HIP(hipMemcpyAsync(lq.data(), A.lq[cur].p, n3 * sizeof(float), hipMemcpyDeviceToHost, s));
+    CC_HIP(hipMemcpyAsync(lp.data(), A.lp.p, n3 * sizeof(float), hipMemcpyDeviceToHost, s));
+    CC_HIP(hipMemcpyAsync(lq.data(), A.lq.p, n3 * sizeof(float), hipMemcpyDeviceToHost, s));
     CC_HIP(hipMemcpyAsync(g, A.out.p, sizeof(g), hipMemcpyDeviceToHost, s));
     CC_HIP(hipStreamSynchronize(s));
     if (dl_dtheta) std::memcpy(dl_dtheta, g, sizeof(g));

@@ -131,17 +131,7 @@ __global__ __launch_bounds__(256) void k_collide_quad(BvhView bvh, const float* 
   if (e == 3) ins[i] = in ? 1 : 0;
 }
 
-// Which walk a launch of n vertices or points takes.  Four lanes per vertex
-// shorten a vertex's chain of dependent work (a quarter of the springs, a
-// visit of two loads instead of eight) but make four times the waves, each
-// about 40% of the one-lane kernel's instructions: the better form while
-// the quads' waves all fit on the chip beside each other (four per SIMD, 16
-// quads each: 256 CUs x 4 x 4 x 16).  Measured (us per step, one lane / four
-// lanes): in contact 11.7 / 8.6 at 4,096 vertices, 17.9 / 11.2 at 16,773
-// (24-wide rows), 21.3 / 16.5 at 65,536, 25.9 / 22.4 at 131,044, 53.6 / 60.1
-// at 262,144; falling 4.8 / 3.5 at 4,096, 6.5 / 6.4 at 65,536 and 8.3 / 9.8
-// at 131,044.
-constexpr uint32_t QUAD_MAX_N = 65536;
+// which walk a launch takes: see QUAD_MAX_N
 static bool by_quads(const BvhView& v, uint32_t n) { return n <= QUAD_MAX_N && (v.wide || v.m == 0); }
 
 void launch_collide_points(const BvhView& v, const float* pts, uint32_t n, int32_t* spill, int32_t* hit,
