@@ -68,8 +68,9 @@ struct Sim {
   DBuf<uint32_t> flag;
   // VBO
   uint32_t nf = 0;
-  DBuf<uint32_t> faces, vrow, vcol;
-  DBuf<float> face_n, vnormals;
+  DBuf<uint32_t> faces, vrow;
+  DBuf<uint32_t> vtri;      // [3 * 3 nf] corners of each vertex's faces, in vertex order (vrow)
+  DBuf<float> vnormals;
 
   // Graphs of graph_steps steps, per slot of the first frame and state
   // parity (captured when first needed).
