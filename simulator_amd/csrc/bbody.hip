@@ -60,7 +60,7 @@ __global__ __launch_bounds__(BB_BLOCK) void k_bb_boxes(const BodyDesc* __restric
   __shared__ float red[BB_BLOCK / 64][6];
   const uint4 b = blk[blockIdx.x];    // {body, first triangle, count, partial index}
   const BodyDesc d = desc[b.x];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+  const uint32_t tid = threadIdx.x;
   float mn[3], mx[3];
   box_sentinel(mn, mx);
   if (tid < b.z) {
@@ -70,18 +70,8 @@ __global__ __launch_bounds__(BB_BLOCK) void k_bb_boxes(const BodyDesc* __restric
     prim_box(ld3(V + 3 * (size_t)t[0]), ld3(V + 3 * (size_t)t[1]), ld3(V + 3 * (size_t)t[2]), d.depth, mn, mx);
     put6(boxes + 6 * i, mn, mx);
   }
-  for (int off = 32; off > 0; off >>= 1)
-    for (int c = 0; c < 3; ++c) {
-      mn[c] = fminf(mn[c], __shfl_xor(mn[c], off, 64));
-      mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], off, 64));
-    }
-  if (lane == 0) put6(red[w], mn, mx);
-  __syncthreads();
-  if (tid < 6) {
-    float v = red[0][tid];
-    for (int q = 1; q < BB_BLOCK / 64; ++q) v = tid < 3 ? fminf(v, red[q][tid]) : fmaxf(v, red[q][tid]);
-    partial[6 * (size_t)b.w + tid] = v;
-  }
+  const float v = block_box<BB_BLOCK / 64>(mn, mx, red);
+  if (tid < 6) partial[6 * (size_t)b.w + tid] = v;
 }
 
 // ------------------------------------------------------------ tree + boxes
@@ -104,60 +94,8 @@ __global__ __launch_bounds__(BB_BLOCK) void k_bb_boxes(const BodyDesc* __restric
 // it per workgroup, until one chunk holds the whole body.  The items of a
 // chunk partition its leaf range in order, and a node's range never cuts an
 // item, so one key per item decides whether it belongs to a range.
-constexpr int LV_C = 1024;
-constexpr int LV_LOG = 10;             // LV_C = 2^LV_LOG
 constexpr int LV_CAP = 128;
 constexpr int LV_G = LV_C / LV_CAP;
-static_assert(LV_C == 1 << LV_LOG, "LV_LOG");
-
-struct Box6 {
-  float v[6];
-};
-// LDS boxes are three 8-byte words
-__device__ inline Box6 lds_box(const float2 (*u)[3], int32_t i) {
-  const float2 a = u[i][0], b = u[i][1], c = u[i][2];
-  return Box6{{a.x, a.y, b.x, b.y, c.x, c.y}};
-}
-__device__ inline void lds_box_put(float2 (*u)[3], int32_t i, const Box6& b) {
-  u[i][0] = make_float2(b.v[0], b.v[1]);
-  u[i][1] = make_float2(b.v[2], b.v[3]);
-  u[i][2] = make_float2(b.v[4], b.v[5]);
-}
-__device__ inline Box6 box_or(const Box6& a, const Box6& b) {
-  Box6 r;
-  for (int c = 0; c < 3; ++c) {
-    r.v[c] = fminf(a.v[c], b.v[c]);
-    r.v[3 + c] = fmaxf(a.v[3 + c], b.v[3 + c]);
-  }
-  return r;
-}
-// the box of an internal node starts from the sentinel (cudaBRT.cu:166-206)
-__device__ inline Box6 box_node(const Box6& b) {
-  Box6 r;
-  for (int c = 0; c < 3; ++c) {
-    r.v[c] = fminf(100.0f, b.v[c]);
-    r.v[3 + c] = fmaxf(-100.0f, b.v[3 + c]);
-  }
-  return r;
-}
-
-// One round of the range boxes (see k_bb_level): u holds the boxes of the runs
-// of 2^Q items, v gets those of 2^(Q+1).
-template <int Q>
-__device__ inline void level_round(const float2 (*u)[3], float2 (*v)[3], bool have, int32_t k, int32_t n, int32_t l,
-                                   int32_t r, int32_t qa, int32_t qb, bool more, Box6& run, Box6& A, Box6& B) {
-  constexpr int32_t w = 1 << Q;
-  if (qa == Q) A = box_or(lds_box(u, l), lds_box(u, k - w + 1));
-  if (qb == Q) B = box_or(lds_box(u, k + 1), lds_box(u, r - w + 1));
-  if (!more) return;
-  if (have) {
-    // (a run past the chunk's end stays as it is: nothing reads it)
-    if (k + w < n) run = box_or(run, lds_box(u, k + w));
-    lds_box_put(v, k, run);
-  }
-  __syncthreads();
-}
-
 // One level of the build: one thread per item, and per split between two
 // items.  Boxes of ranges are unions of two overlapping power-of-two runs: in
 // round q the workgroup holds the box of every run of 2^q items in LDS (each

@@ -124,8 +124,9 @@ struct LvBlock {
   uint32_t write_leaves;
 };
 
+constexpr int LV_C = 1024;             // items of a workgroup of a build or refit level
 constexpr int BB_MAX_LEVELS = 8;       // 2^30 leaves: 2^20 -> 2^17 -> ... -> 4 -> 1 chunks
-constexpr uint32_t LV_MAX_LEAVES = 1u << 21;   // leaf indices of the bottom-up build carry 21 bits
+constexpr uint32_t LV_MAX_LEAVES = 1u << 21;   // leaves of a body built by levels
 
 // The bottom-up build (bbody.hip): work tables of its levels for the given
 // bodies (level 0: chunks of 1024 leaves, level L+1: 8 chunks of level L),
@@ -153,6 +154,18 @@ struct LvFrame {
 // nframes (1..MAX_FRAMES) frames of the same tables in each launch (grid.y)
 void launch_build_levels(const LvBlock* const* level, const uint32_t* n_level,
                          const LvFrame* frames, int nframes, hipStream_t s);
+
+// One level of a refit by levels (refit.hip): a fixed topology's items (leaves
+// at level 0, else nodes and leaves that the level below left), cut into
+// groups of at most LV_C; tables made once per topology.
+constexpr int RL_MAX = 8;
+struct RefitLevel {
+  uint32_t nitems = 0, nblk = 0;
+  DBuf<uint4> blk;         // group: {first item, items, first item it leaves to the next level, rounds}
+  DBuf<uint2> rec;         // [nitems] item k, and the split right of it (RL_*)
+  DBuf<uint4> wd;          // [nitems] four-wide entries {entry, link} of that split's children A, B
+  DBuf<uint32_t> node;     // [nitems] the split's node
+};
 
 // One frame of the body as the collision query reads it.
 struct Slot {
@@ -194,7 +207,8 @@ struct Lane {
   // written by every refit
   DBuf<float> top_child;            // [12 * max(m-1, 1)] boxes of the entries' non-top children
   DBuf<float> top_scratch;          // set-up work space and the top pass beyond its LDS size
-  // bottom-up build (rebuilt bodies): unfinished nodes between levels
+  DBuf<float> ritem[RL_MAX];        // refit by levels: [6 * items] boxes of each level's items
+  // build by levels: unfinished nodes between levels
   DBuf<BItem> items[2];
   DBuf<uint32_t> nitems[2];
 
@@ -219,9 +233,9 @@ struct Body {
   DBuf<uint32_t> tris;  // [3*m]
   DBuf<uint4> leaf_tri; // [m] sorted leaves of the shared topology (static and refitted bodies)
 
-  // A rebuilt body of 2..2^21 triangles builds its tree and boxes bottom-up
-  // (the batched build's level kernels) instead of the Karras searches, the
-  // refit description and the refit.
+  // A body of 2..2^21 triangles builds its tree and boxes by levels
+  // (launch_build_levels) instead of the Karras searches, the refit
+  // description and the refit; a refitted one is also refitted by levels.
   DBuf<BodyDesc> desc;              // [1] offsets 0
   SortTable sort_table;
   bool bottom_up = false;
@@ -248,6 +262,9 @@ struct Body {
   DBuf<int4> w_link;
   DBuf<uint2> w_dst;                // [2 * (m - 1)] binary child slot -> {wide entry (record * 4 +
                                     // entry), its link}, entry ~0 for the slots of folded nodes
+
+  RefitLevel rl[RL_MAX];            // a refitted body built by levels
+  int nrl = 0;
 
   int nslots = 1, nlanes = 1;
   // frames per chain of build launches (rebuilt bodies built bottom-up):
@@ -280,15 +297,15 @@ struct Body {
   // set-up: host arrays, vertices stride 3 (already extended); a moving
   // body gets `slots` frame slots and `lanes` update lanes, a rebuilt one
   // built bottom-up `chain` frames per chain of launches (allow_bottom_up
-  // false: a rebuilt body of any size takes the Karras searches and the
-  // refit, the path of bodies beyond the bottom-up build's leaf limit)
+  // false: a body of any size takes the Karras searches and the chunked
+  // refit, the path of bodies beyond the level build's leaf limit)
   void init(const float* verts3, uint32_t nv, const uint32_t* tris, uint32_t nf, uint32_t mode, float depth,
             const cc_capsules* caps, const MotionParams& mp, int slots, int lanes, hipStream_t s,
             int chain = 1, bool allow_bottom_up = true);
 
   // A static body whose vertices its owner replaces: from here on its tree
-  // is built and its wide records are folded on the device, as a rebuilt
-  // body's are (2 <= m <= 2^21; otherwise nothing changes).  The tree is the
+  // wide records are folded on the device after each build, as a rebuilt
+  // body's are (of 2..2^21 triangles; otherwise nothing changes).  The tree is the
   // same; the host layout of wide_setup (some 2 ms at 50,688 triangles: the
   // nodes copied to the host, laid out breadth-first and sorted, a dozen
   // buffers made) pays only for a body that stays, whose walk it makes 3%
@@ -320,9 +337,16 @@ struct Body {
   // (host, synchronous; keeps the binary form when the stack bound fails);
   // later refits write the boxes through w_dst.
   void wide_setup(int k, hipStream_t s);
+  // the layout itself, from the nodes' host copy: child slot -> {entry, link}
+  // into dst (empty: the binary form stays)
+  void wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s);
+  // the tables of a refit by levels
+  void refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s);
   // Rebuilt bodies: the wide records of slots ks[q] from their binary trees
   // (grid.y = frame; nothing when the binary walk is selected).
   void fold_frames(int F, const int* ks, hipStream_t s);
+  // A static body's host layout: its records' boxes from slot k's nodes.
+  void fold_static(int k, hipStream_t s);
 
   // host export in the reference encoding (lane 0 holds the keys and leaf
   // parents of slot k's tree)

@@ -27,23 +27,6 @@ __device__ inline void unite(float* mn, float* mx, const float* b6) {
   }
 }
 
-// Component threadIdx.x (0..5) of the block's box, in its first six threads:
-// lanes reduce by shuffles, waves through red.
-template <int WAVES>
-__device__ inline float block_box(float* mn, float* mx, float (&red)[WAVES][6]) {
-  for (int off = 32; off > 0; off >>= 1)
-    for (int c = 0; c < 3; ++c) {
-      mn[c] = fminf(mn[c], __shfl_xor(mn[c], off, 64));
-      mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], off, 64));
-    }
-  if ((threadIdx.x & 63u) == 0) put6(red[threadIdx.x >> 6], mn, mx);
-  __syncthreads();
-  const uint32_t c = threadIdx.x < 6 ? threadIdx.x : 0;
-  float v = red[0][c];
-  for (int w = 1; w < WAVES; ++w) v = c < 3 ? fminf(v, red[w][c]) : fmaxf(v, red[w][c]);
-  return v;
-}
-
 // A box of the four-wide form: entry d = {record * 4 + entry, link}, ~0 for
 // none.  An entry is one 32-byte sector {min xyz, max x | max yz, link, 0}
 // written whole by one thread (two 16-byte stores).
@@ -57,6 +40,88 @@ __device__ inline void put_wide_at(float4* wide, uint2 d, const float* b6) {
 __device__ inline void box_sentinel(float* mn, float* mx) {   // bbox.h:17-22
   mn[0] = mn[1] = mn[2] = 100.0f;
   mx[0] = mx[1] = mx[2] = -100.0f;
+}
+
+// ---- boxes of item ranges (k_bb_level, k_refit_level)
+struct Box6 {
+  float v[6];
+};
+// fminf / fmaxf as the one instruction they are.  The compiler first passes
+// every operand that it did not compute itself through a v_max with itself,
+// because a signalling NaN has to come out quiet: two more instructions per
+// union component of boxes read from LDS (level 0 of a refit: 666 -> 425 vector
+// instructions a wave).  Box components come out of prim_box's arithmetic,
+// which has quieted them.
+__device__ inline float vmin(float a, float b) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline float vmax(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// Component threadIdx.x (0..5) of the block's box, in its first six threads:
+// lanes reduce by shuffles, waves through red.
+template <int WAVES>
+__device__ inline float block_box(float* mn, float* mx, float (&red)[WAVES][6]) {
+  for (int off = 32; off > 0; off >>= 1)
+    for (int c = 0; c < 3; ++c) {
+      mn[c] = vmin(mn[c], __shfl_xor(mn[c], off, 64));
+      mx[c] = vmax(mx[c], __shfl_xor(mx[c], off, 64));
+    }
+  if ((threadIdx.x & 63u) == 0) put6(red[threadIdx.x >> 6], mn, mx);
+  __syncthreads();
+  const uint32_t c = threadIdx.x < 6 ? threadIdx.x : 0;
+  float v = red[0][c];
+  for (int w = 1; w < WAVES; ++w) v = c < 3 ? vmin(v, red[w][c]) : vmax(v, red[w][c]);
+  return v;
+}
+
+// LDS boxes are three 8-byte words
+__device__ inline Box6 lds_box(const float2 (*u)[3], int32_t i) {
+  const float2 a = u[i][0], b = u[i][1], c = u[i][2];
+  return Box6{{a.x, a.y, b.x, b.y, c.x, c.y}};
+}
+__device__ inline void lds_box_put(float2 (*u)[3], int32_t i, const Box6& b) {
+  u[i][0] = make_float2(b.v[0], b.v[1]);
+  u[i][1] = make_float2(b.v[2], b.v[3]);
+  u[i][2] = make_float2(b.v[4], b.v[5]);
+}
+__device__ inline Box6 box_or(const Box6& a, const Box6& b) {
+  Box6 r;
+  for (int c = 0; c < 3; ++c) {
+    r.v[c] = vmin(a.v[c], b.v[c]);
+    r.v[3 + c] = vmax(a.v[3 + c], b.v[3 + c]);
+  }
+  return r;
+}
+// the box of an internal node starts from the sentinel (cudaBRT.cu:166-206)
+__device__ inline Box6 box_node(const Box6& b) {
+  Box6 r;
+  for (int c = 0; c < 3; ++c) {
+    r.v[c] = vmin(100.0f, b.v[c]);
+    r.v[3 + c] = vmax(-100.0f, b.v[3 + c]);
+  }
+  return r;
+}
+
+// One round of the range boxes (see k_bb_level): u holds the boxes of the runs
+// of 2^Q items, v gets those of 2^(Q+1).
+template <int Q>
+__device__ inline void level_round(const float2 (*u)[3], float2 (*v)[3], bool have, int32_t k, int32_t n, int32_t l,
+                                   int32_t r, int32_t qa, int32_t qb, bool more, Box6& run, Box6& A, Box6& B) {
+  constexpr int32_t w = 1 << Q;
+  if (qa == Q) A = box_or(lds_box(u, l), lds_box(u, k - w + 1));
+  if (qb == Q) B = box_or(lds_box(u, k + 1), lds_box(u, r - w + 1));
+  if (!more) return;
+  if (have) {
+    // (a run past the chunk's end stays as it is: nothing reads it)
+    if (k + w < n) run = box_or(run, lds_box(u, k + w));
+    lds_box_put(v, k, run);
+  }
+  __syncthreads();
 }
 
 // capsule of vertex v: the last k with vstart[k] <= v

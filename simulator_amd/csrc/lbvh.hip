@@ -123,16 +123,21 @@ void Body::build_levels(int F, const int* ks, const int* ls, hipStream_t s) {
 void Lane::alloc(uint32_t m, bool full_lane, bool bottom_up, hipStream_t s) {
   full = full_lane;
   const size_t mi = std::max<uint32_t>(m, 2) - 1;
-  top_child.alloc(12 * mi);
-  top_scratch.alloc(Body::top_scratch_floats(m));
+  if (!bottom_up) {
+    top_child.alloc(12 * mi);
+    top_scratch.alloc(Body::top_scratch_floats(m));
+  }
   if (!full) return;
   nblk_box = grid_for(m, BOX_THREADS);
   boxes.alloc(6 * (size_t)m);
   partial.alloc(6 * (size_t)nblk_box);
   for (auto& b : kv) b.alloc(m);
   sort.alloc(sort_tiles(m), m > SORT_SUM_MAX ? 1 : 0);
-  if (bottom_up) alloc_levels(m, s);
   keys.alloc(m);
+  if (bottom_up) {
+    alloc_levels(m, s);
+    return;
+  }
   leaf_parent.alloc(m);
   leaf_parent.zero(s);
   top_list.alloc(mi);
@@ -179,16 +184,14 @@ void Body::level_setup(hipStream_t s) {
 }
 
 void Body::rebuild_on_device(hipStream_t s) {
-  if (mode != CC_BODY_STATIC || bottom_up || m < 2 || m > LV_MAX_LEAVES) return;
-  lane[0].alloc_levels(m, s);
-  level_setup(s);
+  if (mode != CC_BODY_STATIC || !bottom_up || grouped) return;
   slot[0].wide.alloc(8 * (size_t)(m - 1));
   w_src.release();
   w_link.release();
   w_dst.release();
   nwide = m - 1;
   wide_stack = STACK_LIMIT;
-  grouped = bottom_up = true;
+  grouped = true;
 }
 
 void Body::init(const float* v3, uint32_t nv_, const uint32_t* t3, uint32_t nf, uint32_t mode_, float depth_,
@@ -238,7 +241,7 @@ void Body::init(const float* v3, uint32_t nv_, const uint32_t* t3, uint32_t nf, 
     S.motion.alloc(12 + (size_t)ncaps);
     S.motion.zero(s);
   }
-  bottom_up = mode == CC_BODY_REBUILD && m >= 2 && m <= LV_MAX_LEAVES && allow_bottom_up;
+  bottom_up = m >= 2 && m <= LV_MAX_LEAVES && allow_bottom_up;
   BodyDesc d{};
   d.nv = nv;
   d.m = m;
@@ -296,9 +299,12 @@ void Body::build_frames(int F, const int* ks, const int* ls, hipStream_t s) {
   k_prim_boxes<<<dim3(nblk_box, (unsigned)F), BOX_THREADS, 0, s>>>(verts, tris.p, m, depth, boxes, partial);
   CC_LAUNCHED();
   launch_sort(desc.p, sort_table, tris.p, sf, F, s);
-  if (bottom_up) {                      // tree, parent links and boxes, bottom-up
+  if (bottom_up) {                      // tree and boxes by levels
     build_levels(F, ks, ls, s);
-    fold_frames(F, ks, s);
+    if (grouped)
+      fold_frames(F, ks, s);
+    else
+      wide_setup(ks[0], s);
     return;
   }
   const int k = ks[0], l = ls[0];

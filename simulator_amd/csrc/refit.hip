@@ -1,5 +1,10 @@
 // refit.hip -- bottom-up LBVH box refit on gfx950.
 //
+// A body built by levels is refitted by levels (k_refit_level, below): the
+// build's range boxes over tables of the fixed topology.  The chunked refit
+// that follows here is the path of bodies beyond 2^21 triangles and of a
+// single triangle.
+//
 // calculateBoudingBox (cudaBRT.cu:166-206) gives every internal node the box
 // sentinel U A U B, computed bottom-up by the second of its two children to
 // arrive.  Here the same boxes are computed level by level:
@@ -527,7 +532,198 @@ __global__ __launch_bounds__(TOP_REFIT_THREADS) void k_refit_top(PF<Node> nodes_
   }
 }
 
+// ======================================================== refit by levels
+// One level of a refitted body's boxes, by the range boxes of the level build
+// (k_bb_level): thread k holds item k of its group, and the split right of it,
+// whose children's ranges come from a table of the fixed topology.  A node's
+// children go straight to their four-wide entries (or, without `wide`, to the
+// binary node); boxes of nodes and items whose parent is not in the group go
+// to the next level's items.
+//
+// What bounds it: level 0 the bytes (40 read per leaf and 3 of vertices, 42
+// written) and the LDS rounds, two groups per CU; the levels above latency.
+// 501,120 triangles, three frames in a chain: 69 us at level 0 and 11 at each
+// of the two above, against 97-109 us of chunks (96 KB of LDS and 1024 threads
+// each, up to 21 height levels of which most lanes sit out, 76 bytes read per
+// leaf) and 30 us in one workgroup for the nodes across chunks.  One frame
+// alone: 36 against 50 us.  Groups of 512 and 256 items are quicker at level 0
+// (50 and 45 us), but add a level and take more of the chip from the step
+// beside them: 10.48 and 10.64 against 9.95 ms for 240 steps of 262,144
+// vertices.
+constexpr uint32_t RL_VALID = 1u << 31, RL_ROOT = 1u << 30, RL_NONE = 0xffffu;
+
+template <bool LEAVES>
+__global__ __launch_bounds__(LV_C) void k_refit_level(const uint4* __restrict__ blk, const uint2* __restrict__ rec,
+                                                      const uint4* __restrict__ wdst,
+                                                      const uint32_t* __restrict__ node_of, PF<const float> verts_f,
+                                                      const uint4* __restrict__ leaf_tri, float depth,
+                                                      PF<const float> in_f, PF<float> out_f, PF<Node> nodes_f,
+                                                      PF<float4> wide_f, PF<float> root_f) {
+  __shared__ float2 U[2][LV_C][3];
+  const uint4 b = blk[blockIdx.x];         // {first item, items, first output item, rounds}
+  const int32_t k = (int32_t)threadIdx.x, n = (int32_t)b.y;
+  const bool have = k < n;
+  const uint32_t at = b.x + (uint32_t)min(k, n - 1);
+  const uint2 r2 = rec[at];
+  float4* __restrict__ wide = pick(wide_f);
+  uint4 wd = make_uint4(~0u, 0u, ~0u, 0u);
+  if (wide) wd = wdst[at];
+  Box6 own;
+  if constexpr (LEAVES) {
+    const uint4 t = leaf_tri[at];
+    const float* __restrict__ verts = pick(verts_f);
+    prim_box(ld3(verts + 3 * (size_t)t.x), ld3(verts + 3 * (size_t)t.y), ld3(verts + 3 * (size_t)t.z), depth, own.v,
+             own.v + 3);
+  } else {
+    const float* src = pick(in_f) + 6 * (size_t)at;
+    for (int c = 0; c < 6; ++c) own.v[c] = src[c];
+  }
+  const bool node = have && (r2.x & RL_VALID);
+  const int32_t l = (int32_t)(r2.x & 1023u), r = (int32_t)((r2.x >> 10) & 1023u);
+  const int32_t qa = node ? 31 - __clz(k - l + 1) : -1, qb = node ? 31 - __clz(r - k) : -1;
+  if (have) lds_box_put(U[0], k, own);
+  __syncthreads();
+  Box6 run = own, A{}, B{};
+  const int32_t rounds = (int32_t)b.w;     // rounds 0 .. rounds - 1
+#define CC_ROUND(Q) \
+  if (rounds > Q) level_round<Q>(U[Q & 1], U[(Q & 1) ^ 1], have, k, n, l, r, qa, qb, rounds > Q + 1, run, A, B)
+  CC_ROUND(0); CC_ROUND(1); CC_ROUND(2); CC_ROUND(3); CC_ROUND(4);
+  CC_ROUND(5); CC_ROUND(6); CC_ROUND(7); CC_ROUND(8); CC_ROUND(9);
+#undef CC_ROUND
+  float* __restrict__ out = pick(out_f);
+  if (node) {
+    // a child of several items is a node (one of a single item is that item)
+    if (l < k) A = box_node(A);
+    if (k + 1 < r) B = box_node(B);
+    if (wide) {
+      put_wide_at(wide, make_uint2(wd.x, wd.y), A.v);
+      put_wide_at(wide, make_uint2(wd.z, wd.w), B.v);
+    } else {
+      float4* d = reinterpret_cast<float4*>(pick(nodes_f) + node_of[at]);
+      d[0] = make_float4(A.v[0], A.v[1], A.v[2], A.v[3]);
+      d[1] = make_float4(A.v[4], A.v[5], B.v[0], B.v[1]);
+      d[2] = make_float4(B.v[2], B.v[3], B.v[4], B.v[5]);
+    }
+    const uint32_t to = r2.y & 0xffffu;
+    if ((r2.x & RL_ROOT) || to != RL_NONE) {
+      const Box6 box = box_node(box_or(A, B));
+      float* d = (r2.x & RL_ROOT) ? pick(root_f) : out + 6 * (size_t)(b.z + to);
+      put6(d, box.v, box.v + 3);
+    }
+  }
+  if (have && (r2.y >> 16) != RL_NONE) put6(out + 6 * (size_t)(b.z + (r2.y >> 16)), own.v, own.v + 3);
+}
+
 // ======================================================== host side
+void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s) {
+  struct Item {
+    uint32_t first, last;
+    int32_t node;          // the item's node, -1 for a leaf
+  };
+  // by splits: the node of the split right of leaf i, its leaf range
+  const uint32_t mi = m - 1;
+  std::vector<uint32_t> node_at(mi), first(mi), last(mi);
+  std::vector<int32_t> parent(mi, -1);
+  for (uint32_t x = 0; x < mi; ++x) {
+    const Node& N = nd[x];
+    const uint32_t sp = (uint32_t)(N.childA < 0 ? ~N.childA : N.childA);
+    const uint32_t f = x == 0 ? 0 : std::min<uint32_t>(x, (uint32_t)N.other);
+    const uint32_t e = x == 0 ? m - 1 : std::max<uint32_t>(x, (uint32_t)N.other);
+    CC_REQUIRE(sp < mi && f <= sp && sp < e && e < m, "refit levels: bad node");
+    node_at[sp] = x;
+    first[x] = f;
+    last[x] = e;
+    for (const int32_t c : {N.childA, N.childB})
+      if (c >= 0) {
+        CC_REQUIRE((uint32_t)c < mi, "refit levels: bad link");
+        parent[c] = (int32_t)x;
+      }
+  }
+  std::vector<Item> items(m);
+  for (uint32_t i = 0; i < m; ++i) items[i] = {i, i, -1};
+  std::vector<uint32_t> at_first(m), at_last(m);   // item starting / ending at a leaf
+  for (nrl = 0; nrl < RL_MAX; ++nrl) {
+    RefitLevel& R = rl[nrl];
+    const uint32_t G = LV_C;
+    const uint32_t ni = (uint32_t)items.size();
+    std::vector<uint4> blk;
+    std::vector<uint2> rec(ni);
+    std::vector<uint4> wd(ni, make_uint4(~0u, 0u, ~0u, 0u));
+    std::vector<uint32_t> node(ni, 0u);
+    std::vector<Item> next;
+    for (uint32_t i0 = 0; i0 < ni; i0 += G) {
+      const uint32_t n = std::min<uint32_t>(G, ni - i0);
+      const uint32_t f0 = items[i0].first, l0 = items[i0 + n - 1].last, out0 = (uint32_t)next.size();
+      for (uint32_t k = 0; k < n; ++k) {
+        at_first[items[i0 + k].first] = k;
+        at_last[items[i0 + k].last] = k;
+      }
+      auto inside = [&](int32_t x) { return x >= 0 && first[x] >= f0 && last[x] <= l0; };
+      uint32_t rounds = 0;
+      for (uint32_t k = 0; k < n; ++k) {
+        rec[i0 + k] = make_uint2(0u, RL_NONE | (RL_NONE << 16));
+        if (k + 1 == n) continue;
+        const uint32_t x = node_at[items[i0 + k].last];
+        if (!inside((int32_t)x)) continue;
+        const uint32_t l = at_first[first[x]], r = at_last[last[x]];
+        rec[i0 + k].x = l | (r << 10) | RL_VALID | (x == 0 ? RL_ROOT : 0u);
+        node[i0 + k] = x;
+        if (!dst.empty()) {
+          const uint2 a = dst[2 * (size_t)x], b = dst[2 * (size_t)x + 1];
+          wd[i0 + k] = make_uint4(a.x, a.y, b.x, b.y);
+        }
+        for (uint32_t len = std::max(k - l + 1, r - k), q = 1; len; len >>= 1, ++q) rounds = std::max(rounds, q);
+      }
+      // what the group leaves, in leaf order: from each position the largest
+      // node of the group that starts there and was finished here, else the item
+      for (uint32_t k = 0; k < n;) {
+        // the topmost finished node over item k: climb from the item
+        const Item& it = items[i0 + k];
+        int32_t x = it.node, up = -1;
+        // the parent of a leaf or node with range [first, last]: the node whose
+        // split is at last, or at first - 1
+        if (x >= 0) {
+          up = parent[x];
+        } else {
+          const int32_t a = it.last < mi ? (int32_t)node_at[it.last] : -1;
+          const int32_t c = it.first > 0 ? (int32_t)node_at[it.first - 1] : -1;
+          up = (a >= 0 && nd[a].childA == ~(int32_t)it.first) ? a : c;
+        }
+        while (inside(up)) {
+          x = up;
+          up = parent[x];
+        }
+        if (x >= 0 && x != it.node) {          // a node finished here
+          const uint32_t sp = (uint32_t)(nd[x].childA < 0 ? ~nd[x].childA : nd[x].childA);
+          if (x != 0) {
+            rec[i0 + at_last[sp]].y = (rec[i0 + at_last[sp]].y & 0xffff0000u) | ((uint32_t)next.size() - out0);
+            next.push_back({first[x], last[x], x});
+          }
+          k = at_last[last[x]] + 1;
+        } else {                               // the item itself
+          rec[i0 + k].y = (rec[i0 + k].y & 0xffffu) | (((uint32_t)next.size() - out0) << 16);
+          next.push_back(it);
+          ++k;
+        }
+      }
+      blk.push_back(make_uint4(i0, n, out0, rounds));
+    }
+    R.nitems = ni;
+    R.nblk = (uint32_t)blk.size();
+    R.blk.upload(blk.data(), blk.size(), s);
+    R.rec.upload(rec.data(), ni, s);
+    R.wd.upload(wd.data(), ni, s);
+    R.node.upload(node.data(), ni, s);
+    CC_HIP(hipStreamSynchronize(s));           // the tables' host copies end here
+    if (nrl > 0)
+      for (int l = 0; l < nlanes * chain; ++l) lane[l].ritem[nrl].alloc(6 * (size_t)ni);
+    items.swap(next);
+    if (items.empty()) break;                  // the root was finished
+  }
+  CC_REQUIRE(items.empty(), "refit levels: too many levels");
+  ++nrl;
+}
+
 void Body::top_setup(int k, int l, hipStream_t s) {
   // top_count was zeroed by k_karras (no memset node in captured graphs)
   if (mode == CC_BODY_NONE || m < 2) return;
@@ -555,9 +751,10 @@ void Body::top_setup(int k, int l, hipStream_t s) {
 
 void Body::refit(int k, int l, hipStream_t s, bool binary) {
   if (mode == CC_BODY_NONE || m == 0) return;
-  if (bottom_up) {                      // same keys, so the same tree; new boxes
+  if (bottom_up && mode != CC_BODY_REFIT) {   // same keys, so the same tree; new boxes
     prim_boxes_of(k, l, s);
     build_levels(1, &k, &l, s);
+    if (!grouped) fold_static(k, s);
   } else {
     refit_frames(1, &k, &l, s, binary);
   }
@@ -565,7 +762,7 @@ void Body::refit(int k, int l, hipStream_t s, bool binary) {
 }
 
 void Body::refit_frames(int F, const int* ks, const int* ls, hipStream_t s, bool binary) {
-  CC_REQUIRE(F >= 1 && F <= MAX_FRAMES && !bottom_up, "body: frames per refit chain");
+  CC_REQUIRE(F >= 1 && F <= MAX_FRAMES, "body: frames per refit chain");
   // every frame of a chain shares the topology (that of lane 0 for a
   // refitted body, of lane ls[0] for a rebuilt one refitted in place)
   Lane& T = topo(ls[0]);
@@ -589,6 +786,22 @@ void Body::refit_frames(int F, const int* ks, const int* ls, hipStream_t s, bool
     leaf0.p[f] = S.leaf0_box.p;
     scratch.p[f] = L.top_scratch.p;
     wide.p[f] = W ? S.wide.p : nullptr;
+  }
+  if (nrl) {
+    for (int L = 0; L < nrl; ++L) {
+      const RefitLevel& R = rl[L];
+      PF<const float> in{};
+      PF<float> out{};
+      for (int f = 0; f < F; ++f) {
+        in.p[f] = L > 0 ? lane[ls[f]].ritem[L].p : nullptr;
+        out.p[f] = L + 1 < nrl ? lane[ls[f]].ritem[L + 1].p : nullptr;
+      }
+      auto kern = L == 0 ? k_refit_level<true> : k_refit_level<false>;
+      kern<<<dim3(R.nblk, (unsigned)F), LV_C, 0, s>>>(R.blk.p, R.rec.p, R.wd.p, R.node.p, verts, leaf_tri.p, depth, in,
+                                                      out, nodes, wide, root);
+      CC_LAUNCHED();
+    }
+    return;
   }
   k_refit_chunks<<<dim3(grid_for(m, RC_CHUNK), (unsigned)F), RC_THREADS, 0, s>>>(
       verts, leaf_tri_of(ks[0]), T.leaf_parent.p, T.links.p, nodes, m, depth, T.nflag.p, T.lflag.p, T.chunk_h.p,

@@ -107,6 +107,12 @@ __global__ __launch_bounds__(256) void k_fold_grouped(PF<const Node> nodes_f, ui
   o[1] = o1;
 }
 
+void Body::fold_static(int k, hipStream_t s) {
+  if (!nwide || !wide_enabled) return;
+  k_fold_wide<<<grid_for(nwide, 256), 256, 0, s>>>(slot[k].nodes.p, w_src.p, w_link.p, nwide, slot[k].wide.p);
+  CC_LAUNCHED();
+}
+
 void Body::fold_frames(int F, const int* ks, hipStream_t s) {
   if (!grouped || !wide_enabled) return;
   PF<const Node> nodes{};
@@ -123,10 +129,16 @@ void Body::wide_setup(int k, hipStream_t s) {
   nwide = 0;
   wide_stack = 0;
   if (mode == CC_BODY_NONE || mode == CC_BODY_REBUILD || m < 2) return;
-  const uint32_t mi = m - 1;
-  std::vector<Node> nd(mi);
-  CC_HIP(hipMemcpyAsync(nd.data(), slot[k].nodes.p, mi * sizeof(Node), hipMemcpyDeviceToHost, s));
+  std::vector<Node> nd(m - 1);
+  CC_HIP(hipMemcpyAsync(nd.data(), slot[k].nodes.p, nd.size() * sizeof(Node), hipMemcpyDeviceToHost, s));
   CC_HIP(hipStreamSynchronize(s));
+  std::vector<uint2> dst;
+  wide_layout(k, nd, dst, s);
+  if (mode == CC_BODY_REFIT && bottom_up) refit_setup(nd, dst, s);
+}
+
+void Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s) {
+  const uint32_t mi = m - 1;
   // Breadth-first over the kept binary nodes (the root, then the internal
   // entries of each kept node); wid maps a kept binary node to its record.
   std::vector<int32_t> wid(mi, -1), order;
@@ -239,7 +251,7 @@ void Body::wide_setup(int k, hipStream_t s) {
     src.swap(src2);
     link.swap(link2);
   }
-  std::vector<uint2> dst(2 * (size_t)mi, make_uint2(~0u, 0u));
+  dst.assign(2 * (size_t)mi, make_uint2(~0u, 0u));
   for (size_t w = 0; w < src.size(); ++w) {
     const uint32_t* e = &src[w].x;
     const int32_t* lk = &link[w].x;
