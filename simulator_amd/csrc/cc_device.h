@@ -200,100 +200,91 @@ __device__ inline int32_t wstk_get(const Spill& sp, int k) {
 }
 
 // One visit of a wide record q[0..7] (entry e is q[2e], q[2e + 1]) takes
-// the first entry whose box holds p: a leaf is the hit (returned, >= 0), an
-// internal entry the next record (WIDE_NEXT, in `node`); with none, the
-// walk pops (a deferred leaf is the hit) or misses (WIDE_MISS).  The later
-// candidates of a visit (at most three) are deferred with three
+// the first entry whose box holds p: a leaf is the hit, an internal entry the
+// next record; with none, the walk pops (a deferred leaf is the hit) or misses.
+// The later candidates of a visit (at most three) are deferred with three
 // unconditional stores at the stack top, highest entry first, and the stack
 // pointer then moves by their number: a slot above the new top holds
-// nothing the walk reads.  This takes far fewer instructions than shifting
-// a register stack entry by entry, which matters because all four waves of
-// a SIMD walk at once.
-enum : int { WIDE_NEXT = -1, WIDE_MISS = -2 };
-template <bool GROUPED>
-__device__ inline int32_t wide_visit(f3 p, float4 q0, float4 q1, float4 q2, float4 q3, float4 q4, float4 q5,
-                                     float4 q6, float4 q7, const Spill& spill, int& sp, int32_t& node,
-                                     int limit) {
-  // Kept as booleans (lane masks): the first candidate and the deferred set
-  // follow from them by selects, with no per-lane bit mask to build.
-  const bool i0 = in_box(p, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y), i1 = in_box(p, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y);
-  bool i2 = in_box(p, q4.x, q4.y, q4.z, q4.w, q5.x, q5.y), i3 = in_box(p, q6.x, q6.y, q6.z, q6.w, q7.x, q7.y);
-  const int32_t c0 = __float_as_int(q1.z), c1 = __float_as_int(q3.z), c3 = __float_as_int(q7.z);
-  int32_t c2 = __float_as_int(q5.z);
-  if constexpr (GROUPED) {
-    // A split record whose first candidate is in entries 0-1: entries 2-3
-    // become one candidate, the record of their parent (the split word;
-    // the root is no node's child, so a split is never 0) when both hold
-    // p, else the one that does (the same next step as that record's
-    // visit, one visit fewer).
-    const int32_t split = __float_as_int(q1.w);
-    const bool in_a = (split != 0) & (i0 | i1);
-    const int32_t b_next = (i2 & i3) ? split : (i2 ? c2 : c3);
-    c2 = in_a ? b_next : c2;
-    i2 = in_a ? (i2 | i3) : i2;
-    i3 = i3 & !in_a;
-  }
-  if (!(i0 | i1 | i2 | i3)) {
-    if (sp == 0) return WIDE_MISS;
-    --sp;
-    node = wstk_get(spill, sp);
-    return node < 0 ? ~node : WIDE_NEXT;
-  }
-  // the first candidate's link
-  const int32_t c = i0 ? c0 : (i1 ? c1 : (i2 ? c2 : c3));
-  if (c < 0) return ~c;
-  // the later candidates (a candidate with one before it), popped lowest
-  // entry first
-  const bool r1 = i1 & i0, r2 = i2 & (i0 | i1), r3 = i3 & (i0 | i1 | i2);
-  const int32_t x0 = r3 ? c3 : (r2 ? c2 : c1);
-  const int32_t x1 = r3 ? (r2 ? c2 : c1) : c1;
-  const int k = (int)r1 + (int)r2 + (int)r3;
-  if (sp + k > limit) {                 // unreachable at the default limit (both layouts
-    trav_fault(spill, TRAV_OVERFLOW);   // bound the deferrals by 64)
-    return WIDE_MISS;
-  }
-  if (sp + 3 <= WSTK_LDS) {
-    int32_t* t = spill.lds + sp * WSTK_LANES;
-    t[0] = x0;
-    t[WSTK_LANES] = x1;
-    t[2 * WSTK_LANES] = c1;
-  } else {
-    if (k > 0) wstk_put(spill, sp, x0);
-    if (k > 1) wstk_put(spill, sp + 1, x1);
-    if (k > 2) wstk_put(spill, sp + 2, c1);
-  }
-  sp += k;
-  node = c;
-  return WIDE_NEXT;
-}
-
-// GROUPED: a rebuilt body's records (split words); the walk of static and
-// refitted bodies is compiled without them.
+// nothing the walk reads.  The top of the stack is read while the next record
+// arrives, and the loop has one way out: a walk at four waves per SIMD is bound
+// by its instructions as much as by its loads (90,000 vertices 25.8 -> 23.6 us
+// per step, 262,144 36.5 -> 35.3, with the springs' branches gone from 126 to 88
+// VGPRs).
 template <bool GROUPED>
 __device__ inline int32_t wide_first_hit(const BvhView& b, f3 p, uint32_t& visits, Spill spill, const WideRoot& rt) {
-  int sp = 0;
-  int32_t node = 0;
   const int limit = stack_limit(spill);
+  int sp = 0, k;
+  int32_t c, top = 0;
+  bool any;
+  float4 q0 = rt.q[0], q1 = rt.q[1], q2 = rt.q[2], q3 = rt.q[3], q4 = rt.q[4], q5 = rt.q[5], q6 = rt.q[6],
+         q7 = rt.q[7];
   ++visits;
-  int32_t r = wide_visit<GROUPED>(p, rt.q[0], rt.q[1], rt.q[2], rt.q[3], rt.q[4], rt.q[5], rt.q[6], rt.q[7], spill, sp, node,
-                         limit);
-  uint32_t guard = 0;
-  for (; r == WIDE_NEXT && guard < b.m; ++guard) {
+  for (uint32_t guard = 0;; ++guard) {
+    // Kept as booleans (lane masks): the first candidate and the deferred set
+    // follow from them by selects, with no per-lane bit mask to build.
+    const bool i0 = in_box(p, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y), i1 = in_box(p, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y);
+    bool i2 = in_box(p, q4.x, q4.y, q4.z, q4.w, q5.x, q5.y), i3 = in_box(p, q6.x, q6.y, q6.z, q6.w, q7.x, q7.y);
+    const int32_t c0 = __float_as_int(q1.z), c1 = __float_as_int(q3.z), c3 = __float_as_int(q7.z);
+    int32_t c2 = __float_as_int(q5.z);
+    if constexpr (GROUPED) {
+      // A split record whose first candidate is in entries 0-1: entries 2-3
+      // become one candidate, the record of their parent (the split word;
+      // the root is no node's child, so a split is never 0) when both hold
+      // p, else the one that does (the same next step as that record's
+      // visit, one visit fewer).
+      const int32_t split = __float_as_int(q1.w);
+      const bool in_a = (split != 0) & (i0 | i1);
+      const int32_t b_next = (i2 & i3) ? split : (i2 ? c2 : c3);
+      c2 = in_a ? b_next : c2;
+      i2 = in_a ? (i2 | i3) : i2;
+      i3 = i3 & !in_a;
+    }
+    any = i0 | i1 | i2 | i3;
+    // the first candidate's link
+    c = i0 ? c0 : (i1 ? c1 : (i2 ? c2 : (i3 ? c3 : top)));
+    // the later candidates (a candidate with one before it), popped lowest
+    // entry first
+    const bool r1 = i1 & i0, r2 = i2 & (i0 | i1), r3 = i3 & (i0 | i1 | i2);
+    const int32_t x0 = r3 ? c3 : (r2 ? c2 : c1);
+    const int32_t x1 = r3 ? (r2 ? c2 : c1) : c1;
+    k = (int)r1 + (int)r2 + (int)r3;
+    // a miss; a leaf; more entries than the limit (both layouts bound the
+    // deferrals by 64, the default); the bound of a corrupted tree
+    if ((!any & (sp == 0)) | (c < 0) | (sp + k > limit) | (guard >= b.m)) break;
     // a 32-bit byte offset (records < 4 GiB): the loads take the base in
     // scalar registers
-    const float4* nd = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(b.wide) +
-                                                       ((uint32_t)node << 7));
-    const float4 q0 = nd[0], q1 = nd[1], q2 = nd[2], q3 = nd[3], q4 = nd[4], q5 = nd[5], q6 = nd[6],
-                 q7 = nd[7];
+    const float4* nd = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(b.wide) + ((uint32_t)c << 7));
+    q0 = nd[0]; q1 = nd[1]; q2 = nd[2]; q3 = nd[3]; q4 = nd[4]; q5 = nd[5]; q6 = nd[6]; q7 = nd[7];
+    const int at = any ? sp : sp - 1;
+    sp = at + k;
+    if (at + 3 <= WSTK_LDS) {
+      int32_t* t = spill.lds + at * WSTK_LANES;
+      t[0] = x0;
+      t[WSTK_LANES] = x1;
+      t[2 * WSTK_LANES] = c1;
+      top = spill.lds[max(sp - 1, 0) * WSTK_LANES];
+    } else {
+      if (k > 0) wstk_put(spill, at, x0);
+      if (k > 1) wstk_put(spill, at + 1, x1);
+      if (k > 2) wstk_put(spill, at + 2, c1);
+      top = wstk_get(spill, sp - 1);
+      // waited for here: a load left pending on this path makes the other one
+      // wait for its record before it touches the stack
+      asm volatile("" : "+v"(top));
+    }
     // All four links arrive with the boxes: otherwise the compiler loads
     // entry 0's link apart, inside the branch that reads it, one more
     // memory round trip per descending visit.
     asm volatile("" ::"v"(q1.z), "v"(q3.z), "v"(q5.z), "v"(q7.z));
+    // and the unread last words keep their registers until then: taken for the
+    // stack's values, they make it wait for the record
+    if constexpr (GROUPED) asm volatile("" ::"v"(q1.w), "v"(q3.w), "v"(q5.w), "v"(q7.w));
     ++visits;
-    r = wide_visit<GROUPED>(p, q0, q1, q2, q3, q4, q5, q6, q7, spill, sp, node, limit);
   }
-  if (r == WIDE_NEXT) trav_fault(spill, TRAV_BOUND);
-  return r >= 0 ? r : -1;
+  if (!any && sp == 0) return -1;
+  if (c < 0) return ~c;
+  trav_fault(spill, sp + k > limit ? TRAV_OVERFLOW : TRAV_BOUND);
+  return -1;
 }
 
 // ---- the four-wide walk by quads
@@ -333,14 +324,17 @@ __device__ inline int32_t qstk_get(const Spill& sp, int k) {
   return v;
 }
 
-// One visit: lane e holds entry e = {a, b} of the record.  Every lane of the
-// quad returns the same (see wide_visit).
+// Which entries of a record are candidates (bit e: entry e; the same in every
+// lane), lane e holding entry e = {a, b}, and the lane's link (see wide_first_hit).
 template <bool GROUPED>
-__device__ inline int32_t quad_visit(f3 p, int e, float4 a, float4 b, const Spill& spill, int& sp, int32_t& node,
-                                     int limit) {
-  const bool in = in_box(p, a.x, a.y, a.z, a.w, b.x, b.y);
-  int32_t link = __float_as_int(b.z);
-  int32_t m = quad_or(in ? 1 << e : 0);
+__device__ inline int32_t quad_candidates(f3 p, int e, float4 a, float4 b, int32_t& link) {
+  // in_box as lane masks: six compares and five scalar ands (the compiler turns
+  // the booleans into words of bits otherwise)
+  const uint64_t in = __ballot(p.x >= a.x) & __ballot(p.y >= a.y) & __ballot(p.z >= a.z) & __ballot(p.x <= a.w) &
+                      __ballot(p.y <= b.x) & __ballot(p.z <= b.y);
+  link = __float_as_int(b.z);
+  const int lane = (int)(threadIdx.x & 63u);
+  int32_t m = (int32_t)(((lane & 32) ? (uint32_t)(in >> 32) : (uint32_t)in) >> (lane & 28)) & 15;
   if constexpr (GROUPED) {
     // a split record whose first candidate is in entries 0-1: entries 2-3,
     // when both hold p, become one candidate, their parent's record
@@ -349,25 +343,7 @@ __device__ inline int32_t quad_visit(f3 p, int e, float4 a, float4 b, const Spil
     link = (fold && e == 2) ? split : link;
     m = fold ? m & 7 : m;
   }
-  if (m == 0) {
-    if (sp == 0) return WIDE_MISS;
-    --sp;
-    node = qstk_get(spill, sp);
-    return node < 0 ? ~node : WIDE_NEXT;
-  }
-  const int f = __builtin_ctz(m);
-  const int32_t c = quad_or(e == f ? link : 0);
-  if (c < 0) return ~c;
-  const int k = __builtin_popcount(m) - 1;
-  if (sp + k > limit) {
-    trav_fault(spill, TRAV_OVERFLOW);
-    return WIDE_MISS;
-  }
-  // the later candidates, the lowest entry on top
-  if (e > f && ((m >> e) & 1)) qstk_put(spill, sp + __builtin_popcount(m >> (e + 1)), link);
-  sp += k;
-  node = c;
-  return WIDE_NEXT;
+  return m;
 }
 
 // Lane e's entry of the root record, loaded by the caller with its other
@@ -380,27 +356,101 @@ __device__ inline QuadRoot load_quad_root(const BvhView& b, int e) {
   return QuadRoot{make_float4(0.0f, 0.0f, 0.0f, 0.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f)};
 }
 
+__device__ inline QuadRoot load_quad_rec(const BvhView& b, int32_t node, int e) {
+  // a 32-bit byte offset (records < 4 GiB), as in wide_first_hit
+  const float4* nd = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(b.wide) +
+                                                     (((uint32_t)node << 7) + ((uint32_t)e << 5)));
+  return QuadRoot{nd[0], nd[1]};
+}
+
 // The first hit of p (the same in every lane of the quad; likewise the
 // result) through the four-wide form of a body of at least two triangles.
-template <bool GROUPED>
+// AHEAD: a round visits the two first nodes of the walk's frontier; the
+// second's candidates take its place behind the first's, so a first hit is the
+// same, and a walk that finds no hit in the first subtree is already one
+// record into the second.  What bounds these launches is the longest walk of
+// the chip, one memory round trip and about 130 instructions after another: 16
+// rounds become 10 at the 5,120-triangle body, 21 become 13 at the
+// 50,688-triangle one (us per pipelined step: 8.7 -> 8.1 for 4,096 vertices,
+// 26.7 -> 24.7 for 12,321; 8.1 -> 7.7 and 24.7 -> 23.1 more by one way out of
+// the loop and no branch around the stack's stores).  One lane per vertex does
+// not take it (262,144 vertices: 35.3 -> 39.9 us, two records being loaded
+// where the loads are what is short).
+// A look-ahead leaves at most AHEAD_SP + 7 entries, and a plain walk from
+// there adds the 64 of its own bound at most.
+constexpr int AHEAD_SP = 5;
+static_assert(64 + AHEAD_SP + 7 <= WSTK_LDS + STACK_SPILL, "look-ahead stack exceeds LDS and spill area");
+template <bool GROUPED, bool AHEAD>
 __device__ inline int32_t quad_first_hit(const BvhView& b, f3 p, int e, uint32_t& visits, Spill spill,
                                          const QuadRoot& rt) {
-  int sp = 0;
-  int32_t node = 0;
-  const int limit = stack_limit(spill);
-  ++visits;
-  int32_t r = quad_visit<GROUPED>(p, e, rt.a, rt.b, spill, sp, node, limit);
-  uint32_t guard = 0;
-  for (; r == WIDE_NEXT && guard < b.m; ++guard) {
-    const float4* nd = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(b.wide) +
-                                                       (((uint32_t)node << 7) + ((uint32_t)e << 5)));
-    const float4 qa = nd[0], qb = nd[1];
-    asm volatile("" ::"v"(qb.z), "v"(qb.w));
-    ++visits;
-    r = quad_visit<GROUPED>(p, e, qa, qb, spill, sp, node, limit);
+  // a lowered stack limit is a plain walk's
+  int cap = stack_limit(spill), ahead = -1;
+  if (AHEAD && cap == STACK_LIMIT) {
+    cap += AHEAD_SP + 7;
+    ahead = AHEAD_SP;
   }
-  if (r == WIDE_NEXT) trav_fault(spill, TRAV_BOUND);
-  return r >= 0 ? r : -1;
+  int sp = 0, left, kept, add;
+  int32_t l0, l1 = 0, t0 = 0, t1 = 0;          // links of the two records, top entries of the stack
+  int32_t c0, m = quad_candidates<GROUPED>(p, e, rt.a, rt.b, l0);
+  ++visits;
+  for (uint32_t guard = 0;; ++guard) {
+    // the candidates in order: bits 0-3 of m the first record's entries, 4-7
+    // the second's, then the stack
+    left = __builtin_popcount(m) + sp;
+    const int f0 = __builtin_ctz(m | 0x100);
+    const int32_t s0 = quad_or(e == (f0 & 3) ? (f0 < 4 ? l0 : l1) : 0);
+    c0 = m ? s0 : t0;
+    int32_t rest = m & (m - 1);                 // without the first (0 of none)
+    kept = m ? sp : sp - 1;
+    int32_t c1 = 0;
+    bool take = false;
+    if constexpr (AHEAD) {
+      const int f1 = __builtin_ctz(rest | 0x100);
+      const int32_t s1 = quad_or(e == (f1 & 3) ? (f1 < 4 ? l0 : l1) : 0);
+      c1 = rest ? s1 : (m ? t0 : t1);
+      take = (left >= 2) & (c1 >= 0) & (left - 2 <= ahead);
+      kept = (take & (rest == 0)) ? kept - 1 : kept;
+      rest = take ? rest & (rest - 1) : rest;
+    }
+    add = __builtin_popcount(rest);
+    // one way out of the loop
+    if ((left == 0) | (c0 < 0) | (kept + add > cap) | (guard >= b.m)) break;
+    sp = kept + add;
+    const QuadRoot r0 = load_quad_rec(b, c0, e);
+    QuadRoot r1;
+    if constexpr (AHEAD) r1 = load_quad_rec(b, take ? c1 : c0, e);
+    // the later candidates, the lowest on top; the stack's top entries for the
+    // next round arrive while the records do
+    const bool put0 = (rest >> e) & 1, put1 = AHEAD && ((rest >> (e + 4)) & 1);
+    const int at0 = kept + __builtin_popcount(rest >> (e + 1)), at1 = kept + __builtin_popcount(rest >> (e + 5));
+    if (sp <= WSTK_LDS) {
+      // no branch: a lane with nothing to defer writes the row past the stack
+      spill.lds[(put0 ? at0 : WSTK_LDS) * QSTK_QUADS] = l0;
+      if constexpr (AHEAD) spill.lds[(put1 ? at1 : WSTK_LDS) * QSTK_QUADS] = l1;
+      t0 = spill.lds[max(sp - 1, 0) * QSTK_QUADS];
+      if constexpr (AHEAD) t1 = spill.lds[max(sp - 2, 0) * QSTK_QUADS];
+    } else {
+      if (put0) qstk_put(spill, at0, l0);
+      if (put1) qstk_put(spill, at1, l1);
+      t0 = qstk_get(spill, sp - 1);
+      if constexpr (AHEAD) t1 = qstk_get(spill, sp - 2);
+      // waited for here: a load left pending on this path makes the other one
+      // wait for its records before it touches the stack
+      asm volatile("" : "+v"(t0), "+v"(t1));
+    }
+    asm volatile("" ::"v"(r0.b.z), "v"(r0.b.w));
+    ++visits;
+    m = quad_candidates<GROUPED>(p, e, r0.a, r0.b, l0);
+    if constexpr (AHEAD) {
+      asm volatile("" ::"v"(r1.b.z), "v"(r1.b.w));
+      const int32_t m1 = quad_candidates<GROUPED>(p, e, r1.a, r1.b, l1);
+      m |= take ? m1 << 4 : 0;
+    }
+  }
+  if (left == 0) return -1;
+  if (c0 < 0) return ~c0;
+  trav_fault(spill, kept + add > cap ? TRAV_OVERFLOW : TRAV_BOUND);
+  return -1;
 }
 
 // First-hit traversal (D_BVH::intersect, cudaBRT.cu:239-285): one node
@@ -473,10 +523,13 @@ __device__ inline bool collide_project(const BvhView& b, f3& p, f3& n_out, int32
 
 // The same by the four lanes of a quad (lane e; p and every result are the
 // same in all four).  The view has no body, or its four-wide form.
+template <bool AHEAD>
 __device__ inline bool collide_project_quad(const BvhView& b, f3& p, f3& n_out, int32_t& hit, uint32_t& visits,
                                             int e, Spill spill, const QuadRoot& rt) {
   hit = -1;
-  if (b.m) hit = b.grouped ? quad_first_hit<true>(b, p, e, visits, spill, rt) : quad_first_hit<false>(b, p, e, visits, spill, rt);
+  if (b.m)
+    hit = b.grouped ? quad_first_hit<true, AHEAD>(b, p, e, visits, spill, rt)
+                    : quad_first_hit<false, AHEAD>(b, p, e, visits, spill, rt);
   return project_hit(b, hit, p, n_out);
 }
 

@@ -23,15 +23,16 @@ constexpr int ELL_W2 = 24;
 constexpr uint32_t PAD_TYPE = 3u << 30;
 // Launches of up to this many vertices or points take four lanes each.  Four lanes per vertex
 // shorten a vertex's chain of dependent work (a quarter of the springs, a
-// visit of two loads instead of eight) but make four times the waves, each
-// about 40% of the one-lane kernel's instructions: the better form while
-// the quads' waves all fit on the chip beside each other (four per SIMD, 16
-// quads each: 256 CUs x 4 x 4 x 16).  Measured (us per step, one lane / four
-// lanes): in contact 11.7 / 8.6 at 4,096 vertices, 17.9 / 11.2 at 16,773
-// (24-wide rows), 21.3 / 16.5 at 65,536, 25.9 / 22.4 at 131,044, 53.6 / 60.1
-// at 262,144; falling 4.8 / 3.5 at 4,096, 6.5 / 6.4 at 65,536 and 8.3 / 9.8
-// at 131,044.
-constexpr uint32_t QUAD_MAX_N = 65536;
+// round of four loads for two records instead of eight for one) but make four
+// times the waves, each about 40% of the one-lane kernel's instructions: the
+// better form while most of the quads' waves fit on the chip beside each other
+// (seven per SIMD, 16 quads each: 256 CUs x 4 x 7 x 16 = 114,688).  Measured
+// (us of the step alone, one lane / four lanes): in contact 11.7 / 8.6 at 4,096
+// vertices, 21.6 / 15.9 at 32,761, 23.8 / 18.5 at 65,536, 23.9 / 20.4 at 90,000,
+// 28.3 / 25.5 at 131,044, 35.0 / 40.3 at 262,144; falling 8.9 / 8.6 at 65,536, 9.8 /
+// 10.8 at 90,000 (pipelined steps 11.8 / 11.2), 9.8 / 11.9 at 131,044 (13.1 /
+// 13.4).
+constexpr uint32_t QUAD_MAX_N = 98304;
 
 struct StepArgs {
   float inv_dt, dt2, inv_mass;

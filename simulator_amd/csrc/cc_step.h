@@ -38,7 +38,12 @@ __device__ inline SpringTerm spring_scale(f3 p, f3 vel, const NState& g, uint2 r
   const float rinv = rsqrtf(L2);
   const float L = L2 * rinv;
   const float vd = fmaf(dV.z, dP.z, fmaf(dV.y, dP.y, dV.x * dP.x));
-  const float sc = real ? fmaf(-ks, L - rest, a.kd * vd * rinv) * rinv : 0.0f;
+  // +0 for an empty slot by a mask the compiler cannot see through: from a select
+  // it makes a branch around the term and moves a part of the gather into it,
+  // one more memory round trip per vertex
+  uint32_t keep = real ? ~0u : 0u;
+  asm("" : "+v"(keep));
+  const float sc = __uint_as_float(__float_as_uint(fmaf(-ks, L - rest, a.kd * vd * rinv) * rinv) & keep);
   return SpringTerm{dP, sc};
 }
 
@@ -181,10 +186,18 @@ template <int K, int NB>
 __device__ inline void quad_add(const SpringTerm (&t)[NB], f3& S) {
 #pragma unroll
   for (int k = 0; k < NB; ++k) {
-    const float sc = quad_bcast<K>(t[k].sc);
-    S.x = fmaf(quad_bcast<K>(t[k].dP.x), sc, S.x);
-    S.y = fmaf(quad_bcast<K>(t[k].dP.y), sc, S.y);
-    S.z = fmaf(quad_bcast<K>(t[k].dP.z), sc, S.z);
+    // fmaf(dP, sc, S) with lane K's dP read by the multiply-add itself (the
+    // compiler takes a move for each).  A register is read across lanes two
+    // cycles after the vector unit wrote it at the earliest, which the compiler
+    // does not see to inside an asm block: the wait is part of it.
+    float sc;
+#define CC_LANE " quad_perm:[%c8,%c8,%c8,%c8] row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t"
+        "v_mov_b32_dpp %0, %4" CC_LANE "v_fmac_f32_dpp %1, %5, %0" CC_LANE "v_fmac_f32_dpp %2, %6, %0" CC_LANE
+        "v_fmac_f32_dpp %3, %7, %0" CC_LANE
+        : "=&v"(sc), "+v"(S.x), "+v"(S.y), "+v"(S.z)
+        : "v"(t[k].sc), "v"(t[k].dP.x), "v"(t[k].dP.y), "v"(t[k].dP.z), "n"(K));
+#undef CC_LANE
   }
 }
 
@@ -192,7 +205,7 @@ __device__ inline void quad_add(const SpringTerm (&t)[NB], f3& S) {
 // through its four-wide form.  Lane e takes a quarter of the springs; the
 // terms are then added in row order in every lane, so the sums, and with
 // them every result, equal step_vertex's bit for bit.
-template <bool DEBUG, int EW>
+template <bool DEBUG, int EW, bool AHEAD>
 __device__ inline void step_vertex_quad(uint32_t i, int e, const float* __restrict__ sin_, float* __restrict__ sout,
                                         const float* contact_in, float* contact_out, const uint32_t* __restrict__ row,
                                         const uint2* __restrict__ rec, const StepArgs& a, const BvhView& bvh,
@@ -255,7 +268,7 @@ __device__ inline void step_vertex_quad(uint32_t i, int e, const float* __restri
     } while (!ELL);
     np = verlet_update(p, q, c, F + S, a);
     if (DEBUG && e == 0) st3(dbg_pre + 3 * (size_t)i, np);
-    inside = collide_project_quad(bvh, np, nc, hit, visits, e, spill, root);
+    inside = collide_project_quad<AHEAD>(bvh, np, nc, hit, visits, e, spill, root);
     if (inside) nq = np;
   } else if (DEBUG && e == 0) {
     st3(dbg_pre + 3 * (size_t)i, np);

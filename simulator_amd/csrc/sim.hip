@@ -74,8 +74,10 @@ __global__ __launch_bounds__(256) void k_verlet(const float* __restrict__ sin_, 
 // whose waves leave most of the chip idle (by_quads): bound by the chain of
 // dependent loads of a vertex (its records, the gathers, a record per visit,
 // the hit's triangle), which a quad walks with fewer instructions and fewer
-// cache-line requests between them.  63 VGPRs (12-wide rows) against 126, so
-// eight waves per SIMD.
+// cache-line requests between them.  65 VGPRs (12-wide rows) against 88; held
+// to 64 for an eighth wave per SIMD, the small cloths lose what the large ones
+// gain (4,096 vertices 6.9 -> 7.1 us per pipelined step).  A counting launch
+// takes the plain walk, whose visits are counted.
 template <bool DEBUG, bool COUNT, int EW>
 __global__ __launch_bounds__(256) void k_verlet_quad(const float* __restrict__ sin_, float* __restrict__ sout,
                                                      const float* contact_in, float* contact_out,
@@ -84,14 +86,15 @@ __global__ __launch_bounds__(256) void k_verlet_quad(const float* __restrict__ s
                                                      float* __restrict__ dbg_pre, int32_t* __restrict__ dbg_hit,
                                                      uint8_t* __restrict__ dbg_in,
                                                      unsigned long long* __restrict__ ctr) {
-  __shared__ int32_t qstk[WSTK_LDS * QSTK_QUADS];
+  __shared__ int32_t qstk[(WSTK_LDS + 1) * QSTK_QUADS];
   const uint32_t i = blockIdx.x * QSTK_QUADS + (threadIdx.x >> 2);
   const int e = (int)(threadIdx.x & 3u);
   uint32_t visits = 0;
   const bool active = i < n;
   if (active)
-    step_vertex_quad<DEBUG, EW>(i, e, sin_, sout, contact_in, contact_out, row, rec, a, bvh,
-                                spill_of(spill, i, n, qstk + (threadIdx.x >> 2)), visits, dbg_pre, dbg_hit, dbg_in);
+    step_vertex_quad<DEBUG, EW, !COUNT>(i, e, sin_, sout, contact_in, contact_out, row, rec, a, bvh,
+                                        spill_of(spill, i, n, qstk + (threadIdx.x >> 2)), visits, dbg_pre, dbg_hit,
+                                        dbg_in);
   if (COUNT) count_block(e == 0 ? visits : 0u, active && e == 0, ctr);
 }
 
@@ -119,13 +122,13 @@ __global__ __launch_bounds__(256) void k_collide_quad(BvhView bvh, const float* 
                                                       float* __restrict__ out_n) {
   const uint32_t i = blockIdx.x * QSTK_QUADS + (threadIdx.x >> 2);
   const int e = (int)(threadIdx.x & 3u);
-  __shared__ int32_t qstk[WSTK_LDS * QSTK_QUADS];
+  __shared__ int32_t qstk[(WSTK_LDS + 1) * QSTK_QUADS];
   if (i >= n) return;
   f3 p = ld3(pts + 3 * (size_t)i), nc;
   int32_t h;
   uint32_t visits = 0;
-  const bool in = collide_project_quad(bvh, p, nc, h, visits, e, spill_of(spill, i, n, qstk + (threadIdx.x >> 2)),
-                                       load_quad_root(bvh, e));
+  const bool in = collide_project_quad<true>(bvh, p, nc, h, visits, e,
+                                             spill_of(spill, i, n, qstk + (threadIdx.x >> 2)), load_quad_root(bvh, e));
   if (e < 2) st3((e ? out_n : out_pos) + 3 * (size_t)i, e ? nc : p);
   if (e == 2) hit[i] = h;
   if (e == 3) ins[i] = in ? 1 : 0;
