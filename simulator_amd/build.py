@@ -13,7 +13,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libclothcore.so")
 
-SOURCES = ["host_scene.cpp", "host_obj.cpp", "lbvh.hip", "sort.hip", "refit.hip", "sim.hip", "bbody.hip", "batch.hip", "adjoint.hip", "wide.hip", "noalloc.hip"]
+SOURCES = ["host_scene.cpp", "host_obj.cpp", "lbvh.hip", "sort.hip", "refit.hip", "sim.hip", "bbody.hip", "batch.hip", "adjoint.hip", "wide.hip", "noalloc.hip", "host_io.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -ffp-contract=off: a*b+c stays two roundings unless fmaf is written out;

@@ -41,6 +41,7 @@ constexpr int TILES[3] = {64, 128, 256};
 constexpr int GRAPH_STEPS_B = 16;
 
 struct Batch {
+  Stage stage;                               // host arrays on their way (host_io.hip)
   hipStream_t stream = nullptr;
   uint32_t count = 0, ntotal = 0;
   std::vector<uint32_t> v_off;               // [count+1] first vertex of each instance
@@ -394,15 +395,8 @@ int cc_batch_get_state(cc_batch* b, uint32_t inst, float* x_cur, float* x_prev, 
     Batch& B = b->b;
     CC_HIP(hipDeviceSynchronize());
     const uint32_t o = B.v_off[inst], n = B.v_off[inst + 1] - o;
-    std::vector<float> st(6 * (size_t)n), c(3 * (size_t)n);
-    copy_on(st.data(), B.state[B.cur].p + 6 * (size_t)o, st.size() * 4, hipMemcpyDeviceToHost, b->b.stream);
-    copy_on(c.data(), B.contact.p + 3 * (size_t)o, c.size() * 4, hipMemcpyDeviceToHost, b->b.stream);
-    for (uint32_t i = 0; i < n; ++i)
-      for (int k = 0; k < 3; ++k) {
-        if (x_cur) x_cur[3 * (size_t)i + k] = st[6 * (size_t)i + k];
-        if (x_prev) x_prev[3 * (size_t)i + k] = st[6 * (size_t)i + 3 + k];
-        if (contact_n) contact_n[3 * (size_t)i + k] = c[3 * (size_t)i + k];
-      }
+    read_state(B.stage, B.state[B.cur].p + 6 * (size_t)o, B.contact.p + 3 * (size_t)o, n, x_cur, x_prev, contact_n,
+               B.stream);
   });
 }
 

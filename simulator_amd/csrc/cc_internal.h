@@ -8,6 +8,7 @@
 #include <atomic>
 #include <cstdint>
 #include <stdexcept>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -109,6 +110,36 @@ struct DBuf {
   }
   void zero(hipStream_t s) {
     if (n) CC_HIP(hipMemsetAsync(p, 0, n * sizeof(T), s));
+  }
+};
+
+// Pinned host memory, grown as needed, that kernels read and write directly,
+// and the spill area of a handle's point queries (see host_io.hip).  The mutex
+// is held from a call's first write of it to its last read.
+struct Stage {
+  std::mutex m;
+  char* p = nullptr;
+  size_t n = 0;
+  DBuf<int32_t> spill;
+  Stage() = default;
+  Stage(const Stage&) = delete;
+  Stage& operator=(const Stage&) = delete;
+  ~Stage() {
+    if (p) (void)hipHostFree(p);
+  }
+  char* host(size_t bytes) {
+    if (bytes <= n) return p;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+    if (fault_now(FAULT_ALLOC)) throw Error(CC_ERR_ALLOC, "hipHostMalloc: injected failure (cc_fault_inject)");
+    const hipError_t e = hipHostMalloc((void**)&p, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) {
+      p = nullptr;
+      throw Error(CC_ERR_ALLOC, std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
+    }
+    n = bytes;
+    return p;
   }
 };
 

@@ -46,6 +46,7 @@ StepArgs step_args(const cc_params& prm, uint32_t ntypes);
 // ------------------------------------------------------------------ Sim
 struct Sim {
   int device = 0;
+  Stage stage;              // host arrays on their way (host_io.hip)
   hipStream_t stream = nullptr;
   uint32_t n = 0, ntypes = 0;
   cc_params prm{};
@@ -532,6 +533,21 @@ struct Sim {
 // tail the caller has set.  Asynchronous on s.
 void launch_collide_points(const BvhView& v, const float* pts, uint32_t n, int32_t* spill, int32_t* hit,
                            uint8_t* ins, float* out_pos, float* out_n, hipStream_t s);
+
+// the tail of a spill area set to no faults and the default stack limit, and its
+// faults to a word that the device reaches
+void launch_spill_tail(int32_t* tail, hipStream_t s);
+void launch_spill_status(const int32_t* tail, uint32_t* status, hipStream_t s);
+
+// Host arrays of a caller through a handle's pinned memory: n states to up to
+// three arrays of vec3 (any may be NULL), and the collision query of n host
+// points (returns its traversal faults), both synchronous on s; n vec3 to two
+// device arrays, asynchronous: the caller holds st.m until s has done it.
+void read_state(Stage& st, const float* state, const float* contact, uint32_t n, float* x_cur, float* x_prev,
+                float* contact_n, hipStream_t s);
+void write_points(Stage& st, const float* src, uint32_t n, float* a, float* b, hipStream_t s);
+uint32_t query_points(Stage& st, const BvhView& v, const float* pts, uint32_t n, int32_t* hit, uint8_t* inside,
+                      float* out_pos, float* out_n, hipStream_t s);
 
 // All spring types of a cloth merged into one CSR row per vertex (types in
 // order, each row in its CSR order); records {end | type << 30, rest bits}.

@@ -1,7 +1,7 @@
 // noalloc.hip -- the collision query without device allocation.
 //
-// cc_collide_points allocates its inputs, outputs and the traversal spill
-// area on every call.  cc_collide_points_noalloc takes device inputs and
+// cc_collide_points takes host arrays and keeps pinned memory and a spill area in
+// its handle.  cc_collide_points_noalloc takes device inputs and
 // outputs from the caller and keeps its spill area in `scratch`, a
 // file-scope device array of fixed size (each GPU the library runs on holds
 // one copy until the process ends), so that callers which cannot allocate
@@ -42,7 +42,7 @@ static int32_t* scratch_of(int dev) {
 }
 
 // the spill tail of this call: no faults, the default stack limit
-__global__ void k_noalloc_tail(int32_t* __restrict__ tail) {
+__global__ void k_spill_tail(int32_t* __restrict__ tail) {
   if (threadIdx.x == 0) {
     tail[0] = 0;
     tail[1] = STACK_LIMIT;
@@ -50,8 +50,18 @@ __global__ void k_noalloc_tail(int32_t* __restrict__ tail) {
 }
 
 // the call's traversal faults to the caller's status word
-__global__ void k_noalloc_status(const int32_t* __restrict__ tail, uint32_t* __restrict__ status) {
+__global__ void k_spill_status(const int32_t* __restrict__ tail, uint32_t* __restrict__ status) {
   if (threadIdx.x == 0) *status = (uint32_t)tail[0];
+}
+
+void launch_spill_tail(int32_t* tail, hipStream_t s) {
+  k_spill_tail<<<1, 64, 0, s>>>(tail);
+  CC_LAUNCHED();
+}
+
+void launch_spill_status(const int32_t* tail, uint32_t* status, hipStream_t s) {
+  k_spill_status<<<1, 64, 0, s>>>(tail, status);
+  CC_LAUNCHED();
 }
 
 }  // namespace cc
@@ -85,13 +95,9 @@ extern "C" int cc_collide_points_noalloc(cc_sim* sim, const float* pts3, uint32_
         CC_HIP(hipStreamWaitEvent(s, S.ev_pose[k], 0));
       }
       int32_t* tail = spill + (size_t)STACK_SPILL * n;
-      k_noalloc_tail<<<1, 64, 0, s>>>(tail);
-      CC_LAUNCHED();
+      launch_spill_tail(tail, s);
       launch_collide_points(S.body.view(k), pts3, n, spill, hit, inside, out_pos, out_n, s);
-      if (status) {
-        k_noalloc_status<<<1, 64, 0, s>>>(tail, status);
-        CC_LAUNCHED();
-      }
+      if (status) launch_spill_status(tail, status, s);
     } catch (...) {
       if (prev != S.device) (void)hipSetDevice(prev);
       throw;

@@ -579,14 +579,7 @@ int cc_sim_get_state(cc_sim* sim, float* x_cur, float* x_prev, float* contact_n)
     CC_REQUIRE(sim, "cc_sim_get_state: null");
     Sim& S = sim->s;
     CC_HIP(hipDeviceSynchronize());
-    std::vector<float> packed(6 * (size_t)S.n);
-    copy_on(packed.data(), S.state[S.cur].p, packed.size() * 4, hipMemcpyDeviceToHost, sim->s.stream);
-    for (uint32_t i = 0; i < S.n; ++i)
-      for (int c = 0; c < 3; ++c) {
-        if (x_cur) x_cur[3 * (size_t)i + c] = packed[6 * (size_t)i + c];
-        if (x_prev) x_prev[3 * (size_t)i + c] = packed[6 * (size_t)i + 3 + c];
-      }
-    if (contact_n) copy_on(contact_n, S.contact.p, 3 * (size_t)S.n * 4, hipMemcpyDeviceToHost, sim->s.stream);
+    read_state(S.stage, S.state[S.cur].p, S.contact.p, S.n, x_cur, x_prev, contact_n, S.stream);
   });
 }
 
@@ -839,9 +832,8 @@ int cc_body_set_vertices(cc_sim* sim, const float* verts3) {
     CC_HIP(hipDeviceSynchronize());
     Sim& S = sim->s;
     const int k = B.slot_of(S.frame);
-    const size_t bytes = 3 * (size_t)B.nv * 4;
-    CC_HIP(hipMemcpyAsync(B.rest.p, verts3, bytes, hipMemcpyHostToDevice, S.stream));
-    CC_HIP(hipMemcpyAsync(B.slot[k].verts.p, B.rest.p, bytes, hipMemcpyDeviceToDevice, S.stream));
+    std::lock_guard<std::mutex> g(S.stage.m);
+    write_points(S.stage, verts3, B.nv, B.rest.p, B.slot[k].verts.p, S.stream);
     // new rest pose: the topology from it as given, then the current frame's
     // pose (a static body's is the one just built)
     S.rebuild_body(k);
@@ -949,26 +941,9 @@ int cc_collide_points(cc_sim* sim, const float* pts3, uint32_t n, int32_t* hit, 
     CC_REQUIRE(sim && pts3 && hit && inside && out_pos && out_n, "cc_collide_points: null argument");
     if (n == 0) return;
     Sim& S = sim->s;
-    hipStream_t s = S.stream;
     CC_HIP(hipDeviceSynchronize());
-    DBuf<float> p, op, on;
-    DBuf<int32_t> h;
-    DBuf<uint8_t> in;
-    DBuf<int32_t> sp;
-    p.upload(pts3, 3 * (size_t)n, s);
-    alloc_spill(sp, n, s);
-    op.alloc(3 * (size_t)n);
-    on.alloc(3 * (size_t)n);
-    h.alloc(n);
-    in.alloc(n);
-    launch_collide_points(S.body.view(S.body.slot_of(S.frame)), p.p, n, sp.p, h.p, in.p, op.p, on.p, s);
-    CC_HIP(hipMemcpyAsync(hit, h.p, 4 * (size_t)n, hipMemcpyDeviceToHost, s));
-    CC_HIP(hipMemcpyAsync(inside, in.p, n, hipMemcpyDeviceToHost, s));
-    CC_HIP(hipMemcpyAsync(out_pos, op.p, 12 * (size_t)n, hipMemcpyDeviceToHost, s));
-    CC_HIP(hipMemcpyAsync(out_n, on.p, 12 * (size_t)n, hipMemcpyDeviceToHost, s));
-    uint32_t fault = 0;
-    CC_HIP(hipMemcpyAsync(&fault, sp.p + (size_t)STACK_SPILL * n, 4, hipMemcpyDeviceToHost, s));
-    CC_HIP(hipStreamSynchronize(s));
+    const uint32_t fault = query_points(S.stage, S.body.view(S.body.slot_of(S.frame)), pts3, n, hit, inside, out_pos,
+                                        out_n, S.stream);
     if (fault) throw Error(CC_ERR_TRAVERSAL, "cc_collide_points: traversal fault (stack overflow or visit bound)");
   });
 }
