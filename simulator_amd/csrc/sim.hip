@@ -482,26 +482,25 @@ int cc_sim_create(const cc_cloth_desc* cloth, const cc_body_desc* bd, const cc_p
       mp.py = bd->pivot[1];
       mp.pz = bd->pivot[2];
       mp.dt = (double)params->dt;
-      // Update lanes and frames per chain of launches.  A refitted body:
-      // three lanes (the 501k-triangle body, A/B in one process per setting
-      // on the same GPU: 44.6-44.8 us per step in graph blocks, frames
-      // 50-530, against 49.3-49.5 with two lanes and 52.6-53.5 with four;
-      // one call per frame 52.4-52.7 against 52.2-52.4 with two) of three
-      // frames (20 single steps 33.8-34.5 us against 34.5-35.4 with two,
-      // 500 steps 41.7-42.0 against 42.2-42.6, one call per frame the same).
-      // A rebuilt body, whose update is a chain of 17 small launches: two
-      // lanes of three frames (111 x 111 over the 50,688-triangle body:
-      // 35.4-35.6 us per step over 500 steps through the graphs against
-      // 37.0-37.5 with three lanes of two, 40.0-40.1 against 41.0-42.0 in
-      // contact; one call per frame the same).
+      // Update lanes and frames per chain of launches: four frames share each
+      // launch, which is bound by latency far more than by their work.  A
+      // refitted body, an update of five launches, keeps to one lane: more run
+      // into one another and into the step (us per step of a 480-step run / of
+      // one call per frame, three lanes of three frames against one of four:
+      // 12.4 / 12.1 against 10.5 / 11.5 at 5,760 triangles, 15.3 / 15.5 against
+      // 13.6 / 14.9 at 50,688, 44.6 / 48.2 against 43.3 / 47.4 at 501,120).  A
+      // rebuilt body, a chain of 14 launches, fills two (two of three against
+      // two of four and one of four: 14.8, 13.5, 16.6 at 5,760; 20.6, 20.8, 25.4
+      // at 50,688) and from some 100,000 triangles on three (two, three lanes of
+      // four: 35.6, 32.9 at 146,400; 95.0, 90.2 at 501,120).
       const bool rebuilt = bd->mode == CC_BODY_REBUILD;
-      int lanes = rebuilt ? 2 : 3;
+      int lanes = rebuilt ? (bd->nf > 100000 ? 3 : 2) : 1;
       if (const char* e = std::getenv("CC_BODY_LANES")) lanes = std::atoi(e);
       CC_REQUIRE(lanes >= 1 && lanes <= MAX_LANES, "cc_sim_create: CC_BODY_LANES must be 1..4");
       if (const char* e = std::getenv("CC_GRAPH_STEPS")) S.graph_steps = std::atoi(e);
       CC_REQUIRE(S.graph_steps >= 2 && S.graph_steps % 2 == 0 && 2 * S.graph_steps <= MAX_SLOTS,
                  "cc_sim_create: CC_GRAPH_STEPS must be even, 2..MAX_SLOTS/2");
-      int chain = 3;
+      int chain = MAX_FRAMES;
       if (const char* e = std::getenv("CC_BUILD_FRAMES")) chain = std::atoi(e);
       CC_REQUIRE(chain >= 1 && chain <= MAX_FRAMES, "cc_sim_create: CC_BUILD_FRAMES must be 1..4");
       // 0: rebuilt bodies of any size take the Karras searches and the
