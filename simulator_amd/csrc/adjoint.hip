@@ -133,61 +133,85 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_force(
 
 // One spring's adjoint terms (the forward's f_ij in F_i and f_ji in F_j):
 // gp += a1, gq -= v1 / dt, gp -= a2, gq += v2 / dt, in that order, and its
-// parts gk, gr of the gradients of its type's stiffness and of rest_scale.
-// All zero for an empty slot.
+// parts gk0 .. gk2 (its type's, the others 0) and gr of the gradients of the
+// stiffnesses and of rest_scale.  All zero for an empty slot.
 struct AdjTerm {
   f3 a1, v1, a2, v2;
-  float gk, gr;
-  uint32_t t;
+  float gk0, gk1, gk2, gr;
 };
 __device__ inline AdjTerm adj_spring(f3 pi, f3 vi, f3 lFi, f3 pj, f3 vj, f3 lFj, uint2 r, bool real,
-                                     const AdjArgs& a) {
+                                     const AdjArgs& a, float ks0, float ks1, float ks2) {
   AdjTerm o;
-  o.t = r.x >> 30;
+  const uint32_t ty = r.x >> 30;
   const float rest0 = __uint_as_float(r.y), rest = rest0 * a.rest_scale;
-  const float ks = o.t == 0 ? a.k0 : (o.t == 1 ? a.k1 : a.k2);
+  const float ks = ty == 0 ? ks0 : (ty == 1 ? ks1 : ks2);
   f3 gd;
   float dl, L;
   // f_ij, in F_i
   spring_vjp(mk((pi.x - pj.x) + a.eps, (pi.y - pj.y) + a.eps, (pi.z - pj.z) + a.eps), vi - vj, ks, rest, a.kd, lFi,
              gd, o.v1, dl, L);
   o.a1 = mk(fmaf(o.v1.x, a.inv_dt, gd.x), fmaf(o.v1.y, a.inv_dt, gd.y), fmaf(o.v1.z, a.inv_dt, gd.z));
-  o.gk = -(L - rest) * dl;
+  const float gk = -(L - rest) * dl;
   o.gr = ks * rest0 * dl;
   // f_ji, in F_j (the same type and rest length)
   spring_vjp(mk((pj.x - pi.x) + a.eps, (pj.y - pi.y) + a.eps, (pj.z - pi.z) + a.eps), vj - vi, ks, rest, a.kd, lFj,
              gd, o.v2, dl, L);
   o.a2 = mk(fmaf(o.v2.x, a.inv_dt, gd.x), fmaf(o.v2.y, a.inv_dt, gd.y), fmaf(o.v2.z, a.inv_dt, gd.z));
-  if (!real) {
-    const f3 z = mk(0.0f, 0.0f, 0.0f);
-    o = AdjTerm{z, z, z, z, 0.0f, 0.0f, 3u};
-  }
+  // by a mask and not by a select, as in spring_scale
+  uint32_t keep = real ? ~0u : 0u;
+  asm("" : "+v"(keep));
+  auto masked = [keep](float v) { return __uint_as_float(__float_as_uint(v) & keep); };
+  auto masked3 = [&](f3 v) { return mk(masked(v.x), masked(v.y), masked(v.z)); };
+  o.a1 = masked3(o.a1);
+  o.v1 = masked3(o.v1);
+  o.a2 = masked3(o.a2);
+  o.v2 = masked3(o.v2);
+  o.gr = masked(o.gr);
+  o.gk0 = masked(ty == 0 ? gk : 0.0f);
+  o.gk1 = masked(ty == 1 ? gk : 0.0f);
+  o.gk2 = masked(ty == 2 ? gk : 0.0f);
   return o;
 }
 // Its sum into gp, gq and the parameter gradients g = {k0, k1, k2, -, rest_scale}.
 __device__ inline void adj_add(const AdjTerm& o, float inv_dt, f3& gp, f3& gq, float (&g)[NPARAM]) {
   gp = gp + o.a1;
   gq = mk(fmaf(-o.v1.x, inv_dt, gq.x), fmaf(-o.v1.y, inv_dt, gq.y), fmaf(-o.v1.z, inv_dt, gq.z));
-  g[0] += o.t == 0 ? o.gk : 0.0f;
-  g[1] += o.t == 1 ? o.gk : 0.0f;
-  g[2] += o.t == 2 ? o.gk : 0.0f;
+  g[0] += o.gk0;
+  g[1] += o.gk1;
+  g[2] += o.gk2;
   g[4] += o.gr;
   gp = gp - o.a2;
   gq = mk(fmaf(o.v2.x, inv_dt, gq.x), fmaf(o.v2.y, inv_dt, gq.y), fmaf(o.v2.z, inv_dt, gq.z));
 }
-template <int K>
-__device__ inline f3 quad_bcast3(f3 v) {
-  return mk(quad_bcast<K>(v.x), quad_bcast<K>(v.y), quad_bcast<K>(v.z));
-}
-// lane K's terms added in every lane of the quad, in their order
+// adj_add of lane K's terms in every lane of the quad, the operands read across
+// lanes by the additions themselves (see quad_add of cc_step.h for the wait).
 template <int K, int NB>
 __device__ inline void quad_adj_add(const AdjTerm (&t)[NB], float inv_dt, f3& gp, f3& gq, float (&g)[NPARAM]) {
 #pragma unroll
   for (int k = 0; k < NB; ++k) {
-    const AdjTerm o{quad_bcast3<K>(t[k].a1), quad_bcast3<K>(t[k].v1), quad_bcast3<K>(t[k].a2),
-                    quad_bcast3<K>(t[k].v2), quad_bcast<K>(t[k].gk),  quad_bcast<K>(t[k].gr),
-                    (uint32_t)quad_perm<K * 0x55>((int32_t)t[k].t)};
-    adj_add(o, inv_dt, gp, gq, g);
+    const AdjTerm& o = t[k];
+#define CC_LANE " quad_perm:[%c[K],%c[K],%c[K],%c[K]] row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %[ax], %0" CC_LANE "v_add_f32_dpp %1, %[ay], %1" CC_LANE "v_add_f32_dpp %2, %[az], %2" CC_LANE
+        "v_fmac_f32_dpp %3, -%[vx], %[dt]" CC_LANE "v_fmac_f32_dpp %4, -%[vy], %[dt]" CC_LANE
+        "v_fmac_f32_dpp %5, -%[vz], %[dt]" CC_LANE
+        : "+v"(gp.x), "+v"(gp.y), "+v"(gp.z), "+v"(gq.x), "+v"(gq.y), "+v"(gq.z)
+        : [ax] "v"(o.a1.x), [ay] "v"(o.a1.y), [az] "v"(o.a1.z), [vx] "v"(o.v1.x), [vy] "v"(o.v1.y),
+          [vz] "v"(o.v1.z), [dt] "v"(inv_dt), [K] "n"(K));
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %[g0], %0" CC_LANE "v_add_f32_dpp %1, %[g1], %1" CC_LANE "v_add_f32_dpp %2, %[g2], %2" CC_LANE
+        "v_add_f32_dpp %3, %[gr], %3" CC_LANE
+        : "+v"(g[0]), "+v"(g[1]), "+v"(g[2]), "+v"(g[4])
+        : [g0] "v"(o.gk0), [g1] "v"(o.gk1), [g2] "v"(o.gk2), [gr] "v"(o.gr), [K] "n"(K));
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, -%[ax], %0" CC_LANE "v_add_f32_dpp %1, -%[ay], %1" CC_LANE
+        "v_add_f32_dpp %2, -%[az], %2" CC_LANE
+        "v_fmac_f32_dpp %3, %[vx], %[dt]" CC_LANE "v_fmac_f32_dpp %4, %[vy], %[dt]" CC_LANE
+        "v_fmac_f32_dpp %5, %[vz], %[dt]" CC_LANE
+        : "+v"(gp.x), "+v"(gp.y), "+v"(gp.z), "+v"(gq.x), "+v"(gq.y), "+v"(gq.z)
+        : [ax] "v"(o.a2.x), [ay] "v"(o.a2.y), [az] "v"(o.a2.z), [vx] "v"(o.v2.x), [vy] "v"(o.v2.y),
+          [vz] "v"(o.v2.z), [dt] "v"(inv_dt), [K] "n"(K));
+#undef CC_LANE
   }
 }
 
@@ -207,16 +231,19 @@ struct AdjStep {
 // row order in every lane); the parameter sums go out per 64 vertices, so they
 // add the same numbers in the same order either way.  EW > 0: `rec` holds EW
 // records per vertex (the forward's fixed-width rows); EW == 0: the merged CSR
-// at `row`.  Bound by the chain from the records to the gathers and the terms
-// (two square roots and divisions each) on a chip that one lane per vertex
-// fills to a quarter at 128 x 128: 200 steps back take 1.3 ms (6.1 us a step,
-// 101 VGPRs), against 3.6 with two launches a step (9.2 + 2.9), one lane per
-// vertex and the states recomputed (5.3).
+// at `row`.  Bound by the chain
+// from the records to the gathers and by the terms' instructions (two square
+// roots and divisions each), one wave per SIMD at 128 x 128.  So the records load
+// with the vertex's own data, the gathers are waited for once, empty slots are
+// masked and the sums read across lanes by the additions themselves: 200 steps
+// back take 1.16 ms (5.6 us a step) against 1.28 without (6.2), and 3.6 with two
+// launches a step (9.2 + 2.9), one lane per vertex and the states recomputed (5.3).
 template <int EW, int LANES>
 __global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint32_t* __restrict__ row,
                                                           const uint2* __restrict__ rec, AdjStep S, AdjArgs a) {
   constexpr bool QUAD = LANES == 4;
   constexpr int NB = EW && QUAD ? EW / 4 : (QUAD ? 3 : (EW ? 6 : 4));   // springs of a lane at a time
+  constexpr bool PRE = EW > 0 && QUAD;   // all records load with the vertex's own data
   constexpr uint32_t VERTS = ADJ_THREADS / LANES;
   __shared__ float sg[QUAD ? VERTS : 1][NPARAM];
   const uint32_t v = threadIdx.x / LANES, i = blockIdx.x * VERTS + v;
@@ -224,6 +251,11 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint
   float g[NPARAM] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   if (i < n) {
     const size_t o = 3 * (size_t)i;
+    uint2 er[NB];
+    if constexpr (PRE) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k) er[k] = rec[(size_t)i * EW + (uint32_t)(e * NB + k)];
+    }
     const uint32_t r0raw = row[i], r1raw = EW ? 0u : row[i + 1];
     const f3 pi = ld3(S.state + 2 * o), qi = ld3(S.state + 2 * o + 3);
     const f3 lFi = ld3(S.lf + o);
@@ -237,15 +269,18 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint
       q1 = ld3(S.state1 + 2 * o + 3);
     }
     const f3 vi = mk((pi.x - qi.x) * a.inv_dt, (pi.y - qi.y) * a.inv_dt, (pi.z - qi.z) * a.inv_dt);
+    // in registers, as in step_vertex (selects between fields of `a` become loads)
+    const float ks0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k0)));
+    const float ks1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k1)));
+    const float ks2 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k2)));
     const uint32_t r0 = EW ? i * (uint32_t)EW : r0raw & ROW_MASK, r1 = EW ? r0 + EW : r1raw & ROW_MASK;
-    for (uint32_t k0 = r0; k0 < r1; k0 += NB * LANES) {
-      uint2 er[NB];
+    for (uint32_t k0 = r0; PRE || k0 < r1; k0 += NB * LANES) {
       bool real[NB];
       float sj[NB][6], lj[NB][3];
 #pragma unroll
       for (int k = 0; k < NB; ++k) {
         const uint32_t at = k0 + (uint32_t)(e * NB + k);
-        er[k] = rec[EW ? at : min(at, r1 - 1)];
+        if (!PRE) er[k] = rec[EW ? at : min(at, r1 - 1)];
         real[k] = EW ? (er[k].x & PAD_TYPE) != PAD_TYPE : at < r1;
         if (!EW && !real[k]) er[k] = make_uint2(i | PAD_TYPE, 0u);
       }
@@ -257,13 +292,20 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint
         sj[k][0] = u.x; sj[k][1] = u.y; sj[k][2] = w.x; sj[k][3] = w.y; sj[k][4] = x.x; sj[k][5] = x.y;
         for (int c = 0; c < 3; ++c) lj[k][c] = S.lf[3 * (size_t)j + c];
       }
+      // waited for once: the compiler issues some of them at their first use
+      // otherwise, one memory round trip after another
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        asm volatile("" ::"v"(sj[k][0]), "v"(sj[k][1]), "v"(sj[k][2]), "v"(sj[k][3]), "v"(sj[k][4]), "v"(sj[k][5]),
+                     "v"(lj[k][0]), "v"(lj[k][1]), "v"(lj[k][2]));
       AdjTerm t[NB];
 #pragma unroll
       for (int k = 0; k < NB; ++k) {
         const f3 pj = mk(sj[k][0], sj[k][1], sj[k][2]);
         const f3 vj = mk((sj[k][0] - sj[k][3]) * a.inv_dt, (sj[k][1] - sj[k][4]) * a.inv_dt,
                          (sj[k][2] - sj[k][5]) * a.inv_dt);
-        t[k] = adj_spring(pi, vi, lFi, pj, vj, mk(lj[k][0], lj[k][1], lj[k][2]), er[k], real[k], a);
+        t[k] = adj_spring(pi, vi, lFi, pj, vj, mk(lj[k][0], lj[k][1], lj[k][2]), er[k], real[k], a,
+                          ks0, ks1, ks2);
         if constexpr (!QUAD) adj_add(t[k], a.inv_dt, gp, gq, g);
       }
       if constexpr (QUAD) {
@@ -272,6 +314,7 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint
         quad_adj_add<2>(t, a.inv_dt, gp, gq, g);
         quad_adj_add<3>(t, a.inv_dt, gp, gq, g);
       }
+      if (PRE) break;
     }
     if (S.state1) {
       const AdjForce r = adj_force(gp, gq, (r0raw & PIN_BIT) != 0, c1, n1, p1, q1, a);
@@ -304,25 +347,39 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint
 }
 
 // acc[b] += the sums of L steps, last step first, over blocks of ADJ_THREADS
-// vertices (four waves each, added in order in FP32): thread = block and
-// parameter.
+// vertices (four waves each, added in order in FP32): one workgroup per block.
+// Bound by the latency of the loads: all threads fetch ACC_STEPS steps' sums
+// together, then one thread per parameter adds them in order (200 steps of 16,384
+// vertices: 6 us against 31 with one thread per sum fetching its own).
+constexpr uint32_t ACC_STEPS = 256;
 __global__ __launch_bounds__(256) void k_adj_acc(const float* __restrict__ part, uint32_t L, uint32_t nw,
-                                                 uint32_t nblk, double* __restrict__ acc) {
-  const uint32_t q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= NPARAM * nblk) return;
-  const uint32_t b = q / NPARAM, p = q % NPARAM, w0 = 4 * b;
-  double s = acc[q];
+                                                 double* __restrict__ acc) {
+  __shared__ float f[ACC_STEPS * NPARAM];
+  const uint32_t w0 = 4 * blockIdx.x;
+  double s = threadIdx.x < NPARAM ? acc[blockIdx.x * NPARAM + threadIdx.x] : 0.0;
+  for (uint32_t t = L; t > 0;) {
+    const uint32_t k = min(t, ACC_STEPS);
+#pragma unroll
+    for (uint32_t r = 0; r < NPARAM; ++r) {
+      const uint32_t q = r * 256 + threadIdx.x, u = q / NPARAM, p = q % NPARAM;
+      if (u >= k) continue;
+      const float* x = part + NPARAM * ((size_t)(t - 1 - u) * nw + w0) + p;
+      float v = 0.0f;
+      v += x[0];
+      v += w0 + 1 < nw ? x[NPARAM] : 0.0f;
+      v += w0 + 2 < nw ? x[2 * NPARAM] : 0.0f;
+      v += w0 + 3 < nw ? x[3 * NPARAM] : 0.0f;
+      f[q] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < NPARAM) {
 #pragma unroll 8
-  for (uint32_t t = L; t-- > 0;) {
-    const float* x = part + NPARAM * ((size_t)t * nw + w0) + p;
-    float f = 0.0f;
-    f += x[0];
-    f += w0 + 1 < nw ? x[NPARAM] : 0.0f;
-    f += w0 + 2 < nw ? x[2 * NPARAM] : 0.0f;
-    f += w0 + 3 < nw ? x[3 * NPARAM] : 0.0f;
-    s += (double)f;
+      for (uint32_t u = 0; u < k; ++u) s += (double)f[u * NPARAM + threadIdx.x];
+    }
+    __syncthreads();
+    t -= k;
   }
-  acc[q] = s;
+  if (threadIdx.x < NPARAM) acc[blockIdx.x * NPARAM + threadIdx.x] = s;
 }
 
 // out[p] = sum over blocks of acc[p], in FP64 (one workgroup)
@@ -569,7 +626,7 @@ int cc_adj_backward(cc_adj* adj, const float* dl_dx_final, double dl_dtheta[5], 
         CC_LAUNCHED();
         cur ^= 1;
       }
-      k_adj_acc<<<grid_for(NPARAM * (size_t)A.nblk, 256), 256, 0, s>>>(A.part.p, L, nw, A.nblk, A.acc.p);
+      k_adj_acc<<<A.nblk, 256, 0, s>>>(A.part.p, L, nw, A.acc.p);
       CC_LAUNCHED();
     }
     k_reduce_f64<<<1, 256, 0, s>>>(A.acc.p, A.nblk, A.out.p);
