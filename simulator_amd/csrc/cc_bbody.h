@@ -50,6 +50,7 @@ struct XcdMap {
 // the grid-wide kernels, the tiles of the sort, and the workgroups of each
 // build level.
 struct BodyPass {
+  bool refit = false;                 // the REFIT bodies by levels (else built like the others)
   DBuf<uint4> deform, boxes;
   SortTable sort;
   DBuf<LvBlock> level[BB_MAX_LEVELS];
@@ -94,8 +95,14 @@ struct BatchBodies {
   hipEvent_t ev_motion[2] = {nullptr, nullptr};
   int hm = 0;
 
+  // REFIT bodies of two or more triangles keep the topology of their frame-0
+  // pose: refitted by levels (refit.hip) over tables of all of them
+  RefitLevel rl[RL_MAX];
+  int nrl = 0;
+  DBuf<float> ritem[RL_MAX];          // [6 * items] boxes of each level's items
+
   BodyPass all;    // set-up: every body built from its frame-0 pose
-  BodyPass step;   // per frame: moving bodies posed, REBUILD ones re-sorted
+  BodyPass step;   // per frame: moving bodies posed, REBUILD ones sorted and built, REFIT ones refitted
 
   BatchBodies() = default;
   BatchBodies(const BatchBodies&) = delete;
@@ -110,6 +117,8 @@ struct BatchBodies {
             hipStream_t s);
   XcdMap xcd;
   BvhView view(uint32_t j, int slot) const;
+  bool by_refit(uint32_t j) const { return h[j].mode == CC_BODY_REFIT && h[j].m >= 2; }
+  void refit_setup(hipStream_t s);
   // motion of frames [frame0, frame0 + nframes) into the device table
   void upload_motion(uint64_t frame0, int nframes, hipStream_t s);
   // One pass into a slot, in three parts: pose + boxes (k selects the

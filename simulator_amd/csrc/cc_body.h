@@ -159,13 +159,41 @@ void launch_build_levels(const LvBlock* const* level, const uint32_t* n_level,
 // at level 0, else nodes and leaves that the level below left), cut into
 // groups of at most LV_C; tables made once per topology.
 constexpr int RL_MAX = 8;
+struct RefitGroup {
+  uint32_t first, n, out0, rounds;   // first item, items, first item it leaves to the next level, rounds
+  uint32_t v0, n0, body;             // its body's first vertex and node, and number (0 for a single body)
+  float depth;
+};
 struct RefitLevel {
   uint32_t nitems = 0, nblk = 0;
-  DBuf<uint4> blk;         // group: {first item, items, first item it leaves to the next level, rounds}
+  DBuf<RefitGroup> blk;
   DBuf<uint2> rec;         // [nitems] item k, and the split right of it (RL_*)
   DBuf<uint4> wd;          // [nitems] four-wide entries {entry, link} of that split's children A, B
   DBuf<uint32_t> node;     // [nitems] the split's node
 };
+// The same on the host, of one body or of several after one another (items of
+// level 0 at their triangles' places).
+struct RefitTables {
+  std::vector<RefitGroup> blk[RL_MAX];
+  std::vector<uint2> rec[RL_MAX];
+  std::vector<uint4> wd[RL_MAX];
+  std::vector<uint32_t> node[RL_MAX];
+  int nlevels = 0;
+  // adds a body of m >= 2 triangles, the first one's place base0, with nodes
+  // nd and, or empty, the four-wide entries of their child slots
+  void add(const Node* nd, uint32_t m, uint32_t base0, const RefitGroup& body, const std::vector<uint2>& dst);
+  void upload(RefitLevel* rl, hipStream_t s) const;
+};
+// One frame's refit by levels; items[L]: the boxes of level L's items (L > 0).
+struct RefitFrame {
+  const float* verts;
+  float* items[RL_MAX];
+  Node* nodes;
+  float4* wide;              // or nullptr: the boxes go to the nodes
+  float* root;
+};
+void launch_refit_levels(const RefitLevel* rl, int nrl, const uint4* leaf_tri, const RefitFrame* frames, int nframes,
+                         hipStream_t s);
 
 // One frame of the body as the collision query reads it.
 struct Slot {

@@ -553,17 +553,16 @@ __global__ __launch_bounds__(TOP_REFIT_THREADS) void k_refit_top(PF<Node> nodes_
 constexpr uint32_t RL_VALID = 1u << 31, RL_ROOT = 1u << 30, RL_NONE = 0xffffu;
 
 template <bool LEAVES>
-__global__ __launch_bounds__(LV_C) void k_refit_level(const uint4* __restrict__ blk, const uint2* __restrict__ rec,
-                                                      const uint4* __restrict__ wdst,
+__global__ __launch_bounds__(LV_C) void k_refit_level(const RefitGroup* __restrict__ blk,
+                                                      const uint2* __restrict__ rec, const uint4* __restrict__ wdst,
                                                       const uint32_t* __restrict__ node_of, PF<const float> verts_f,
-                                                      const uint4* __restrict__ leaf_tri, float depth,
-                                                      PF<const float> in_f, PF<float> out_f, PF<Node> nodes_f,
+                                                      const uint4* __restrict__ leaf_tri, PF<const float> in_f, PF<float> out_f, PF<Node> nodes_f,
                                                       PF<float4> wide_f, PF<float> root_f) {
   __shared__ float2 U[2][LV_C][3];
-  const uint4 b = blk[blockIdx.x];         // {first item, items, first output item, rounds}
-  const int32_t k = (int32_t)threadIdx.x, n = (int32_t)b.y;
+  const RefitGroup b = blk[blockIdx.x];
+  const int32_t k = (int32_t)threadIdx.x, n = (int32_t)b.n;
   const bool have = k < n;
-  const uint32_t at = b.x + (uint32_t)min(k, n - 1);
+  const uint32_t at = b.first + (uint32_t)min(k, n - 1);
   const uint2 r2 = rec[at];
   float4* __restrict__ wide = pick(wide_f);
   uint4 wd = make_uint4(~0u, 0u, ~0u, 0u);
@@ -571,8 +570,8 @@ __global__ __launch_bounds__(LV_C) void k_refit_level(const uint4* __restrict__ 
   Box6 own;
   if constexpr (LEAVES) {
     const uint4 t = leaf_tri[at];
-    const float* __restrict__ verts = pick(verts_f);
-    prim_box(ld3(verts + 3 * (size_t)t.x), ld3(verts + 3 * (size_t)t.y), ld3(verts + 3 * (size_t)t.z), depth, own.v,
+    const float* __restrict__ verts = pick(verts_f) + 3 * (size_t)b.v0;
+    prim_box(ld3(verts + 3 * (size_t)t.x), ld3(verts + 3 * (size_t)t.y), ld3(verts + 3 * (size_t)t.z), b.depth, own.v,
              own.v + 3);
   } else {
     const float* src = pick(in_f) + 6 * (size_t)at;
@@ -584,7 +583,7 @@ __global__ __launch_bounds__(LV_C) void k_refit_level(const uint4* __restrict__ 
   if (have) lds_box_put(U[0], k, own);
   __syncthreads();
   Box6 run = own, A{}, B{};
-  const int32_t rounds = (int32_t)b.w;     // rounds 0 .. rounds - 1
+  const int32_t rounds = (int32_t)b.rounds;     // rounds 0 .. rounds - 1
 #define CC_ROUND(Q) \
   if (rounds > Q) level_round<Q>(U[Q & 1], U[(Q & 1) ^ 1], have, k, n, l, r, qa, qb, rounds > Q + 1, run, A, B)
   CC_ROUND(0); CC_ROUND(1); CC_ROUND(2); CC_ROUND(3); CC_ROUND(4);
@@ -599,7 +598,7 @@ __global__ __launch_bounds__(LV_C) void k_refit_level(const uint4* __restrict__ 
       put_wide_at(wide, make_uint2(wd.x, wd.y), A.v);
       put_wide_at(wide, make_uint2(wd.z, wd.w), B.v);
     } else {
-      float4* d = reinterpret_cast<float4*>(pick(nodes_f) + node_of[at]);
+      float4* d = reinterpret_cast<float4*>(pick(nodes_f) + b.n0 + node_of[at]);
       d[0] = make_float4(A.v[0], A.v[1], A.v[2], A.v[3]);
       d[1] = make_float4(A.v[4], A.v[5], B.v[0], B.v[1]);
       d[2] = make_float4(B.v[2], B.v[3], B.v[4], B.v[5]);
@@ -607,15 +606,16 @@ __global__ __launch_bounds__(LV_C) void k_refit_level(const uint4* __restrict__ 
     const uint32_t to = r2.y & 0xffffu;
     if ((r2.x & RL_ROOT) || to != RL_NONE) {
       const Box6 box = box_node(box_or(A, B));
-      float* d = (r2.x & RL_ROOT) ? pick(root_f) : out + 6 * (size_t)(b.z + to);
+      float* d = (r2.x & RL_ROOT) ? pick(root_f) + 6 * (size_t)b.body : out + 6 * (size_t)(b.out0 + to);
       put6(d, box.v, box.v + 3);
     }
   }
-  if (have && (r2.y >> 16) != RL_NONE) put6(out + 6 * (size_t)(b.z + (r2.y >> 16)), own.v, own.v + 3);
+  if (have && (r2.y >> 16) != RL_NONE) put6(out + 6 * (size_t)(b.out0 + (r2.y >> 16)), own.v, own.v + 3);
 }
 
 // ======================================================== host side
-void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s) {
+void RefitTables::add(const Node* nd, uint32_t m, uint32_t base0, const RefitGroup& body,
+                      const std::vector<uint2>& dst) {
   struct Item {
     uint32_t first, last;
     int32_t node;          // the item's node, -1 for a leaf
@@ -642,17 +642,18 @@ void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& ds
   std::vector<Item> items(m);
   for (uint32_t i = 0; i < m; ++i) items[i] = {i, i, -1};
   std::vector<uint32_t> at_first(m), at_last(m);   // item starting / ending at a leaf
-  for (nrl = 0; nrl < RL_MAX; ++nrl) {
-    RefitLevel& R = rl[nrl];
-    const uint32_t G = LV_C;
-    const uint32_t ni = (uint32_t)items.size();
-    std::vector<uint4> blk;
-    std::vector<uint2> rec(ni);
-    std::vector<uint4> wd(ni, make_uint4(~0u, 0u, ~0u, 0u));
-    std::vector<uint32_t> node(ni, 0u);
+  int L = 0;
+  for (; L < RL_MAX && !items.empty(); ++L) {
+    const uint32_t ni = (uint32_t)items.size(), base = L == 0 ? base0 : (uint32_t)rec[L].size();
+    const uint32_t end = std::max((uint32_t)rec[L].size(), base + ni);
+    rec[L].resize(end, make_uint2(0u, RL_NONE | (RL_NONE << 16)));
+    node[L].resize(end, 0u);
+    if (!dst.empty()) wd[L].resize(end, make_uint4(~0u, 0u, ~0u, 0u));
+    uint2* R = rec[L].data() + base;
+    const uint32_t next0 = L + 1 < RL_MAX ? (uint32_t)rec[L + 1].size() : 0u;
     std::vector<Item> next;
-    for (uint32_t i0 = 0; i0 < ni; i0 += G) {
-      const uint32_t n = std::min<uint32_t>(G, ni - i0);
+    for (uint32_t i0 = 0; i0 < ni; i0 += LV_C) {
+      const uint32_t n = std::min<uint32_t>(LV_C, ni - i0);
       const uint32_t f0 = items[i0].first, l0 = items[i0 + n - 1].last, out0 = (uint32_t)next.size();
       for (uint32_t k = 0; k < n; ++k) {
         at_first[items[i0 + k].first] = k;
@@ -661,16 +662,16 @@ void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& ds
       auto inside = [&](int32_t x) { return x >= 0 && first[x] >= f0 && last[x] <= l0; };
       uint32_t rounds = 0;
       for (uint32_t k = 0; k < n; ++k) {
-        rec[i0 + k] = make_uint2(0u, RL_NONE | (RL_NONE << 16));
+        R[i0 + k] = make_uint2(0u, RL_NONE | (RL_NONE << 16));
         if (k + 1 == n) continue;
         const uint32_t x = node_at[items[i0 + k].last];
         if (!inside((int32_t)x)) continue;
         const uint32_t l = at_first[first[x]], r = at_last[last[x]];
-        rec[i0 + k].x = l | (r << 10) | RL_VALID | (x == 0 ? RL_ROOT : 0u);
-        node[i0 + k] = x;
+        R[i0 + k].x = l | (r << 10) | RL_VALID | (x == 0 ? RL_ROOT : 0u);
+        node[L][base + i0 + k] = x;
         if (!dst.empty()) {
           const uint2 a = dst[2 * (size_t)x], b = dst[2 * (size_t)x + 1];
-          wd[i0 + k] = make_uint4(a.x, a.y, b.x, b.y);
+          wd[L][base + i0 + k] = make_uint4(a.x, a.y, b.x, b.y);
         }
         for (uint32_t len = std::max(k - l + 1, r - k), q = 1; len; len >>= 1, ++q) rounds = std::max(rounds, q);
       }
@@ -696,32 +697,78 @@ void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& ds
         if (x >= 0 && x != it.node) {          // a node finished here
           const uint32_t sp = (uint32_t)(nd[x].childA < 0 ? ~nd[x].childA : nd[x].childA);
           if (x != 0) {
-            rec[i0 + at_last[sp]].y = (rec[i0 + at_last[sp]].y & 0xffff0000u) | ((uint32_t)next.size() - out0);
+            R[i0 + at_last[sp]].y = (R[i0 + at_last[sp]].y & 0xffff0000u) | ((uint32_t)next.size() - out0);
             next.push_back({first[x], last[x], x});
           }
           k = at_last[last[x]] + 1;
         } else {                               // the item itself
-          rec[i0 + k].y = (rec[i0 + k].y & 0xffffu) | (((uint32_t)next.size() - out0) << 16);
+          R[i0 + k].y = (R[i0 + k].y & 0xffffu) | (((uint32_t)next.size() - out0) << 16);
           next.push_back(it);
           ++k;
         }
       }
-      blk.push_back(make_uint4(i0, n, out0, rounds));
+      RefitGroup g = body;
+      g.first = base + i0;
+      g.n = n;
+      g.out0 = next0 + out0;
+      g.rounds = rounds;
+      blk[L].push_back(g);
     }
-    R.nitems = ni;
-    R.nblk = (uint32_t)blk.size();
-    R.blk.upload(blk.data(), blk.size(), s);
-    R.rec.upload(rec.data(), ni, s);
-    R.wd.upload(wd.data(), ni, s);
-    R.node.upload(node.data(), ni, s);
-    CC_HIP(hipStreamSynchronize(s));           // the tables' host copies end here
-    if (nrl > 0)
-      for (int l = 0; l < nlanes * chain; ++l) lane[l].ritem[nrl].alloc(6 * (size_t)ni);
     items.swap(next);
-    if (items.empty()) break;                  // the root was finished
   }
   CC_REQUIRE(items.empty(), "refit levels: too many levels");
-  ++nrl;
+  nlevels = std::max(nlevels, L);
+}
+
+void RefitTables::upload(RefitLevel* rl, hipStream_t s) const {
+  for (int L = 0; L < nlevels; ++L) {
+    RefitLevel& R = rl[L];
+    R.nitems = (uint32_t)rec[L].size();
+    R.nblk = (uint32_t)blk[L].size();
+    R.blk.upload(blk[L].data(), blk[L].size(), s);
+    R.rec.upload(rec[L].data(), rec[L].size(), s);
+    R.wd.upload(wd[L].data(), wd[L].size(), s);
+    R.node.upload(node[L].data(), node[L].size(), s);
+  }
+  CC_HIP(hipStreamSynchronize(s));             // the host copies end here
+}
+
+void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s) {
+  RefitTables t;
+  RefitGroup g{};
+  g.depth = depth;
+  t.add(nd.data(), m, 0, g, dst);
+  t.upload(rl, s);
+  nrl = t.nlevels;
+  for (int L = 1; L < nrl; ++L)
+    for (int l = 0; l < nlanes * chain; ++l) lane[l].ritem[L].alloc(6 * (size_t)rl[L].nitems);
+}
+
+void launch_refit_levels(const RefitLevel* rl, int nrl, const uint4* leaf_tri, const RefitFrame* frames, int nframes,
+                         hipStream_t s) {
+  PF<const float> verts{};
+  PF<Node> nodes{};
+  PF<float> root{};
+  PF<float4> wide{};
+  for (int f = 0; f < nframes; ++f) {
+    verts.p[f] = frames[f].verts;
+    nodes.p[f] = frames[f].nodes;
+    root.p[f] = frames[f].root;
+    wide.p[f] = frames[f].wide;
+  }
+  for (int L = 0; L < nrl; ++L) {
+    const RefitLevel& R = rl[L];
+    PF<const float> in{};
+    PF<float> out{};
+    for (int f = 0; f < nframes; ++f) {
+      in.p[f] = L > 0 ? frames[f].items[L] : nullptr;
+      out.p[f] = L + 1 < nrl ? frames[f].items[L + 1] : nullptr;
+    }
+    auto kern = L == 0 ? k_refit_level<true> : k_refit_level<false>;
+    kern<<<dim3(R.nblk, (unsigned)nframes), LV_C, 0, s>>>(R.blk.p, R.rec.p, R.wd.p, R.node.p, verts, leaf_tri, in, out,
+                                                          nodes, wide, root);
+    CC_LAUNCHED();
+  }
 }
 
 void Body::top_setup(int k, int l, hipStream_t s) {
@@ -788,19 +835,12 @@ void Body::refit_frames(int F, const int* ks, const int* ls, hipStream_t s, bool
     wide.p[f] = W ? S.wide.p : nullptr;
   }
   if (nrl) {
-    for (int L = 0; L < nrl; ++L) {
-      const RefitLevel& R = rl[L];
-      PF<const float> in{};
-      PF<float> out{};
-      for (int f = 0; f < F; ++f) {
-        in.p[f] = L > 0 ? lane[ls[f]].ritem[L].p : nullptr;
-        out.p[f] = L + 1 < nrl ? lane[ls[f]].ritem[L + 1].p : nullptr;
-      }
-      auto kern = L == 0 ? k_refit_level<true> : k_refit_level<false>;
-      kern<<<dim3(R.nblk, (unsigned)F), LV_C, 0, s>>>(R.blk.p, R.rec.p, R.wd.p, R.node.p, verts, leaf_tri.p, depth, in,
-                                                      out, nodes, wide, root);
-      CC_LAUNCHED();
+    RefitFrame fr[MAX_FRAMES];
+    for (int f = 0; f < F; ++f) {
+      fr[f] = RefitFrame{verts.p[f], {}, nodes.p[f], wide.p[f], root.p[f]};
+      for (int L = 1; L < nrl; ++L) fr[f].items[L] = lane[ls[f]].ritem[L].p;
     }
+    launch_refit_levels(rl, nrl, leaf_tri.p, fr, F, s);
     return;
   }
   k_refit_chunks<<<dim3(grid_for(m, RC_CHUNK), (unsigned)F), RC_THREADS, 0, s>>>(
