@@ -491,10 +491,11 @@ int cc_sim_create(const cc_cloth_desc* cloth, const cc_body_desc* bd, const cc_p
       // 13.6 / 14.9 at 50,688, 44.6 / 48.2 against 43.3 / 47.4 at 501,120).  A
       // rebuilt body, a chain of 14 launches, fills two (two of three against
       // two of four and one of four: 14.8, 13.5, 16.6 at 5,760; 20.6, 20.8, 25.4
-      // at 50,688) and from some 100,000 triangles on three (two, three lanes of
-      // four: 35.6, 32.9 at 146,400; 95.0, 90.2 at 501,120).
+      // at 50,688; 38.1, 35.6, 46.0 at 146,400; 98.8, 95.0, 109 at 501,120).  A
+      // third is quicker for large bodies only while no other simulator's
+      // streams share its hardware queue (32.9 or 43.1 at 146,400).
       const bool rebuilt = bd->mode == CC_BODY_REBUILD;
-      int lanes = rebuilt ? (bd->nf > 100000 ? 3 : 2) : 1;
+      int lanes = rebuilt ? 2 : 1;
       if (const char* e = std::getenv("CC_BODY_LANES")) lanes = std::atoi(e);
       CC_REQUIRE(lanes >= 1 && lanes <= MAX_LANES, "cc_sim_create: CC_BODY_LANES must be 1..4");
       if (const char* e = std::getenv("CC_GRAPH_STEPS")) S.graph_steps = std::atoi(e);
