@@ -77,9 +77,8 @@ struct Sim {
   // Graphs of graph_steps steps, per slot of the first frame and state
   // parity (captured when first needed).
   // Steps per block (even; a moving body's ring holds 2 * graph_steps
-  // poses).  24 = 8 updates on each of three lanes: at the 501k-triangle
-  // refitted body, 52.4 us per step against 54.5 with 16 (6/5/5 updates:
-  // the step stream waits for the lane with six) and 53.8 with 32.
+  // poses).  24 is three chains of four frames on each of two lanes; measured with three lanes of one frame at the 501k-triangle refitted
+  // body: 52.4 us per step against 54.5 with 16 and 53.8 with 32.
   int graph_steps = 24;
   hipGraphExec_t gmain[MAX_SLOTS][2] = {};
   // update lanes (moving bodies): streams and the events that order them

@@ -483,19 +483,21 @@ int cc_sim_create(const cc_cloth_desc* cloth, const cc_body_desc* bd, const cc_p
       mp.pz = bd->pivot[2];
       mp.dt = (double)params->dt;
       // Update lanes and frames per chain of launches: four frames share each
-      // launch, which is bound by latency far more than by their work.  A
-      // refitted body, an update of five launches, keeps to one lane: more run
-      // into one another and into the step (us per step of a 480-step run / of
-      // one call per frame, three lanes of three frames against one of four:
-      // 12.4 / 12.1 against 10.5 / 11.5 at 5,760 triangles, 15.3 / 15.5 against
-      // 13.6 / 14.9 at 50,688, 44.6 / 48.2 against 43.3 / 47.4 at 501,120).  A
-      // rebuilt body, a chain of 14 launches, fills two (two of three against
-      // two of four and one of four: 14.8, 13.5, 16.6 at 5,760; 20.6, 20.8, 25.4
-      // at 50,688; 38.1, 35.6, 46.0 at 146,400; 98.8, 95.0, 109 at 501,120).  A
-      // third is quicker for large bodies only while no other simulator's
-      // streams share its hardware queue (32.9 or 43.1 at 146,400).
-      const bool rebuilt = bd->mode == CC_BODY_REBUILD;
-      int lanes = rebuilt ? 2 : 1;
+      // launch, which is bound by latency far more than by their work, and a
+      // body takes two lanes.  A refitted body, an update of five launches, would
+      // be a little quicker with one (us per step of a 480-step run / of one
+      // call per frame, one lane / two, four frames each / three of three:
+      // 10.0, 12.1 / 10.7, 11.0 / 13.9, 14.5 at 5,760 triangles; 13.1, 13.4 /
+      // 13.8, 14.0 / 17.2, 17.7 at 50,688; 41.5, 41.5 / 41.8, 42.1 / 48.9, 49.7 at
+      // 501,120), but where that lane shares a hardware queue with its own step
+      // stream, as a process's second simulator's may, its updates and steps run
+      // one after another (5,760: 13.9, 19.6; 501,120: 58.7 per call against
+      // 42.5 with two).  A rebuilt body, a chain of 14 launches, fills two (two of
+      // three against two of four and one of four: 14.8, 13.5, 16.6 at 5,760; 20.6,
+      // 20.8, 25.4 at 50,688; 38.1, 35.6, 46.0 at 146,400; 98.8, 95.0, 109 at
+      // 501,120).  A third is quicker for large bodies only while no other
+      // simulator's streams share its hardware queue (32.9 or 43.1 at 146,400).
+      int lanes = 2;
       if (const char* e = std::getenv("CC_BODY_LANES")) lanes = std::atoi(e);
       CC_REQUIRE(lanes >= 1 && lanes <= MAX_LANES, "cc_sim_create: CC_BODY_LANES must be 1..4");
       if (const char* e = std::getenv("CC_GRAPH_STEPS")) S.graph_steps = std::atoi(e);
