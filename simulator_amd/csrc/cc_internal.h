@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <stdexcept>
@@ -121,6 +122,7 @@ struct Stage {
   char* p = nullptr;
   size_t n = 0;
   DBuf<int32_t> spill;
+  size_t least = 0;   // bytes of an allocation at least
   Stage() = default;
   Stage(const Stage&) = delete;
   Stage& operator=(const Stage&) = delete;
@@ -129,6 +131,7 @@ struct Stage {
   }
   char* host(size_t bytes) {
     if (bytes <= n) return p;
+    bytes = std::max(bytes, least);
     if (p) (void)hipHostFree(p);
     p = nullptr;
     n = 0;

@@ -542,6 +542,8 @@ void launch_spill_status(const int32_t* tail, uint32_t* status, hipStream_t s);
 // three arrays of vec3 (any may be NULL), and the collision query of n host
 // points (returns its traversal faults), both synchronous on s; n vec3 to two
 // device arrays, asynchronous: the caller holds st.m until s has done it.
+// state_bytes: the pinned memory that reading n states takes.
+size_t state_bytes(uint32_t n);
 void read_state(Stage& st, const float* state, const float* contact, uint32_t n, float* x_cur, float* x_prev,
                 float* contact_n, hipStream_t s);
 void write_points(Stage& st, const float* src, uint32_t n, float* a, float* b, hipStream_t s);

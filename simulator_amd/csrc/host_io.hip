@@ -21,6 +21,7 @@ namespace cc {
 // and the 15.7 MB of its spill area, the most a handle keeps (two chunks of
 // pinned memory)
 constexpr uint32_t IO_CHUNK = 65536;
+constexpr size_t STATE_BYTES = 36;   // of a vertex: x_cur, x_prev, contact normal
 
 // {x_cur, x_prev} records and normals to three arrays of vec3, one after the
 // other.  Bound by the link to the host (36 bytes per vertex).
@@ -44,6 +45,9 @@ __global__ __launch_bounds__(256) void k_points_in(const float* __restrict__ in,
 }
 
 namespace {
+// pinned memory of a chunk (two alternate where there are several)
+size_t chunk_bytes(uint32_t n, size_t bytes) { return (bytes * std::min(n, IO_CHUNK) + 255) / 256 * 256; }
+
 // Chunks of [0, n): fill(o, k, h) before a chunk's launch(o, k, h), drain(o, k,
 // h) after it has run, h the chunk's pinned memory (`bytes` per item).  Returns
 // with every chunk drained, or, when there is nothing to drain, with the last
@@ -55,7 +59,7 @@ template <class Fill, class Launch, class Drain>
 void by_chunks(Stage& st, uint32_t n, size_t bytes, hipStream_t s, Fill&& fill, Launch&& launch, Drain&& drain) {
   constexpr bool wait = !std::is_same_v<std::decay_t<Drain>, Nothing>;
   const uint32_t c = std::min(n, IO_CHUNK), chunks = (n + c - 1) / c;
-  const size_t half = (bytes * c + 255) / 256 * 256;
+  const size_t half = chunk_bytes(n, bytes);
   char* h = st.host(half * std::min(chunks, 2u));
   if (chunks == 1) {
     fill(0u, n, h);
@@ -81,11 +85,13 @@ void by_chunks(Stage& st, uint32_t n, size_t bytes, hipStream_t s, Fill&& fill, 
 }
 }  // namespace
 
+size_t state_bytes(uint32_t n) { return chunk_bytes(n, STATE_BYTES) * (n > IO_CHUNK ? 2 : 1); }
+
 void read_state(Stage& st, const float* state, const float* contact, uint32_t n, float* x_cur, float* x_prev,
                 float* contact_n, hipStream_t s) {
   std::lock_guard<std::mutex> g(st.m);
   by_chunks(
-      st, n, 36, s, Nothing{},
+      st, n, STATE_BYTES, s, Nothing{},
       [&](uint32_t o, uint32_t k, char* h) {
         k_state_out<<<grid_for(k, 256), 256, 0, s>>>(state + 6 * (size_t)o, contact + 3 * (size_t)o, k,
                                                      reinterpret_cast<float*>(h));
