@@ -672,7 +672,7 @@ void BatchBodies::post(const BodyPass& P, int slot, hipStream_t s) {
   if (P.refit) {
     RefitFrame r{verts[slot].p, {}, nodes[slot].p, nullptr, root[slot].p};
     for (int L = 1; L < nrl; ++L) r.items[L] = ritem[L].p;
-    launch_refit_levels(rl, nrl, leaf_tri[slot].p, &r, 1, s);
+    launch_refit_levels(rl, nrl, leaf_tri[slot].p, nullptr, &r, 1, s);
   }
   const LvFrame f{keys.p, tris.p, boxes.p, leaf_tri[slot].p, {items[0].p, items[1].p}, {nitems[0].p, nitems[1].p},
                   nodes[slot].p, root[slot].p, leaf0[slot].p};

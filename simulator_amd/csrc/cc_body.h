@@ -162,7 +162,7 @@ constexpr int RL_MAX = 8;
 struct RefitGroup {
   uint32_t first, n, out0, rounds;   // first item, items, first item it leaves to the next level, rounds
   uint32_t v0, n0, body;             // its body's first vertex and node, and number (0 for a single body)
-  float depth;
+  float depth;                       // a batch's: its body's box depth (fixed)
 };
 struct RefitLevel {
   uint32_t nitems = 0, nblk = 0;
@@ -192,8 +192,10 @@ struct RefitFrame {
   float4* wide;              // or nullptr: the boxes go to the nodes
   float* root;
 };
-void launch_refit_levels(const RefitLevel* rl, int nrl, const uint4* leaf_tri, const RefitFrame* frames, int nframes,
-                         hipStream_t s);
+// depth: the box depth of a single body, as it is now (a batch's: nullptr, each
+// group holds its body's)
+void launch_refit_levels(const RefitLevel* rl, int nrl, const uint4* leaf_tri, const float* depth,
+                         const RefitFrame* frames, int nframes, hipStream_t s);
 
 // One frame of the body as the collision query reads it.
 struct Slot {

@@ -556,7 +556,8 @@ template <bool LEAVES>
 __global__ __launch_bounds__(LV_C) void k_refit_level(const RefitGroup* __restrict__ blk,
                                                       const uint2* __restrict__ rec, const uint4* __restrict__ wdst,
                                                       const uint32_t* __restrict__ node_of, PF<const float> verts_f,
-                                                      const uint4* __restrict__ leaf_tri, PF<const float> in_f, PF<float> out_f, PF<Node> nodes_f,
+                                                      const uint4* __restrict__ leaf_tri, bool one, float depth,
+                                                      PF<const float> in_f, PF<float> out_f, PF<Node> nodes_f,
                                                       PF<float4> wide_f, PF<float> root_f) {
   __shared__ float2 U[2][LV_C][3];
   const RefitGroup b = blk[blockIdx.x];
@@ -571,8 +572,9 @@ __global__ __launch_bounds__(LV_C) void k_refit_level(const RefitGroup* __restri
   if constexpr (LEAVES) {
     const uint4 t = leaf_tri[at];
     const float* __restrict__ verts = pick(verts_f) + 3 * (size_t)b.v0;
-    prim_box(ld3(verts + 3 * (size_t)t.x), ld3(verts + 3 * (size_t)t.y), ld3(verts + 3 * (size_t)t.z), b.depth, own.v,
-             own.v + 3);
+    // a single body's depth comes with the launch: its owner may change it
+    prim_box(ld3(verts + 3 * (size_t)t.x), ld3(verts + 3 * (size_t)t.y), ld3(verts + 3 * (size_t)t.z),
+             one ? depth : b.depth, own.v, own.v + 3);
   } else {
     const float* src = pick(in_f) + 6 * (size_t)at;
     for (int c = 0; c < 6; ++c) own.v[c] = src[c];
@@ -735,17 +737,15 @@ void RefitTables::upload(RefitLevel* rl, hipStream_t s) const {
 
 void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s) {
   RefitTables t;
-  RefitGroup g{};
-  g.depth = depth;
-  t.add(nd.data(), m, 0, g, dst);
+  t.add(nd.data(), m, 0, RefitGroup{}, dst);
   t.upload(rl, s);
   nrl = t.nlevels;
   for (int L = 1; L < nrl; ++L)
     for (int l = 0; l < nlanes * chain; ++l) lane[l].ritem[L].alloc(6 * (size_t)rl[L].nitems);
 }
 
-void launch_refit_levels(const RefitLevel* rl, int nrl, const uint4* leaf_tri, const RefitFrame* frames, int nframes,
-                         hipStream_t s) {
+void launch_refit_levels(const RefitLevel* rl, int nrl, const uint4* leaf_tri, const float* depth,
+                         const RefitFrame* frames, int nframes, hipStream_t s) {
   PF<const float> verts{};
   PF<Node> nodes{};
   PF<float> root{};
@@ -765,8 +765,9 @@ void launch_refit_levels(const RefitLevel* rl, int nrl, const uint4* leaf_tri, c
       out.p[f] = L + 1 < nrl ? frames[f].items[L + 1] : nullptr;
     }
     auto kern = L == 0 ? k_refit_level<true> : k_refit_level<false>;
-    kern<<<dim3(R.nblk, (unsigned)nframes), LV_C, 0, s>>>(R.blk.p, R.rec.p, R.wd.p, R.node.p, verts, leaf_tri, in, out,
-                                                          nodes, wide, root);
+    kern<<<dim3(R.nblk, (unsigned)nframes), LV_C, 0, s>>>(R.blk.p, R.rec.p, R.wd.p, R.node.p, verts, leaf_tri,
+                                                          depth != nullptr, depth ? *depth : 0.0f, in, out, nodes, wide,
+                                                          root);
     CC_LAUNCHED();
   }
 }
@@ -840,7 +841,7 @@ void Body::refit_frames(int F, const int* ks, const int* ls, hipStream_t s, bool
       fr[f] = RefitFrame{verts.p[f], {}, nodes.p[f], wide.p[f], root.p[f]};
       for (int L = 1; L < nrl; ++L) fr[f].items[L] = lane[ls[f]].ritem[L].p;
     }
-    launch_refit_levels(rl, nrl, leaf_tri.p, fr, F, s);
+    launch_refit_levels(rl, nrl, leaf_tri.p, &depth, fr, F, s);
     return;
   }
   k_refit_chunks<<<dim3(grid_for(m, RC_CHUNK), (unsigned)F), RC_THREADS, 0, s>>>(
