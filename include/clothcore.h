@@ -428,7 +428,8 @@ int cc_sim_get_timing(cc_sim* sim, cc_timing* out);
    reference, whose safe_cuda prints an error and continues, common.h:4-10).
    After `count` further successful operations of the kind, the next one
    fails as if the runtime had failed it, and the switch is off again:
-   CC_FAULT_ALLOC a device (or pinned host) allocation -> CC_ERR_ALLOC,
+   CC_FAULT_ALLOC a device (or pinned host) allocation -> CC_ERR_ALLOC (with
+   the runtime's last error set, as a real failure sets it),
    CC_FAULT_LAUNCH the check after a kernel launch -> CC_ERR_HIP (the
    kernel itself was launched and runs).  count < 0 turns the kind off.
    Process-wide.  A call that failed this way leaves its object usable

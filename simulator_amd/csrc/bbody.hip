@@ -544,7 +544,7 @@ void BatchBodies::init(const cc_body_desc* bodies, const cc_params* params, cons
   motion.alloc((size_t)BB_FRAMES * nb * BB_MF);
   motion.zero(s);
   for (int q = 0; q < 2; ++q) {
-    if (fault_now(FAULT_ALLOC)) throw Error(CC_ERR_ALLOC, "hipHostMalloc: injected failure (cc_fault_inject)");
+    if (alloc_fault_now()) alloc_failed("hipHostMalloc: injected failure (cc_fault_inject)");
     CC_HIP(hipHostMalloc((void**)&h_motion[q], (size_t)BB_FRAMES * nb * BB_MF * sizeof(float), hipHostMallocDefault));
     std::memset(h_motion[q], 0, (size_t)BB_FRAMES * nb * BB_MF * sizeof(float));
     CC_HIP(hipEventCreate(&ev_motion[q]));

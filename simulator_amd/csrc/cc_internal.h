@@ -49,6 +49,14 @@ inline bool fault_now(int kind) {
   return false;
 }
 
+// An injected allocation failure leaves the runtime's last error set, as a real
+// one does (the runtime refuses an allocation without a result).
+inline bool alloc_fault_now() {
+  if (!fault_now(FAULT_ALLOC)) return false;
+  (void)hipMalloc(static_cast<void**>(nullptr), 16);
+  return true;
+}
+
 // The check after a kernel launch (and where a fault is injected).
 #define CC_LAUNCHED()                                                                       \
   do {                                                                                      \
@@ -79,6 +87,13 @@ int guard(F&& f) {
   }
 }
 
+// A failed allocation: the caller may go on without it, so the runtime's last
+// error is cleared here as CC_HIP does.
+[[noreturn]] inline void alloc_failed(const std::string& msg) {
+  (void)hipGetLastError();
+  throw Error(CC_ERR_ALLOC, msg);
+}
+
 // Device buffer owning a hipMalloc'd allocation.
 template <class T>
 struct DBuf {
@@ -97,11 +112,11 @@ struct DBuf {
     if (count == n && p) return;
     release();
     if (count == 0) return;
-    if (fault_now(FAULT_ALLOC)) throw Error(CC_ERR_ALLOC, "hipMalloc: injected failure (cc_fault_inject)");
+    if (alloc_fault_now()) alloc_failed("hipMalloc: injected failure (cc_fault_inject)");
     hipError_t e = hipMalloc(&p, count * sizeof(T));
     if (e != hipSuccess) {
       p = nullptr;
-      throw Error(CC_ERR_ALLOC, std::string("hipMalloc failed: ") + hipGetErrorString(e));
+      alloc_failed(std::string("hipMalloc failed: ") + hipGetErrorString(e));
     }
     n = count;
   }
@@ -135,11 +150,11 @@ struct Stage {
     if (p) (void)hipHostFree(p);
     p = nullptr;
     n = 0;
-    if (fault_now(FAULT_ALLOC)) throw Error(CC_ERR_ALLOC, "hipHostMalloc: injected failure (cc_fault_inject)");
+    if (alloc_fault_now()) alloc_failed("hipHostMalloc: injected failure (cc_fault_inject)");
     const hipError_t e = hipHostMalloc((void**)&p, bytes, hipHostMallocDefault);
     if (e != hipSuccess) {
       p = nullptr;
-      throw Error(CC_ERR_ALLOC, std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
+      alloc_failed(std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
     }
     n = bytes;
     return p;

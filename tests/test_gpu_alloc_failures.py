@@ -1,0 +1,54 @@
+"""A failed allocation is reported once (CC_ERR_ALLOC) and leaves nothing
+behind: the runtime keeps the error of its last failed call until it is read,
+and the next launch check on the thread must not find it.  The requests here
+are refused by the runtime itself (more memory than any card has) or made to
+fail by cc_fault_inject, which leaves the runtime's error set like a real
+failure."""
+import numpy as np
+import pytest
+
+from simulator_amd import _lib as L
+from simulator_amd import scene as S
+from simulator_amd.adjoint import Adjoint
+from simulator_amd.simulator import Simulator
+
+pytestmark = pytest.mark.gpu
+
+
+def refused(fn):
+    with pytest.raises(L.ClothCoreError) as e:
+        fn()
+    assert e.value.code == L.CC_ERR_ALLOC, str(e.value)
+
+
+def test_a_refused_request_leaves_no_error(gpu):
+    sim, ref = (Simulator.from_scene(S.small(side=16)) for _ in range(2))
+    for _ in range(2):
+        refused(lambda: Adjoint(sim, 2**31, 1))          # 13 TB of checkpoints
+        for s in (sim, ref):
+            s.simulate(1)
+            s.check_finite()
+    for x, y in zip(sim.get_state(), ref.get_state()):
+        np.testing.assert_array_equal(x, y)
+    sim.close()
+    ref.close()
+
+
+def test_an_injected_failure_leaves_no_error(gpu):
+    sim, ref = (Simulator.from_scene(S.small(side=16)) for _ in range(2))
+    pts = (np.random.default_rng(0).uniform(-0.4, 0.4, size=(500, 3)) + [0.5, 0.5, 0]).astype(np.float32)
+    want = ref.collide_points(pts)
+    for k in range(2):                                   # the spill area, the pinned memory
+        L.fault_inject(L.CC_FAULT_ALLOC, k)
+        try:
+            refused(lambda: sim.collide_points(pts))
+        finally:
+            L.fault_inject(L.CC_FAULT_ALLOC, -1)
+        for s in (sim, ref):
+            s.simulate(1)
+        for x, y in zip(sim.get_state(), ref.get_state()):
+            np.testing.assert_array_equal(x, y)
+    for x, y in zip(sim.collide_points(pts), want):
+        np.testing.assert_array_equal(x, y)
+    sim.close()
+    ref.close()
