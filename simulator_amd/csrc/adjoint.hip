@@ -434,6 +434,36 @@ static void check_symmetric(const Sim& S) {
     }
 }
 
+// The buffers of a rollout of nsteps steps: all its states, or checkpoints.
+static void alloc_adj(Adj& A, Sim& S, uint32_t nsteps, uint32_t ckpt_every, bool keep) {
+  A.S = &S;
+  A.n = S.n;
+  A.nsteps = nsteps;
+  A.keep = keep;
+  A.ckpt = keep ? nsteps : std::min(ckpt_every, nsteps);
+  A.nck = (uint32_t)(((size_t)nsteps + A.ckpt - 1) / A.ckpt);
+  A.nblk = grid_for(S.n, ADJ_THREADS);
+  const size_t n3 = 3 * (size_t)S.n, n6 = 6 * (size_t)S.n;
+  A.seg_state.alloc(((size_t)A.ckpt + 1) * n6);
+  A.seg_contact.alloc(((size_t)A.ckpt + 1) * n3);
+  if (!keep) {
+    for (int b = 0; b < 2; ++b) A.st[b].alloc(n6);
+    A.contact.alloc(n3);
+    A.ck_state.alloc(A.nck * n6);
+    A.ck_contact.alloc(A.nck * n3);
+  }
+  A.lp.alloc(n3);
+  A.lq.alloc(n3);
+  for (int b = 0; b < 2; ++b) {
+    A.lf[b].alloc(n3);
+    A.locp[b].alloc(n3);
+    A.locq[b].alloc(n3);
+  }
+  A.part.alloc((size_t)A.ckpt * grid_for(S.n, 64) * NPARAM);
+  A.acc.alloc(NPARAM * (size_t)A.nblk);
+  A.out.alloc(NPARAM);
+}
+
 }  // namespace cc
 
 using namespace cc;
@@ -452,45 +482,18 @@ int cc_adj_create(cc_sim* sim, uint32_t nsteps, uint32_t ckpt_every, cc_adj** ou
     *out = nullptr;
     CC_HIP(hipDeviceSynchronize());
     check_symmetric(S);
+    // Every state where that takes little memory; checkpoints otherwise, also
+    // when any part of that memory is not to be had.
+    const size_t keep_bytes = ((size_t)nsteps + 1) * 9 * S.n * sizeof(float);
     std::unique_ptr<cc_adj> h(new cc_adj);
-    Adj& A = h->a;
-    A.S = &S;
-    A.n = S.n;
-    A.nsteps = nsteps;
-    A.ckpt = std::min(ckpt_every, nsteps);
-    A.nck = (nsteps + A.ckpt - 1) / A.ckpt;
-    A.nblk = grid_for(S.n, ADJ_THREADS);
-    const size_t n3 = 3 * (size_t)S.n, n6 = 6 * (size_t)S.n;
-    // Every state where that takes little memory, checkpoints otherwise (also
-    // when that memory is not to be had).
-    if (((size_t)nsteps + 1) * (n6 + n3) * sizeof(float) <= ADJ_KEEP_BYTES) try {
-        A.seg_state.alloc(((size_t)nsteps + 1) * n6);
-        A.seg_contact.alloc(((size_t)nsteps + 1) * n3);
-        A.keep = true;
-        A.ckpt = nsteps;
-        A.nck = 1;
-      } catch (const Error& e) {
-        if (e.code != CC_ERR_ALLOC) throw;
-        A.seg_state.release();
-      }
-    if (!A.keep) {
-      for (int b = 0; b < 2; ++b) A.st[b].alloc(n6);
-      A.contact.alloc(n3);
-      A.ck_state.alloc(A.nck * n6);
-      A.ck_contact.alloc(A.nck * n3);
-      A.seg_state.alloc((A.ckpt + 1) * n6);
-      A.seg_contact.alloc((A.ckpt + 1) * n3);
+    try {
+      alloc_adj(h->a, S, nsteps, ckpt_every, keep_bytes <= ADJ_KEEP_BYTES);
+    } catch (const Error& e) {
+      if (e.code != CC_ERR_ALLOC || !h->a.keep) throw;
+      h.reset();           // the first attempt's memory goes before the second
+      h.reset(new cc_adj);
+      alloc_adj(h->a, S, nsteps, ckpt_every, false);
     }
-    A.lp.alloc(n3);
-    A.lq.alloc(n3);
-    for (int b = 0; b < 2; ++b) {
-      A.lf[b].alloc(n3);
-      A.locp[b].alloc(n3);
-      A.locq[b].alloc(n3);
-    }
-    A.part.alloc((size_t)A.ckpt * grid_for(S.n, 64) * NPARAM);
-    A.acc.alloc(NPARAM * (size_t)A.nblk);
-    A.out.alloc(NPARAM);
     *out = h.release();
   });
 }

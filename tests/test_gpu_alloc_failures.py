@@ -52,3 +52,28 @@ def test_an_injected_failure_leaves_no_error(gpu):
         np.testing.assert_array_equal(x, y)
     sim.close()
     ref.close()
+
+
+def test_a_gradient_falls_back_wherever_the_kept_states_leave_too_little(gpu):
+    """The first allocation that fails, whichever it is, sends the creation to
+    checkpoints; the gradient is the same."""
+    sc = S.small(side=12, y0=0.803)
+    sim = Simulator.from_scene(sc)
+    g = np.random.default_rng(1).normal(size=(sc.n, 3)).astype(np.float32)
+
+    def gradient(adj):
+        x = adj.forward(sc.pos, None, [900.0, 450.0, 90.0, -0.03, 1.01])
+        out = (x, *adj.backward(g))
+        adj.close()
+        return out
+
+    want = gradient(Adjoint(sim, 17, 5))
+    for k in range(13):                                  # a creation that keeps every state makes 13 allocations
+        L.fault_inject(L.CC_FAULT_ALLOC, k)
+        try:
+            adj = Adjoint(sim, 17, 5)
+        finally:
+            L.fault_inject(L.CC_FAULT_ALLOC, -1)
+        for a, b in zip(gradient(adj), want):
+            np.testing.assert_array_equal(a, b)
+    sim.close()
