@@ -306,7 +306,11 @@ int cc_sim_set_stack_limit(cc_sim* sim, int limit);
 /* ------------------------------------------------------------------ body */
 
 /* Replace the body vertices (stride 3 floats, rest pose for the deformation)
-   and rebuild the LBVH from them. */
+   and rebuild the LBVH from them.  Where that fails part way (here or in
+   cc_bvh_rebuild), a static or refitted body whose tree is not whole is
+   refused by steps and queries (CC_ERR_INVALID) until one of the two
+   succeeds; a static body that lacks only its four-wide form is walked in
+   the binary one. */
 int cc_body_set_vertices(cc_sim* sim, const float* verts3);
 /* Current (deformed) body vertices, vec3. */
 int cc_body_get_vertices(cc_sim* sim, float* verts3);

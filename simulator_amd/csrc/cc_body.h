@@ -288,6 +288,10 @@ struct Body {
   uint32_t wide_stack = 0;          // most entries a traversal can defer
   bool wide_enabled = true;
   bool grouped = false;
+  // A static or refitted body whose tree a failed rebuild left half made (of
+  // several slots: in some of them): it is not walked or refitted, but may be
+  // rebuilt.
+  bool torn = false;
   DBuf<uint4> w_src;
   DBuf<int4> w_link;
   DBuf<uint2> w_dst;                // [2 * (m - 1)] binary child slot -> {wide entry (record * 4 +
@@ -312,7 +316,12 @@ struct Body {
   // lane whose topology a refit on lane l reads
   Lane& topo(int l) { return mode == CC_BODY_REBUILD ? lane[l] : lane[0]; }
 
+  void require_whole() const {
+    CC_REQUIRE(!torn, "body: its last rebuild failed; replace its vertices or rebuild it");
+  }
+
   BvhView view(int k) const {
+    require_whole();
     BvhView v;
     v.nodes = slot[k].nodes.p;
     v.leaf_tri = mode == CC_BODY_REBUILD ? slot[k].leaf_tri.p : leaf_tri.p;
@@ -333,14 +342,15 @@ struct Body {
             const cc_capsules* caps, const MotionParams& mp, int slots, int lanes, hipStream_t s,
             int chain = 1, bool allow_bottom_up = true);
 
-  // A static body whose vertices its owner replaces: from here on its tree
+  // A static body whose vertices its owner replaces: from here on its
   // wide records are folded on the device after each build, as a rebuilt
-  // body's are (of 2..2^21 triangles; otherwise nothing changes).  The tree is the
+  // body's are (of 2..2^21 triangles; otherwise nothing changes), and until the
+  // first such build has folded them it has none.  The tree is the
   // same; the host layout of wide_setup (some 2 ms at 50,688 triangles: the
   // nodes copied to the host, laid out breadth-first and sorted, a dozen
   // buffers made) pays only for a body that stays, whose walk it makes 3%
   // shorter.
-  void rebuild_on_device(hipStream_t s);
+  void rebuild_on_device();
   void level_setup(hipStream_t s);    // work tables and scratch of the build by levels, lane 0..
 
   // launches, asynchronous on s
@@ -368,8 +378,8 @@ struct Body {
   // later refits write the boxes through w_dst.
   void wide_setup(int k, hipStream_t s);
   // the layout itself, from the nodes' host copy: child slot -> {entry, link}
-  // into dst (empty: the binary form stays)
-  void wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s);
+  // into dst; returns the number of records (0: the binary form stays)
+  uint32_t wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s);
   // the tables of a refit by levels
   void refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s);
   // Rebuilt bodies: the wide records of slots ks[q] from their binary trees

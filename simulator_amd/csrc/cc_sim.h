@@ -213,20 +213,26 @@ struct Sim {
 
   // A new tree over slot k's vertices, shared with the other slots of a
   // refitted body.  Captured blocks hold the body's views: they go where one
-  // changed (its four-wide records in another buffer).
+  // changed (its four-wide records in another buffer), and where a failure
+  // leaves it open which buffers are left.
   void rebuild_body(int k) {
-    std::vector<BvhView> before;
-    for (int q = 0; q < body.nslots; ++q) before.push_back(body.view(q));
-    body.rebuild_on_device(stream);
-    body.build(k, 0, stream);
-    body.share_topology(k, stream);
-    for (int q = 0; q < body.nslots; ++q) {
-      const BvhView v = body.view(q);
-      if (v.wide != before[q].wide || v.grouped != before[q].grouped) {
-        drop_graphs();
-        return;
-      }
+    std::vector<const float4*> before;
+    const uint32_t nwide = body.nwide;
+    const bool grouped = body.grouped;
+    for (int q = 0; q < body.nslots; ++q) before.push_back(body.slot[q].wide.p);
+    body.torn = body.mode == CC_BODY_STATIC || body.mode == CC_BODY_REFIT;
+    try {
+      body.rebuild_on_device();
+      body.build(k, 0, stream);
+      body.share_topology(k, stream);
+    } catch (...) {
+      drop_graphs();
+      throw;
     }
+    body.torn = false;
+    bool same = !nwide == !body.nwide && grouped == body.grouped;
+    for (int q = 0; q < body.nslots; ++q) same = same && before[q] == body.slot[q].wide.p;
+    if (!same) drop_graphs();
   }
 
   hipGraphExec_t end_capture(int cur0) {

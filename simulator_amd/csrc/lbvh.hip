@@ -183,14 +183,11 @@ void Body::level_setup(hipStream_t s) {
   CC_HIP(hipStreamSynchronize(s));   // the tables' host copies end here
 }
 
-void Body::rebuild_on_device(hipStream_t s) {
+void Body::rebuild_on_device() {
   if (mode != CC_BODY_STATIC || !bottom_up || grouped) return;
-  slot[0].wide.alloc(8 * (size_t)(m - 1));
   w_src.release();
   w_link.release();
   w_dst.release();
-  nwide = m - 1;
-  wide_stack = STACK_LIMIT;
   grouped = true;
 }
 
@@ -301,10 +298,18 @@ void Body::build_frames(int F, const int* ks, const int* ls, hipStream_t s) {
   launch_sort(desc.p, sort_table, tris.p, sf, F, s);
   if (bottom_up) {                      // tree and boxes by levels
     build_levels(F, ks, ls, s);
-    if (grouped)
+    if (mode == CC_BODY_STATIC) torn = false;   // walked as it is until it has wide records
+    if (grouped && mode == CC_BODY_STATIC) {
+      nwide = 0;
+      slot[0].wide.alloc(8 * (size_t)(m - 1));
       fold_frames(F, ks, s);
-    else
+      nwide = m - 1;
+      wide_stack = STACK_LIMIT;
+    } else if (grouped) {
+      fold_frames(F, ks, s);
+    } else {
       wide_setup(ks[0], s);
+    }
     return;
   }
   const int k = ks[0], l = ls[0];
@@ -320,7 +325,8 @@ void Body::build_frames(int F, const int* ks, const int* ls, hipStream_t s) {
     return;
   }
   nwide = 0;             // a new topology: the wide table follows the refit
-  refit(k, l, s);
+  refit_frames(1, &k, &l, s);
+  if (mode == CC_BODY_STATIC) torn = false;
   wide_setup(k, s);
 }
 
@@ -345,6 +351,7 @@ void Body::update_frames(int F, const int* ks, const int* ls, const uint64_t* fr
     return;
   }
   CC_REQUIRE(F <= chain, "body: frames per chain");
+  require_whole();
   deform_frames(F, ks, frames, s);
   if (mode == CC_BODY_REFIT)
     refit_frames(F, ks, ls, s);

@@ -799,6 +799,7 @@ void Body::top_setup(int k, int l, hipStream_t s) {
 
 void Body::refit(int k, int l, hipStream_t s, bool binary) {
   if (mode == CC_BODY_NONE || m == 0) return;
+  require_whole();
   if (bottom_up && mode != CC_BODY_REFIT) {   // same keys, so the same tree; new boxes
     prim_boxes_of(k, l, s);
     build_levels(1, &k, &l, s);

@@ -898,7 +898,13 @@ int cc_sim_set_bvh_width(cc_sim* sim, int width) {
     Sim& S = sim->s;
     S.body.wide_enabled = width == 4;
     S.drop_graphs();
-    if (S.body.mode != CC_BODY_NONE) S.refresh_body();    // fold the current frame's boxes
+    if (S.body.mode == CC_BODY_NONE) return;
+    try {
+      S.refresh_body();    // fold the current frame's boxes
+    } catch (...) {
+      S.body.wide_enabled = false;    // its records may never have been folded
+      throw;
+    }
   });
 }
 

@@ -133,11 +133,12 @@ void Body::wide_setup(int k, hipStream_t s) {
   CC_HIP(hipMemcpyAsync(nd.data(), slot[k].nodes.p, nd.size() * sizeof(Node), hipMemcpyDeviceToHost, s));
   CC_HIP(hipStreamSynchronize(s));
   std::vector<uint2> dst;
-  wide_layout(k, nd, dst, s);
+  const uint32_t nw = wide_layout(k, nd, dst, s);
   if (mode == CC_BODY_REFIT && bottom_up) refit_setup(nd, dst, s);
+  nwide = nw;            // all of it is there
 }
 
-void Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s) {
+uint32_t Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s) {
   const uint32_t mi = m - 1;
   // Breadth-first over the kept binary nodes (the root, then the internal
   // entries of each kept node); wid maps a kept binary node to its record.
@@ -226,7 +227,7 @@ void Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& d
     link.push_back(lv);
   }
   // The traversal stack holds 64 entries; keep the binary form otherwise.
-  if (worst > 64) return;
+  if (worst > 64) return 0;
   // Renumber the records in the order of their binary nodes (Karras
   // indices; the root stays 0): the refit, which walks binary nodes in index
   // order, then writes each chunk's entries into a compact run of records.
@@ -261,14 +262,15 @@ void Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& d
   w_src.upload(src.data(), src.size(), s);
   w_link.upload(link.data(), link.size(), s);
   w_dst.upload(dst.data(), dst.size(), s);
-  nwide = (uint32_t)src.size();
+  const uint32_t nw = (uint32_t)src.size();
   wide_stack = worst;
-  for (int j = 0; j < nslots; ++j) slot[j].wide.alloc(8 * (size_t)nwide);
+  for (int j = 0; j < nslots; ++j) slot[j].wide.alloc(8 * (size_t)nw);
   // Slot k's records in full (links, empty entries, boxes); the other slots
   // get theirs from share_topology, and every refit rewrites the boxes.
-  k_fold_wide<<<grid_for(nwide, 256), 256, 0, s>>>(slot[k].nodes.p, w_src.p, w_link.p, nwide, slot[k].wide.p);
+  k_fold_wide<<<grid_for(nw, 256), 256, 0, s>>>(slot[k].nodes.p, w_src.p, w_link.p, nw, slot[k].wide.p);
   CC_LAUNCHED();
   CC_HIP(hipStreamSynchronize(s));
+  return nw;
 }
 
 }  // namespace cc
