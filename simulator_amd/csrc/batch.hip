@@ -173,9 +173,18 @@ struct Batch {
     if (bodies.moving) {
       CC_HIP(hipEventRecord(ev_fork, s));
       CC_HIP(hipStreamWaitEvent(side, ev_fork, 0));
-      launch(tile, blocks.p, nblocks, side);
-      CC_HIP(hipEventRecord(ev_join, side));
-      bodies.launch(bodies.step, k, nxt, s);
+      try {
+        launch(tile, blocks.p, nblocks, side);
+        CC_HIP(hipEventRecord(ev_join, side));
+        bodies.launch(bodies.step, k, nxt, s);
+      } catch (...) {
+        // the branch is joined all the same: a capture cannot end without it, and
+        // what the caller puts on s next has to come after it
+        (void)hipEventRecord(ev_join, side);
+        (void)hipStreamWaitEvent(s, ev_join, 0);
+        (void)hipGetLastError();
+        throw;
+      }
       CC_HIP(hipStreamWaitEvent(s, ev_join, 0));
     } else {
       launch(tile, blocks.p, nblocks, s);
@@ -185,24 +194,16 @@ struct Batch {
 
   hipGraphExec_t capture() {
     const int cur0 = cur;
-    hipGraph_t graph = nullptr;
     CC_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
       for (int k = 0; k < GRAPH_STEPS_B; ++k) one_step(k, stream);
     } catch (...) {
       cur = cur0;
-      hipGraph_t junk = nullptr;
-      (void)hipStreamEndCapture(stream, &junk);
-      if (junk) (void)hipGraphDestroy(junk);
+      drop_capture(stream);
       throw;
     }
     cur = cur0;
-    CC_HIP(hipStreamEndCapture(stream, &graph));
-    hipGraphExec_t g = nullptr;
-    hipError_t e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (e != hipSuccess) throw Error(CC_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-    return g;
+    return finish_capture(stream);
   }
 
   // Step g collides every cloth with its body's pose of frame g (the single

@@ -198,6 +198,27 @@ struct Events {
   hipEvent_t operator[](int i) const { return e[i].h; }
 };
 
+// The graph of a capture on s, ready to launch; and the end of a capture whose
+// work failed, with whatever error that gives.
+inline hipGraphExec_t finish_capture(hipStream_t s) {
+  hipGraph_t graph = nullptr;
+  CC_HIP(hipStreamEndCapture(s, &graph));
+  hipGraphExec_t g = nullptr;
+  const hipError_t e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(graph);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    throw Error(CC_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+  }
+  return g;
+}
+inline void drop_capture(hipStream_t s) {
+  hipGraph_t junk = nullptr;
+  (void)hipStreamEndCapture(s, &junk);
+  if (junk) (void)hipGraphDestroy(junk);
+  (void)hipGetLastError();
+}
+
 // ------------------------------------------------------------ physics pod
 struct Params {
   float dt, mass, gx, gy, gz, damp, kd, k0, k1, k2, rest_scale, eps, box_depth;

@@ -235,17 +235,6 @@ struct Sim {
     if (!same) drop_graphs();
   }
 
-  hipGraphExec_t end_capture(int cur0) {
-    cur = cur0;
-    hipGraph_t graph = nullptr;
-    CC_HIP(hipStreamEndCapture(stream, &graph));
-    hipGraphExec_t g = nullptr;
-    hipError_t e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (e != hipSuccess) throw Error(CC_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-    return g;
-  }
-
   template <class F>
   hipGraphExec_t capture(F&& body_of_graph) {
     const int cur0 = cur;
@@ -254,12 +243,11 @@ struct Sim {
       body_of_graph();
     } catch (...) {
       cur = cur0;
-      hipGraph_t junk = nullptr;
-      (void)hipStreamEndCapture(stream, &junk);
-      if (junk) (void)hipGraphDestroy(junk);
+      drop_capture(stream);
       throw;
     }
-    return end_capture(cur0);
+    cur = cur0;
+    return finish_capture(stream);
   }
 
   // graph_steps fused steps from a frame in slot k0, starting at the current
