@@ -503,7 +503,14 @@ int cc_sim_create(const cc_cloth_desc* cloth, const cc_body_desc* bd, const cc_p
       if (const char* e = std::getenv("CC_GRAPH_STEPS")) S.graph_steps = std::atoi(e);
       CC_REQUIRE(S.graph_steps >= 2 && S.graph_steps % 2 == 0 && 2 * S.graph_steps <= MAX_SLOTS,
                  "cc_sim_create: CC_GRAPH_STEPS must be even, 2..MAX_SLOTS/2");
-      int chain = MAX_FRAMES;
+      // single steps issue poses up to four frames per lane ahead
+      // (measured at the 501k-triangle refitted body with two-frame
+      // chains: 32.9 us per single step against 33.6 two frames per lane
+      // ahead and 33.0 six)
+      S.lookahead = 4 * lanes;
+      if (const char* e = std::getenv("CC_LOOKAHEAD")) S.lookahead = std::atoi(e);
+      // three frames a chain where four do not fit into the ring
+      int chain = S.lookahead + MAX_FRAMES * lanes + Sim::GO_EVERY < 2 * S.graph_steps ? MAX_FRAMES : MAX_FRAMES - 1;
       if (const char* e = std::getenv("CC_BUILD_FRAMES")) chain = std::atoi(e);
       CC_REQUIRE(chain >= 1 && chain <= MAX_FRAMES, "cc_sim_create: CC_BUILD_FRAMES must be 1..4");
       // 0: rebuilt bodies of any size take the Karras searches and the
@@ -528,12 +535,6 @@ int cc_sim_create(const cc_cloth_desc* cloth, const cc_body_desc* bd, const cc_p
         }
         CC_HIP(hipEventCreate(&S.ev_go));
         for (int k = 0; k < S.body.nslots; ++k) CC_HIP(hipEventCreate(&S.ev_pose[k]));
-        // single steps issue poses up to four frames per lane ahead
-        // (measured at the 501k-triangle refitted body with two-frame
-        // chains: 32.9 us per single step against 33.6 two frames per lane
-        // ahead and 33.0 six)
-        S.lookahead = 4 * S.body.nlanes;
-        if (const char* e = std::getenv("CC_LOOKAHEAD")) S.lookahead = std::atoi(e);
         // single steps of a chained body issue up to nlanes * chain - 1
         // frames past the lookahead
         CC_REQUIRE(S.lookahead >= 1 &&
