@@ -22,6 +22,10 @@ namespace cc {
 // pinned memory)
 constexpr uint32_t IO_CHUNK = 65536;
 constexpr size_t STATE_BYTES = 36;   // of a vertex: x_cur, x_prev, contact normal
+constexpr uint32_t chunks_of(uint32_t n) { return n / IO_CHUNK + (n % IO_CHUNK ? 1 : 0); }
+static_assert(chunks_of(1) == 1 && chunks_of(IO_CHUNK) == 1 && chunks_of(IO_CHUNK + 1) == 2 &&
+                  chunks_of(~0u - IO_CHUNK) == (1u << 16) - 1 && chunks_of(~0u) == 1u << 16,
+              "every count of points is covered, also those a chunk short of 2^32");
 
 // {x_cur, x_prev} records and normals to three arrays of vec3, one after the
 // other.  Bound by the link to the host (36 bytes per vertex).
@@ -58,7 +62,7 @@ struct Nothing {
 template <class Fill, class Launch, class Drain>
 void by_chunks(Stage& st, uint32_t n, size_t bytes, hipStream_t s, Fill&& fill, Launch&& launch, Drain&& drain) {
   constexpr bool wait = !std::is_same_v<std::decay_t<Drain>, Nothing>;
-  const uint32_t c = std::min(n, IO_CHUNK), chunks = (n + c - 1) / c;
+  const uint32_t c = std::min(n, IO_CHUNK), chunks = chunks_of(n);
   const size_t half = chunk_bytes(n, bytes);
   char* h = st.host(half * std::min(chunks, 2u));
   if (chunks == 1) {
