@@ -273,14 +273,16 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_step(uint32_t n, const uint
     const float ks0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k0)));
     const float ks1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k1)));
     const float ks2 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.k2)));
-    const uint32_t r0 = EW ? i * (uint32_t)EW : r0raw & ROW_MASK, r1 = EW ? r0 + EW : r1raw & ROW_MASK;
+    // places in this vertex's own records (EW), or in all of them
+    const uint2* __restrict__ recs = EW ? rec + (size_t)i * EW : rec;
+    const uint32_t r0 = EW ? 0u : r0raw & ROW_MASK, r1 = EW ? (uint32_t)EW : r1raw & ROW_MASK;
     for (uint32_t k0 = r0; PRE || k0 < r1; k0 += NB * LANES) {
       bool real[NB];
       float sj[NB][6], lj[NB][3];
 #pragma unroll
       for (int k = 0; k < NB; ++k) {
         const uint32_t at = k0 + (uint32_t)(e * NB + k);
-        if (!PRE) er[k] = rec[EW ? at : min(at, r1 - 1)];
+        if (!PRE) er[k] = recs[EW ? at : min(at, r1 - 1)];
         real[k] = EW ? (er[k].x & PAD_TYPE) != PAD_TYPE : at < r1;
         if (!EW && !real[k]) er[k] = make_uint2(i | PAD_TYPE, 0u);
       }
