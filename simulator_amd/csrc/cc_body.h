@@ -296,6 +296,7 @@ struct Body {
   DBuf<int4> w_link;
   DBuf<uint2> w_dst;                // [2 * (m - 1)] binary child slot -> {wide entry (record * 4 +
                                     // entry), its link}, entry ~0 for the slots of folded nodes
+                                    // (refits by chunks)
 
   RefitLevel rl[RL_MAX];            // a refitted body built by levels
   int nrl = 0;
@@ -378,10 +379,10 @@ struct Body {
   // later refits write the boxes through w_dst.
   void wide_setup(int k, hipStream_t s);
   // the layout itself, from the nodes' host copy: child slot -> {entry, link}
-  // into dst; returns the number of records (0: the binary form stays)
-  uint32_t wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s);
+  // into dst where a refit needs it; returns the number of records (0: the binary form stays)
+  uint32_t wide_layout(int k, const Node* nd, std::vector<uint2>& dst, hipStream_t s);
   // the tables of a refit by levels
-  void refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s);
+  void refit_setup(const Node* nd, const std::vector<uint2>& dst, hipStream_t s);
   // Rebuilt bodies: the wide records of slots ks[q] from their binary trees
   // (grid.y = frame; nothing when the binary walk is selected).
   void fold_frames(int F, const int* ks, hipStream_t s);

@@ -395,30 +395,22 @@ void export_tree_raw(uint32_t m, const uint64_t* keys_d, const uint4* leaf_tri_d
     if (parent_leaf) parent_leaf[0] = 0;
     return;
   }
-  std::vector<int32_t> lp(m, 0), np(m - 1, -1);
-  for (uint32_t x = 0; x + 1 < m; ++x)
-    for (const int32_t c : {nd[x].childA, nd[x].childB}) {
-      CC_REQUIRE(c < 0 ? (uint32_t)~c < m : (uint32_t)c < m - 1, "bvh export: child link out of range");
-      (c < 0 ? lp[~c] : np[c]) = (int32_t)x;
-    }
-  auto slot_of_child = [&](int32_t par, int32_t child, float* dst) {
-    const Node& p = nd[par];
-    const float* src = (p.childA == child) ? p.a_min : p.b_min;
-    std::memcpy(dst, src, 6 * sizeof(float));
-  };
+  // a node's record tells its children their parent and their boxes
+  if (parent_int) parent_int[0] = 0;
+  if (box_int) std::memcpy(box_int, r, sizeof(r));
   for (uint32_t x = 0; x + 1 < m; ++x) {
     const Node& n = nd[x];
     if (childA) childA[x] = n.childA >= 0 ? n.childA + 1 : n.childA;   // ~l == -(l+1)
     if (childB) childB[x] = n.childB >= 0 ? n.childB + 1 : n.childB;
-    if (parent_int) parent_int[x] = np[x] + 1;
-    if (box_int) {
-      if (np[x] < 0) std::memcpy(box_int + 6 * (size_t)x, r, sizeof(r));
-      else slot_of_child(np[x], (int32_t)x, box_int + 6 * (size_t)x);
+    for (int side = 0; side < 2; ++side) {
+      const int32_t c = side ? n.childB : n.childA;
+      CC_REQUIRE(c < 0 ? (uint32_t)~c < m : (uint32_t)c < m - 1, "bvh export: child link out of range");
+      const size_t at = (size_t)(c < 0 ? ~c : c);
+      int32_t* parent = c < 0 ? parent_leaf : parent_int;
+      float* box = c < 0 ? box_leaf : box_int;
+      if (parent) parent[at] = (int32_t)x + 1;
+      if (box) std::memcpy(box + 6 * at, side ? n.b_min : n.a_min, 6 * sizeof(float));
     }
-  }
-  for (uint32_t l = 0; l < m; ++l) {
-    if (parent_leaf) parent_leaf[l] = lp[l] + 1;
-    if (box_leaf) slot_of_child(lp[l], ~(int32_t)l, box_leaf + 6 * (size_t)l);
   }
 }
 

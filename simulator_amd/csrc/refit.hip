@@ -26,6 +26,9 @@
 //    own L2); the kernel boundary between the passes gives the visibility.
 //  * All boxes go to their parent's child slot (the layout the traversal
 //    reads).  fmin/fmax unions are exact, so the order does not matter.
+#include <algorithm>
+#include <memory>
+
 #include "cc_lbvh.h"
 
 namespace cc {
@@ -616,96 +619,89 @@ __global__ __launch_bounds__(LV_C) void k_refit_level(const RefitGroup* __restri
 }
 
 // ======================================================== host side
+// On the path of every replacement of a refitted body's vertices, so nothing is
+// searched for that the order of the leaves tells: nodes are held by their
+// splits, and what a group leaves follows from the largest node that starts at
+// each item.
 void RefitTables::add(const Node* nd, uint32_t m, uint32_t base0, const RefitGroup& body,
                       const std::vector<uint2>& dst) {
+  // by splits: the node of the split right of leaf i, and its leaf range
+  struct Split {
+    uint32_t node, first, last;
+  };
   struct Item {
     uint32_t first, last;
-    int32_t node;          // the item's node, -1 for a leaf
   };
-  // by splits: the node of the split right of leaf i, its leaf range
   const uint32_t mi = m - 1;
-  std::vector<uint32_t> node_at(mi), first(mi), last(mi);
-  std::vector<int32_t> parent(mi, -1);
+  std::unique_ptr<Split[]> at(new Split[mi]);
+  for (uint32_t i = 0; i < mi; ++i) at[i].node = ~0u;
   for (uint32_t x = 0; x < mi; ++x) {
     const Node& N = nd[x];
     const uint32_t sp = (uint32_t)(N.childA < 0 ? ~N.childA : N.childA);
     const uint32_t f = x == 0 ? 0 : std::min<uint32_t>(x, (uint32_t)N.other);
     const uint32_t e = x == 0 ? m - 1 : std::max<uint32_t>(x, (uint32_t)N.other);
-    CC_REQUIRE(sp < mi && f <= sp && sp < e && e < m, "refit levels: bad node");
-    node_at[sp] = x;
-    first[x] = f;
-    last[x] = e;
-    for (const int32_t c : {N.childA, N.childB})
-      if (c >= 0) {
-        CC_REQUIRE((uint32_t)c < mi, "refit levels: bad link");
-        parent[c] = (int32_t)x;
-      }
+    CC_REQUIRE(sp < mi && f <= sp && sp < e && e < m && at[sp].node == ~0u, "refit levels: bad node");
+    at[sp] = {x, f, e};
   }
-  std::vector<Item> items(m);
-  for (uint32_t i = 0; i < m; ++i) items[i] = {i, i, -1};
-  std::vector<uint32_t> at_first(m), at_last(m);   // item starting / ending at a leaf
+  std::vector<Item> items, next;             // of levels above 0; level 0's are the leaves
+  uint32_t ni = m;
   int L = 0;
-  for (; L < RL_MAX && !items.empty(); ++L) {
-    const uint32_t ni = (uint32_t)items.size(), base = L == 0 ? base0 : (uint32_t)rec[L].size();
+  for (; L < RL_MAX && ni; ++L) {
+    const uint32_t base = L == 0 ? base0 : (uint32_t)rec[L].size();
     const uint32_t end = std::max((uint32_t)rec[L].size(), base + ni);
     rec[L].resize(end, make_uint2(0u, RL_NONE | (RL_NONE << 16)));
     node[L].resize(end, 0u);
     if (!dst.empty()) wd[L].resize(end, make_uint4(~0u, 0u, ~0u, 0u));
-    uint2* R = rec[L].data() + base;
     const uint32_t next0 = L + 1 < RL_MAX ? (uint32_t)rec[L + 1].size() : 0u;
-    std::vector<Item> next;
+    next.clear();
     for (uint32_t i0 = 0; i0 < ni; i0 += LV_C) {
       const uint32_t n = std::min<uint32_t>(LV_C, ni - i0);
-      const uint32_t f0 = items[i0].first, l0 = items[i0 + n - 1].last, out0 = (uint32_t)next.size();
-      for (uint32_t k = 0; k < n; ++k) {
-        at_first[items[i0 + k].first] = k;
-        at_last[items[i0 + k].last] = k;
-      }
-      auto inside = [&](int32_t x) { return x >= 0 && first[x] >= f0 && last[x] <= l0; };
+      const Item* it = L ? items.data() + i0 : nullptr;
+      auto first_of = [&](uint32_t k) { return L ? it[k].first : i0 + k; };
+      auto last_of = [&](uint32_t k) { return L ? it[k].last : i0 + k; };
+      // the item that starts / ends at a leaf of the group
+      auto starts = [&](uint32_t leaf) {
+        if (!L) return leaf - i0;
+        return (uint32_t)(std::lower_bound(it, it + n, leaf, [](const Item& q, uint32_t v) { return q.first < v; }) - it);
+      };
+      auto ends = [&](uint32_t leaf) {
+        if (!L) return leaf - i0;
+        return (uint32_t)(std::lower_bound(it, it + n, leaf, [](const Item& q, uint32_t v) { return q.last < v; }) - it);
+      };
+      const uint32_t f0 = first_of(0), l0 = last_of(n - 1), out0 = (uint32_t)next.size();
+      uint16_t far[LV_C] = {}, by[LV_C];     // end, and split, of the largest node from item k (0: none)
       uint32_t rounds = 0;
-      for (uint32_t k = 0; k < n; ++k) {
-        R[i0 + k] = make_uint2(0u, RL_NONE | (RL_NONE << 16));
-        if (k + 1 == n) continue;
-        const uint32_t x = node_at[items[i0 + k].last];
-        if (!inside((int32_t)x)) continue;
-        const uint32_t l = at_first[first[x]], r = at_last[last[x]];
-        R[i0 + k].x = l | (r << 10) | RL_VALID | (x == 0 ? RL_ROOT : 0u);
+      uint2* R = rec[L].data() + base + i0;
+      for (uint32_t k = 0; k + 1 < n; ++k) {
+        const Split& S = at[last_of(k)];
+        if (S.first < f0 || S.last > l0) continue;
+        const uint32_t l = starts(S.first), r = ends(S.last), x = S.node;
+        R[k].x = l | (r << 10) | RL_VALID | (x == 0 ? RL_ROOT : 0u);
         node[L][base + i0 + k] = x;
         if (!dst.empty()) {
           const uint2 a = dst[2 * (size_t)x], b = dst[2 * (size_t)x + 1];
           wd[L][base + i0 + k] = make_uint4(a.x, a.y, b.x, b.y);
         }
-        for (uint32_t len = std::max(k - l + 1, r - k), q = 1; len; len >>= 1, ++q) rounds = std::max(rounds, q);
+        rounds = std::max(rounds, 32u - (uint32_t)__builtin_clz(std::max(k - l + 1, r - k)));
+        if (r > far[l]) {
+          far[l] = (uint16_t)r;
+          by[l] = (uint16_t)k;
+        }
       }
       // what the group leaves, in leaf order: from each position the largest
-      // node of the group that starts there and was finished here, else the item
+      // node finished here that starts there, else the item
       for (uint32_t k = 0; k < n;) {
-        // the topmost finished node over item k: climb from the item
-        const Item& it = items[i0 + k];
-        int32_t x = it.node, up = -1;
-        // the parent of a leaf or node with range [first, last]: the node whose
-        // split is at last, or at first - 1
-        if (x >= 0) {
-          up = parent[x];
-        } else {
-          const int32_t a = it.last < mi ? (int32_t)node_at[it.last] : -1;
-          const int32_t c = it.first > 0 ? (int32_t)node_at[it.first - 1] : -1;
-          up = (a >= 0 && nd[a].childA == ~(int32_t)it.first) ? a : c;
-        }
-        while (inside(up)) {
-          x = up;
-          up = parent[x];
-        }
-        if (x >= 0 && x != it.node) {          // a node finished here
-          const uint32_t sp = (uint32_t)(nd[x].childA < 0 ? ~nd[x].childA : nd[x].childA);
-          if (x != 0) {
-            R[i0 + at_last[sp]].y = (R[i0 + at_last[sp]].y & 0xffff0000u) | ((uint32_t)next.size() - out0);
-            next.push_back({first[x], last[x], x});
+        const uint32_t to = (uint32_t)next.size() - out0;
+        if (far[k]) {
+          const Split& S = at[last_of(by[k])];
+          if (S.node != 0) {
+            R[by[k]].y = (R[by[k]].y & 0xffff0000u) | to;
+            next.push_back({S.first, S.last});
           }
-          k = at_last[last[x]] + 1;
-        } else {                               // the item itself
-          R[i0 + k].y = (R[i0 + k].y & 0xffffu) | (((uint32_t)next.size() - out0) << 16);
-          next.push_back(it);
+          k = far[k] + 1u;
+        } else {
+          R[k].y = (R[k].y & 0xffffu) | (to << 16);
+          next.push_back({first_of(k), last_of(k)});
           ++k;
         }
       }
@@ -717,8 +713,9 @@ void RefitTables::add(const Node* nd, uint32_t m, uint32_t base0, const RefitGro
       blk[L].push_back(g);
     }
     items.swap(next);
+    ni = (uint32_t)items.size();
   }
-  CC_REQUIRE(items.empty(), "refit levels: too many levels");
+  CC_REQUIRE(!ni, "refit levels: too many levels");
   nlevels = std::max(nlevels, L);
 }
 
@@ -735,9 +732,9 @@ void RefitTables::upload(RefitLevel* rl, hipStream_t s) const {
   CC_HIP(hipStreamSynchronize(s));             // the host copies end here
 }
 
-void Body::refit_setup(const std::vector<Node>& nd, const std::vector<uint2>& dst, hipStream_t s) {
+void Body::refit_setup(const Node* nd, const std::vector<uint2>& dst, hipStream_t s) {
   RefitTables t;
-  t.add(nd.data(), m, 0, RefitGroup{}, dst);
+  t.add(nd, m, 0, RefitGroup{}, dst);
   t.upload(rl, s);
   nrl = t.nlevels;
   for (int L = 1; L < nrl; ++L)

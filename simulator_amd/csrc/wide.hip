@@ -129,29 +129,44 @@ void Body::wide_setup(int k, hipStream_t s) {
   nwide = 0;
   wide_stack = 0;
   if (mode == CC_BODY_NONE || mode == CC_BODY_REBUILD || m < 2) return;
+  // (a vector: the pages are there before the copy, which takes twice as long otherwise)
   std::vector<Node> nd(m - 1);
-  CC_HIP(hipMemcpyAsync(nd.data(), slot[k].nodes.p, nd.size() * sizeof(Node), hipMemcpyDeviceToHost, s));
-  CC_HIP(hipStreamSynchronize(s));
+  copy_on(nd.data(), slot[k].nodes.p, nd.size() * sizeof(Node), hipMemcpyDeviceToHost, s);
   std::vector<uint2> dst;
-  const uint32_t nw = wide_layout(k, nd, dst, s);
-  if (mode == CC_BODY_REFIT && bottom_up) refit_setup(nd, dst, s);
+  const uint32_t nw = wide_layout(k, nd.data(), dst, s);
+  if (mode == CC_BODY_REFIT && bottom_up) refit_setup(nd.data(), dst, s);
   nwide = nw;            // all of it is there
 }
 
-uint32_t Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2>& dst, hipStream_t s) {
+uint32_t Body::wide_layout(int k, const Node* nd, std::vector<uint2>& dst, hipStream_t s) {
   const uint32_t mi = m - 1;
-  // Breadth-first over the kept binary nodes (the root, then the internal
-  // entries of each kept node); wid maps a kept binary node to its record.
+  // Depth-first over the kept binary nodes (the root, then the internal entries
+  // of each kept node), so that the nodes read next lie near those just read;
+  // wid maps a kept binary node to its record.
   std::vector<int32_t> wid(mi, -1), order;
   std::vector<uint4> src;
   std::vector<int4> link;
   std::vector<uint32_t> acc;     // deferrable entries on the path to each record
   order.reserve(mi / 2 + 1);
-  order.push_back(0);
-  wid[0] = 0;
-  acc.push_back(0);
+  src.reserve(mi / 2 + 1);
+  link.reserve(mi / 2 + 1);
+  acc.reserve(mi / 2 + 1);
+  std::vector<uint32_t> open;    // records not laid out yet
+  auto keep = [&](int32_t x, uint32_t deferrable) {
+    const uint32_t h = (uint32_t)order.size();
+    wid[x] = (int32_t)h;
+    order.push_back(x);
+    acc.push_back(deferrable);
+    src.push_back(make_uint4(~0u, ~0u, ~0u, ~0u));
+    link.push_back(make_int4(0, 0, 0, 0));
+    open.push_back(h);
+    return (int32_t)h;
+  };
+  keep(0, 0);
   uint32_t worst = 0;
-  for (size_t h = 0; h < order.size(); ++h) {
+  while (!open.empty()) {
+    const uint32_t h = open.back();
+    open.pop_back();
     const int32_t x = order[h];
     uint32_t es[4], cnt = 0;
     int32_t ref[4];
@@ -217,14 +232,11 @@ uint32_t Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2
         lp[e] = ref[e];
       } else {
         CC_REQUIRE((uint32_t)ref[e] < mi && wid[ref[e]] < 0, "wide form: node reached twice");
-        wid[ref[e]] = (int32_t)order.size();
-        lp[e] = (int32_t)order.size();
-        order.push_back(ref[e]);
-        acc.push_back(deferrable);
+        lp[e] = keep(ref[e], deferrable);
       }
     }
-    src.push_back(sv);
-    link.push_back(lv);
+    src[h] = sv;
+    link[h] = lv;
   }
   // The traversal stack holds 64 entries; keep the binary form otherwise.
   if (worst > 64) return 0;
@@ -233,11 +245,10 @@ uint32_t Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2
   // order, then writes each chunk's entries into a compact run of records.
   {
     const size_t nw = order.size();
-    std::vector<uint32_t> by(nw);
-    for (size_t w = 0; w < nw; ++w) by[w] = (uint32_t)w;
-    std::sort(by.begin(), by.end(), [&](uint32_t a, uint32_t b) { return order[a] < order[b]; });
     std::vector<int32_t> renum(nw);
-    for (size_t r = 0; r < nw; ++r) renum[by[r]] = (int32_t)r;
+    int32_t r = 0;
+    for (uint32_t x = 0; x < mi; ++x)
+      if (wid[x] >= 0) renum[wid[x]] = r++;
     std::vector<uint4> src2(nw);
     std::vector<int4> link2(nw);
     for (size_t w = 0; w < nw; ++w) {
@@ -252,16 +263,20 @@ uint32_t Body::wide_layout(int k, const std::vector<Node>& nd, std::vector<uint2
     src.swap(src2);
     link.swap(link2);
   }
-  dst.assign(2 * (size_t)mi, make_uint2(~0u, 0u));
-  for (size_t w = 0; w < src.size(); ++w) {
-    const uint32_t* e = &src[w].x;
-    const int32_t* lk = &link[w].x;
-    for (int q = 0; q < 4; ++q)
-      if (e[q] != ~0u) dst[e[q]] = make_uint2((uint32_t)(4 * w + q), (uint32_t)lk[q]);
+  // for the refits: the one by levels takes it into its tables, the one by chunks
+  // reads it as it is, and a static body built by levels is folded anew
+  if (!bottom_up || mode == CC_BODY_REFIT) {
+    dst.assign(2 * (size_t)mi, make_uint2(~0u, 0u));
+    for (size_t w = 0; w < src.size(); ++w) {
+      const uint32_t* e = &src[w].x;
+      const int32_t* lk = &link[w].x;
+      for (int q = 0; q < 4; ++q)
+        if (e[q] != ~0u) dst[e[q]] = make_uint2((uint32_t)(4 * w + q), (uint32_t)lk[q]);
+    }
   }
   w_src.upload(src.data(), src.size(), s);
   w_link.upload(link.data(), link.size(), s);
-  w_dst.upload(dst.data(), dst.size(), s);
+  if (!bottom_up) w_dst.upload(dst.data(), dst.size(), s);
   const uint32_t nw = (uint32_t)src.size();
   wide_stack = worst;
   for (int j = 0; j < nslots; ++j) slot[j].wide.alloc(8 * (size_t)nw);
