@@ -427,11 +427,13 @@ __device__ inline int32_t quad_first_hit(const BvhView& b, f3 p, int e, uint32_t
       // no branch: a lane with nothing to defer writes the row past the stack
       spill.lds[(put0 ? at0 : WSTK_LDS) * QSTK_QUADS] = l0;
       if constexpr (AHEAD) spill.lds[(put1 ? at1 : WSTK_LDS) * QSTK_QUADS] = l1;
+      wave_order_lds();                       // one lane's stores, all four lanes' reads
       t0 = spill.lds[max(sp - 1, 0) * QSTK_QUADS];
       if constexpr (AHEAD) t1 = spill.lds[max(sp - 2, 0) * QSTK_QUADS];
     } else {
       if (put0) qstk_put(spill, at0, l0);
       if (put1) qstk_put(spill, at1, l1);
+      wave_order();
       t0 = qstk_get(spill, sp - 1);
       if constexpr (AHEAD) t1 = qstk_get(spill, sp - 2);
       // waited for here: a load left pending on this path makes the other one

@@ -260,6 +260,7 @@ __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const BodyDesc* 
   }
   for (uint32_t q = lane; q < (uint32_t)RADIX_DIGITS / 4; q += 64)
     reinterpret_cast<uint4*>(wcnt[w])[q] = make_uint4(0, 0, 0, 0);
+  wave_order_lds();
 
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
 #pragma unroll
@@ -277,6 +278,7 @@ __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const BodyDesc* 
     const uint32_t prior = wcnt[w][dg], rank = __popcll(msk & lt);
     loc[r] = prior + rank;
     if (ok[r] && rank == 0) wcnt[w][dg] = prior + (uint32_t)__popcll(msk);
+    wave_order_lds();
   }
   __syncthreads();
 #pragma unroll
