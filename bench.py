@@ -184,14 +184,14 @@ def batched_leg(warmup=16, steps=160, plain_steps=48):
     b.synchronize()
     tb = time.perf_counter() - t0
     nv, tile, order = b.info()
-    tuned, fused = b.tuning()
+    tuned, _ = b.tuning()
     b.close()
     out = {"workload": "256 instances, cloth side log-uniform [16,192] (seed 0), capsule bodies of "
                        "2,112-36,096 triangles rebuilt every frame, dt=1e-3",
            "instances": len(scs), "vertices": n, "body_triangles": int(sum(sc.body.tris.shape[0] for sc in scs)),
            "value": n * steps / tb, "unit": "vertex-steps/s", "ms_per_step": 1e3 * tb / steps, "steps": steps,
            "tile": tile, "order": "largest-first" if order else "instance",
-           "tile_ran_in": "a launch with other work" if fused else "k_verlet_batch",
+           "tile_ran_in": "k_verlet_batch",
            "tuner_ms_per_step": {f"tile{t}/{o}": round(float(tuned[i, j]), 4)
                                  for i, t in enumerate((64, 128, 256))
                                  for j, o in enumerate(("instance", "largest-first"))}}

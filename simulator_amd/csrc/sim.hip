@@ -98,24 +98,26 @@ __global__ __launch_bounds__(256) void k_verlet_quad(const float* __restrict__ s
   if (COUNT) count_block(e == 0 ? visits : 0u, active && e == 0, ctr);
 }
 
+// The point query through the binary tree, one lane per point (bodies without
+// the four-wide form, or with the binary walk selected).
 __global__ __launch_bounds__(256) void k_collide_points(BvhView bvh, const float* __restrict__ pts, uint32_t n,
                                                         int32_t* __restrict__ spill, int32_t* __restrict__ hit,
                                                         uint8_t* __restrict__ ins, float* __restrict__ out_pos,
                                                         float* __restrict__ out_n) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  __shared__ int32_t wstk[WSTK_LDS * WSTK_LANES];
   if (i >= n) return;
   f3 p = ld3(pts + 3 * (size_t)i), nc;
   int32_t h;
   uint32_t visits = 0;
-  const bool in = collide_project(bvh, p, nc, h, visits, spill_of(spill, i, n, wstk + threadIdx.x), load_wide_root(bvh));
+  const bool in = collide_project<false>(bvh, p, nc, h, visits, spill_of(spill, i, n), load_wide_root<false>(bvh));
   hit[i] = h;
   ins[i] = in ? 1 : 0;
   st3(out_pos + 3 * (size_t)i, p);
   st3(out_n + 3 * (size_t)i, nc);
 }
 
-// The same query with four lanes per point.
+// The same query through the four-wide form, four lanes per point: a launch
+// has at most 65,536 points, within the sizes where a step takes four.
 __global__ __launch_bounds__(256) void k_collide_quad(BvhView bvh, const float* __restrict__ pts, uint32_t n,
                                                       int32_t* __restrict__ spill, int32_t* __restrict__ hit,
                                                       uint8_t* __restrict__ ins, float* __restrict__ out_pos,
@@ -140,7 +142,7 @@ static bool by_quads(const BvhView& v, uint32_t n) { return n <= QUAD_MAX_N && (
 void launch_collide_points(const BvhView& v, const float* pts, uint32_t n, int32_t* spill, int32_t* hit,
                            uint8_t* ins, float* out_pos, float* out_n, hipStream_t s) {
   if (n == 0) return;
-  if (by_quads(v, n))
+  if (v.wide || v.m == 0)
     k_collide_quad<<<grid_for(n, QSTK_QUADS), 256, 0, s>>>(v, pts, n, spill, hit, ins, out_pos, out_n);
   else
     k_collide_points<<<grid_for(n, 256), 256, 0, s>>>(v, pts, n, spill, hit, ins, out_pos, out_n);
