@@ -453,8 +453,9 @@ int cc_fault_inject(int kind, int64_t count);
    projected in a step is moved by that fixed plane projection, and the
    contact normal entering the next step's force projection is a constant.
    The spring set must be symmetric (each i->j with a j->i of the same type
-   and rest length).  A rollout of up to 1 GiB (36 bytes per vertex and step)
-   keeps every state; states of a longer one (or where that memory is not to
+   and rest length).  A rollout of up to 1 GiB (36 bytes per vertex and step;
+   CC_ADJ_KEEP_MB in the environment sets another limit, 0: none) keeps every
+   state; states of a longer one (or where that memory is not to
    be had) are checkpointed every ckpt_every steps and recomputed in the
    backward pass, with the same results.  sim must outlive the handle. */
 typedef struct cc_adj cc_adj;

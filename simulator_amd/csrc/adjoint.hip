@@ -24,12 +24,13 @@
 // step t - 1, which needs only what this vertex has just finished
 // (k_adj_step); k_adj_force opens a run of steps.
 //
-// A trajectory of up to ADJ_KEEP_BYTES keeps every state of the forward, and
+// A trajectory of up to keep_limit() bytes keeps every state of the forward, and
 // the backward steps through them.  A longer one keeps checkpoints every
 // `ckpt` steps; each segment is recomputed forward with its per-step states
 // kept, then stepped back.  The states are the same either way.  Parameter
 // gradients: FP32 sums per step and block of 256 vertices, accumulated per
 // block in FP64 (k_adj_acc), reduced in FP64 on the GPU at the end.
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 
@@ -42,8 +43,13 @@ constexpr int ADJ_THREADS = 256;
 constexpr int NPARAM = 5;   // k0, k1, k2, damp, rest_scale
 // All states of a rollout are kept up to this size (36 bytes per vertex and
 // step): 128 x 128 vertices over 200 steps take 118 MB, and recomputing them
-// took 1.1 of the 3.6 ms of their backward.  1 GiB is a 1/288 of the card.
-constexpr size_t ADJ_KEEP_BYTES = (size_t)1 << 30;
+// took 1.1 of the 3.6 ms of their backward.  1 GiB is a 1/288 of the card; a
+// program that holds many handles, or little memory, sets CC_ADJ_KEEP_MB.
+constexpr size_t ADJ_KEEP_MB = 1024;
+static size_t keep_limit() {
+  const char* e = std::getenv("CC_ADJ_KEEP_MB");
+  return (e ? (size_t)std::clamp(std::atoll(e), 0ll, 1ll << 30) : ADJ_KEEP_MB) << 20;
+}
 
 struct AdjArgs {
   float dt, inv_dt, w, damp, kd, k0, k1, k2, rest_scale, eps;
@@ -489,7 +495,7 @@ int cc_adj_create(cc_sim* sim, uint32_t nsteps, uint32_t ckpt_every, cc_adj** ou
     const size_t keep_bytes = ((size_t)nsteps + 1) * 9 * S.n * sizeof(float);
     std::unique_ptr<cc_adj> h(new cc_adj);
     try {
-      alloc_adj(h->a, S, nsteps, ckpt_every, keep_bytes <= ADJ_KEEP_BYTES);
+      alloc_adj(h->a, S, nsteps, ckpt_every, keep_bytes <= keep_limit());
     } catch (const Error& e) {
       if (e.code != CC_ERR_ALLOC || !h->a.keep) throw;
       h.reset();           // the first attempt's memory goes before the second
