@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
 
 #include "cc_device.h"
 #include "cc_lbvh.h"
@@ -279,6 +280,18 @@ void Body::deform(int k, uint64_t frame, hipStream_t s) { deform_frames(1, &k, &
 void Body::build_frames(int F, const int* ks, const int* ls, hipStream_t s) {
   if (mode == CC_BODY_NONE || m == 0) return;
   CC_REQUIRE(F >= 1 && F <= MAX_FRAMES && (F == 1 || bottom_up), "body: frames per build chain");
+  // A static body's first fold needs its records: made before any launch (the
+  // old ones' release waits for the device), missed only once the tree is there.
+  const bool fold_here = grouped && mode == CC_BODY_STATIC;
+  std::exception_ptr no_records;
+  if (fold_here) {
+    nwide = 0;
+    try {
+      slot[0].wide.alloc(8 * (size_t)(m - 1));
+    } catch (const Error&) {
+      no_records = std::current_exception();
+    }
+  }
   PF<const float> verts{};
   PF<float> boxes{}, partial{};
   SortFrame sf[MAX_FRAMES];
@@ -299,9 +312,8 @@ void Body::build_frames(int F, const int* ks, const int* ls, hipStream_t s) {
   if (bottom_up) {                      // tree and boxes by levels
     build_levels(F, ks, ls, s);
     if (mode == CC_BODY_STATIC) torn = false;   // walked as it is until it has wide records
-    if (grouped && mode == CC_BODY_STATIC) {
-      nwide = 0;
-      slot[0].wide.alloc(8 * (size_t)(m - 1));
+    if (fold_here) {
+      if (no_records) std::rethrow_exception(no_records);
       fold_frames(F, ks, s);
       nwide = m - 1;
       wide_stack = STACK_LIMIT;
