@@ -244,7 +244,7 @@ int cc_sim_destroy(cc_sim* sim);
    hipGraphs while the lanes compute the next block's poses; the remaining
    steps -- and every call with nsteps = 1, the reference's one call per
    frame -- are launched one by one, each issuing the pose of a frame a few
-   frames ahead (two per lane) on a lane, so the body update of later frames
+   frames ahead (four per lane) on a lane, so the body update of later frames
    runs beside this frame's step.  Asynchronous on stream (NULL: the
    simulator's own stream). */
 int cc_sim_step(cc_sim* sim, int nsteps, void* stream);
@@ -331,8 +331,10 @@ int cc_bvh_size(cc_sim* sim, uint32_t* leaves);
    binary tree.  A static or refitted body whose root paths could defer more
    than 64 entries always walks the binary tree.  cc_bvh_width reports the
    form in use, the wide node count and the deferral bound of the tree (64,
-   the stack limit, for a rebuilt body: its wide walk defers no more than
-   the binary walk, whose stack holds at most the tree depth). */
+   the stack limit, for a rebuilt body and for a static one of 2 to 2^21
+   triangles whose vertices were replaced, which is folded like one: the wide
+   walk then defers no more than the binary walk, whose stack holds at most
+   the tree depth). */
 int cc_sim_set_bvh_width(cc_sim* sim, int width);
 int cc_bvh_width(cc_sim* sim, int* width, uint32_t* wide_nodes, uint32_t* stack_bound);
 

@@ -21,7 +21,8 @@ constexpr uint32_t END_MASK = 0x3fffffffu;
 constexpr int ELL_W = 12;
 constexpr int ELL_W2 = 24;
 constexpr uint32_t PAD_TYPE = 3u << 30;
-// Launches of up to this many vertices or points take four lanes each.  Four lanes per vertex
+// Launches of up to this many vertices take four lanes each (a query's, of at most
+// 65,536 points, always do).  Four lanes per vertex
 // shorten a vertex's chain of dependent work (a quarter of the springs, a
 // round of four loads for two records instead of eight for one) but make four
 // times the waves, each about 40% of the one-lane kernel's instructions: the
@@ -77,8 +78,9 @@ struct Sim {
   // Graphs of graph_steps steps, per slot of the first frame and state
   // parity (captured when first needed).
   // Steps per block (even; a moving body's ring holds 2 * graph_steps
-  // poses).  24 is three chains of four frames on each of two lanes; measured with three lanes of one frame at the 501k-triangle refitted
-  // body: 52.4 us per step against 54.5 with 16 and 53.8 with 32.
+  // poses).  24 is three chains of four frames on each of two lanes; measured
+  // with three lanes of one frame at the 501k-triangle refitted body: 52.4 us
+  // per step against 54.5 with 16 and 53.8 with 32.
   int graph_steps = 24;
   hipGraphExec_t gmain[MAX_SLOTS][2] = {};
   // update lanes (moving bodies): streams and the events that order them
