@@ -8,6 +8,20 @@
 
 namespace cc {
 
+// What the lanes of a wave have written so far (to LDS alone, or anywhere) is
+// what its lanes read from here on.  The hardware keeps a wave's accesses in
+// order by itself; this keeps the compiler from moving them, and is no instruction.
+__device__ inline void wave_order_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+__device__ inline void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Deferred-node stack of one traversal beyond the four entries held in
 // registers: entry k of a lane is p[k * stride] (lanes of a wave adjacent,
 // so spills coalesce).  It lives in global memory that the caller provides,

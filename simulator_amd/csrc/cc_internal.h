@@ -163,20 +163,6 @@ struct Stage {
 
 inline unsigned grid_for(size_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
 
-// What the lanes of a wave have written so far (to LDS alone, or anywhere) is
-// what its lanes read from here on.  The hardware keeps a wave's accesses in
-// order by itself; this keeps the compiler from moving them, and is no instruction.
-__device__ inline void wave_order_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
-__device__ inline void wave_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Synchronous copy / fill on the object's own stream.  The library never
 // uses the null stream: created on first use, it takes one of the process's
 // hardware queues (four on MI355X by default) ahead of streams created later,

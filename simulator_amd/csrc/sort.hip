@@ -24,6 +24,7 @@
 // instead of two: 33 us of scatters against 27.  The 4.2 M
 // triangles of 256 bodies: 156 us, against 244 us with one workgroup per
 // body (bound by the largest body, 36,096 keys on one CU).
+#include "cc_device.h"
 #include "cc_lbvh.h"
 
 namespace cc {
