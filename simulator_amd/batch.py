@@ -137,7 +137,8 @@ class Batch:
 
     def tuning(self):
         """The tuner's ms per step for tiles 64 / 128 / 256 x order 0 / 1
-        (a (3, 2) array) and whether it timed the fused sort + step launch."""
+        (a (3, 2) array) and whether it timed a launch that carries other
+        work beside the step (never)."""
         ms = np.zeros(6, np.float32)
         fused = C.c_uint32()
         L.check(L.lib().cc_batch_tuning(self._h, L.ptr(ms), C.byref(fused)))

@@ -376,7 +376,7 @@ struct Body {
   void share_topology(int from, hipStream_t s); // copy slot `from`'s tree to every other slot
   // Four-wide form: the tables from slot k's tree and slot k's wide records
   // (host, synchronous; keeps the binary form when the stack bound fails);
-  // later refits write the boxes through w_dst.
+  // later refits write the boxes through its map of child slots.
   void wide_setup(int k, hipStream_t s);
   // the layout itself, from the nodes' host copy: child slot -> {entry, link}
   // into dst where a refit needs it; returns the number of records (0: the binary form stays)

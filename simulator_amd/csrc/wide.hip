@@ -14,7 +14,8 @@
 // the topology the refit walks.  The layout is computed once per topology on
 // the host (Body::wide_setup), which writes the records in full from the
 // binary boxes (k_fold_wide).  Later refits write each box straight into the
-// wide entry that mirrors its binary child slot (w_dst) and leave the binary
+// wide entry that mirrors its binary child slot (through the tables of the
+// refit by levels, or w_dst in a refit by chunks) and leave the binary
 // boxes alone; export and the binary walk ask for a binary refit.
 //
 // A rebuilt body's topology changes every frame, so its wide form is folded
